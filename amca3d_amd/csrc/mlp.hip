@@ -1,7 +1,9 @@
 // Temperature surrogate: a 5-128-128-128-128-1 MLP with SiLU, BF16 operands on
 // the gfx950 matrix cores (v_mfma_f32_32x32x16_bf16) and FP32 accumulation.
 //
-// Every layer, forward and backward, is one call of a tiled GEMM
+// Inference is one kernel, k_mlp_fused: the weights sit in LDS and a wave
+// carries 64 rows through the whole network in registers.  In training every
+// layer, forward and backward, is one call of a tiled GEMM
 //   C[M x N] = epilogue( opA(A)[M x K] * opB(B)[K x N] )
 // with A and B read from FP32 or BF16 memory, optionally transposed, rounded
 // to BF16 when staged into LDS, and an epilogue that adds the bias and applies
@@ -10,12 +12,12 @@
 // 128 x 128 block of C; each wave owns 32 rows and four 32 x 32 MFMA tiles.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
+#include <cstddef>
 #include <cstring>
-#include <mutex>
 #include <random>
 #include <string>
-#include <unordered_map>
 #include <vector>
 
 #include "../../include/amca3d.h"
@@ -253,43 +255,47 @@ __global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float
 }  // namespace mlpk
 
 namespace mlpk {
-// fused inference (defined with the sampler below): mode 0 rows of X -> network
-// output, mode 1 lattice points of (d, s, g) -> temperatures
-hipError_t launch_fused(int mode, const float* p, long long n, const float* X, float* out,
-                        const amca_surrogate_desc& d, const amca_scan& s, const SurLattice& g,
-                        hipStream_t st);
-hipError_t launch_fused_timed(amca_mlp* h, int mode, long long n, const float* X, float* out,
+// fused inference (defined with the sampler below)
+enum FusedMode : int {
+  kRowsScaled = 0,  // rows of X -> network output, activations rounded scaled by -log2(e)
+  kLattice = 1,     // lattice points of (d, s, g) -> temperatures, the same rounding
+  kRows = 2,        // rows of X -> network output, activations rounded as they are
+};
+struct FusedImage;
+hipError_t fused_setup();
+hipError_t launch_pack(const float* p, FusedImage* img, hipStream_t st);
+hipError_t launch_fused(FusedMode mode, const FusedImage* img, int cus, long long n, const float* X,
+                        float* out, const amca_surrogate_desc& d, const amca_scan& s,
+                        const SurLattice& g, hipStream_t st);
+hipError_t launch_fused_timed(amca_mlp* h, FusedMode mode, long long n, const float* X, float* out,
                               const amca_surrogate_desc& d, const amca_scan& s,
                               const SurLattice& g);
+size_t fused_image_bytes();
 }  // namespace mlpk
 
 using namespace mlpk;
 
-// Activations of amca_mlp_forward_device_noalloc, which allocates nothing: two
-// ping-pong [kNoAllocRows][128] BF16 buffers (16 MiB), one copy per GPU the
-// library runs on, held until the process ends.  Host code never passes the
-// name itself to a kernel (on the host it is only a stand-in for the symbol);
-// each device's address comes from hipGetSymbolAddress (noalloc_scratch).
-constexpr int kNoAllocRows = AMCA_MLP_NOALLOC_MAX_ROWS;
-static __device__ __align__(256) __bf16 scratch[2 * (size_t)kNoAllocRows * kHid];
-
 struct amca_mlp {
   hipStream_t stream = nullptr;
-  int device = -1;                 // the device current at create
-  __bf16* noalloc_act = nullptr;   // that device's copy of `scratch` (two [rows][128] buffers)
+  int device = -1;          // the device current at create
+  int cus = 256;            // its compute units
   Layout lay;
   float* params = nullptr;  // FP32 master copy
+  FusedImage* image = nullptr;  // the same weights in k_mlp_fused's order (repacked whenever
+                                // the parameters change)
   float* grads = nullptr;
   float* adam_m = nullptr;
   float* adam_v = nullptr;
   long long adam_t = 0;
-  // per-batch work buffers
+  // rows of host-pointer calls
+  int rows_cap = 0;
+  float* X = nullptr;            // [rows_cap][5]
+  float* Y = nullptr;            // [rows_cap]
+  float* T = nullptr;            // outputs [rows_cap]
+  // per-batch work buffers of training
   int cap = 0;
-  float* X = nullptr;            // [cap][5]
-  float* Y = nullptr;            // [cap]
   float* Z[4] = {};              // pre-activations [cap][128]
   __bf16* Aact[4] = {};          // activations [cap][128]
-  float* T = nullptr;            // outputs [cap]
   float* dT = nullptr;           // [cap]
   float* dZ[2] = {};             // ping-pong [cap][128]
   float* loss = nullptr;
@@ -316,11 +322,6 @@ namespace {
 
 thread_local std::string g_mlp_error;
 
-// per-device address of `scratch`, resolved once per device with that device
-// current (amca_mlp_create)
-std::mutex g_scratch_mu;
-std::unordered_map<int, __bf16*> g_scratch_addr;
-
 amca_status mlp_fail(amca_status s, const std::string& m) {
   g_mlp_error = m;
   return s;
@@ -338,21 +339,6 @@ amca_status mlp_fail(amca_status s, const std::string& m) {
     amca_status s_ = (expr);      \
     if (s_ != AMCA_OK) return s_; \
   } while (0)
-
-amca_status noalloc_scratch(int device, __bf16** out) {
-  std::lock_guard<std::mutex> lock(g_scratch_mu);
-  auto it = g_scratch_addr.find(device);
-  if (it == g_scratch_addr.end()) {
-    void* p = nullptr;
-    const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-    if (e != hipSuccess || !p)
-      return mlp_fail(AMCA_ERR_HIP,
-                      std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(e));
-    it = g_scratch_addr.emplace(device, static_cast<__bf16*>(p)).first;
-  }
-  *out = it->second;
-  return AMCA_OK;
-}
 
 template <class T>
 amca_status mlp_alloc(amca_mlp* h, T** p, size_t n) {
@@ -372,12 +358,27 @@ void mlp_release(amca_mlp* h, void* p) {
     }
 }
 
+// input and output rows of the calls that take host pointers
+amca_status ensure_rows(amca_mlp* h, int n) {
+  if (n <= h->rows_cap) return AMCA_OK;
+  MLP_HIP(hipStreamSynchronize(h->stream));
+  h->rows_cap = 0;
+  for (float** p : {&h->X, &h->Y, &h->T}) {
+    mlp_release(h, *p);
+    *p = nullptr;
+  }
+  MLP_TRY(mlp_alloc(h, &h->X, (size_t)n * kIn));
+  MLP_TRY(mlp_alloc(h, &h->Y, (size_t)n));
+  MLP_TRY(mlp_alloc(h, &h->T, (size_t)n));
+  h->rows_cap = n;
+  return AMCA_OK;
+}
+
 amca_status ensure_cap(amca_mlp* h, int n) {
+  MLP_TRY(ensure_rows(h, n));
   if (n <= h->cap) return AMCA_OK;
   MLP_HIP(hipStreamSynchronize(h->stream));
-  mlp_release(h, h->X);
-  mlp_release(h, h->Y);
-  mlp_release(h, h->T);
+  h->cap = 0;
   mlp_release(h, h->dT);
   for (int l = 0; l < 4; l++) {
     mlp_release(h, h->Z[l]);
@@ -385,9 +386,6 @@ amca_status ensure_cap(amca_mlp* h, int n) {
   }
   for (int q = 0; q < 2; q++) mlp_release(h, h->dZ[q]);
   const size_t c = (size_t)n;
-  MLP_TRY(mlp_alloc(h, &h->X, c * kIn));
-  MLP_TRY(mlp_alloc(h, &h->Y, c));
-  MLP_TRY(mlp_alloc(h, &h->T, c));
   MLP_TRY(mlp_alloc(h, &h->dT, c));
   for (int l = 0; l < 4; l++) {
     MLP_TRY(mlp_alloc(h, &h->Z[l], c * kHid));
@@ -395,6 +393,20 @@ amca_status ensure_cap(amca_mlp* h, int n) {
   }
   for (int q = 0; q < 2; q++) MLP_TRY(mlp_alloc(h, &h->dZ[q], c * kHid));
   h->cap = n;
+  return AMCA_OK;
+}
+
+// the fused kernel's weights follow the parameters: on the network's stream
+// after whatever changed them
+amca_status repack(amca_mlp* h) {
+  MLP_HIP(launch_pack(h->params, h->image, h->stream));
+  return AMCA_OK;
+}
+
+// network outputs of n device rows, enqueued on the network's stream
+amca_status infer(amca_mlp* h, long long n, const float* X, float* T) {
+  MLP_HIP(launch_fused(kRows, h->image, h->cus, n, X, T, amca_surrogate_desc{}, amca_scan{},
+                       SurLattice{}, h->stream));
   return AMCA_OK;
 }
 
@@ -409,32 +421,25 @@ hipError_t gemm(hipStream_t s, const TA* A, int lda, const TB* B, int ldb, int M
   return hipGetLastError();
 }
 
-// forward of n rows already in h->X; keeps Z (for a backward pass) when keep_z
-// forward of n rows X[n][5] -> T[n] through the activation buffers act[4]
-// ([n][128] each; act[l] is written by layer l and read by layer l + 1), keeping
-// the pre-activations in h->Z when keep_z
-amca_status forward_rows(amca_mlp* h, int n, const float* X, __bf16* const act[4], float* T,
-                         bool keep_z) {
+// forward of the n rows in h->X, keeping the activations and pre-activations
+// for a backward pass
+amca_status forward(amca_mlp* h, int n) {
   const Layout& L = h->lay;
   hipStream_t s = h->stream;
   for (int l = 0; l < 4; l++) {
-    EpiArgs e{nullptr, kHid, h->params + L.b[l], keep_z ? h->Z[l] : nullptr, act[l]};
+    EpiArgs e{nullptr, kHid, h->params + L.b[l], h->Z[l], h->Aact[l]};
     if (l == 0)
-      MLP_HIP((gemm<float, float, false, false, kEpiBiasSilu>(s, X, kIn, h->params + L.w[0], kHid,
-                                                               n, kHid, kIn, e)));
+      MLP_HIP((gemm<float, float, false, false, kEpiBiasSilu>(s, h->X, kIn, h->params + L.w[0],
+                                                               kHid, n, kHid, kIn, e)));
     else
-      MLP_HIP((gemm<__bf16, float, false, false, kEpiBiasSilu>(s, act[l - 1], kHid,
+      MLP_HIP((gemm<__bf16, float, false, false, kEpiBiasSilu>(s, h->Aact[l - 1], kHid,
                                                                 h->params + L.w[l], kHid, n, kHid,
                                                                 kHid, e)));
   }
-  EpiArgs e{T, 1, h->params + L.b[4], nullptr, nullptr};
-  MLP_HIP((gemm<__bf16, float, false, false, kEpiStore>(s, act[3], kHid, h->params + L.w[4], 1, n,
-                                                         1, kHid, e)));
+  EpiArgs e{h->T, 1, h->params + L.b[4], nullptr, nullptr};
+  MLP_HIP((gemm<__bf16, float, false, false, kEpiStore>(s, h->Aact[3], kHid, h->params + L.w[4], 1,
+                                                         n, 1, kHid, e)));
   return AMCA_OK;
-}
-
-amca_status forward(amca_mlp* h, int n, bool keep_z = true) {
-  return forward_rows(h, n, h->X, h->Aact, h->T, keep_z);
 }
 
 // gradients of the mean squared error over n rows (X, Y on the device) into h->grads
@@ -506,7 +511,17 @@ amca_status amca_mlp_create(uint64_t seed, amca_mlp** out) {
       st = mlp_fail(AMCA_ERR_HIP, "hipGetDevice");
       break;
     }
-    if ((st = noalloc_scratch(h->device, &h->noalloc_act)) != AMCA_OK) break;
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device) ==
+            hipSuccess && cus > 0)
+      h->cus = cus;
+    if (fused_setup() != hipSuccess) {
+      st = mlp_fail(AMCA_ERR_HIP, "LDS size of the fused kernel");
+      break;
+    }
+    unsigned char* img = nullptr;
+    if ((st = mlp_alloc(h, &img, fused_image_bytes())) != AMCA_OK) break;
+    h->image = reinterpret_cast<FusedImage*>(img);
     const int P = h->lay.total;
     if ((st = mlp_alloc(h, &h->params, P)) != AMCA_OK) break;
     if ((st = mlp_alloc(h, &h->grads, P)) != AMCA_OK) break;
@@ -527,6 +542,7 @@ amca_status amca_mlp_create(uint64_t seed, amca_mlp** out) {
       st = mlp_fail(AMCA_ERR_HIP, "upload");
       break;
     }
+    st = repack(h);
   } while (0);
   if (st != AMCA_OK) {
     delete h;
@@ -547,7 +563,7 @@ amca_status amca_mlp_set_params(amca_mlp* h, const float* p) {
   MLP_HIP(hipMemset(h->adam_m, 0, sizeof(float) * h->lay.total));
   MLP_HIP(hipMemset(h->adam_v, 0, sizeof(float) * h->lay.total));
   h->adam_t = 0;
-  return AMCA_OK;
+  return repack(h);
 }
 
 amca_status amca_mlp_get_params(amca_mlp* h, float* p) {
@@ -559,9 +575,9 @@ amca_status amca_mlp_get_params(amca_mlp* h, float* p) {
 
 amca_status amca_mlp_forward(amca_mlp* h, int32_t n, const float* x5, float* t) {
   if (!h || n < 1 || !x5 || !t) return mlp_fail(AMCA_ERR_INVALID, "bad arguments");
-  MLP_TRY(ensure_cap(h, n));
+  MLP_TRY(ensure_rows(h, n));
   MLP_HIP(hipMemcpyAsync(h->X, x5, sizeof(float) * kIn * n, hipMemcpyHostToDevice, h->stream));
-  MLP_TRY(forward(h, n));
+  MLP_TRY(infer(h, n, h->X, h->T));
   MLP_HIP(hipMemcpyAsync(t, h->T, sizeof(float) * n, hipMemcpyDeviceToHost, h->stream));
   MLP_HIP(hipStreamSynchronize(h->stream));
   return AMCA_OK;
@@ -616,16 +632,16 @@ amca_status amca_mlp_train_device(amca_mlp* h, int64_t n, const float* dX, const
       loss_trace[it] = l / (float)batch;
     }
   }
+  MLP_TRY(repack(h));
   MLP_HIP(hipStreamSynchronize(h->stream));
   return AMCA_OK;
 }
 
-// Forward over device-resident rows (no copies): T[n] = mlp(X[n][5]).
 amca_status amca_mlp_forward_fused(amca_mlp* h, int32_t n, const float* x5, float* t) {
   if (!h || n < 1 || !x5 || !t) return mlp_fail(AMCA_ERR_INVALID, "bad arguments");
-  MLP_TRY(ensure_cap(h, n));
+  MLP_TRY(ensure_rows(h, n));
   MLP_HIP(hipMemcpyAsync(h->X, x5, sizeof(float) * kIn * n, hipMemcpyHostToDevice, h->stream));
-  MLP_HIP(launch_fused_timed(h, 0, n, h->X, h->T, amca_surrogate_desc{}, amca_scan{},
+  MLP_HIP(launch_fused_timed(h, kRowsScaled, n, h->X, h->T, amca_surrogate_desc{}, amca_scan{},
                              SurLattice{}));
   MLP_HIP(hipMemcpyAsync(t, h->T, sizeof(float) * n, hipMemcpyDeviceToHost, h->stream));
   MLP_HIP(hipStreamSynchronize(h->stream));
@@ -650,40 +666,27 @@ amca_status amca_mlp_fused_times(amca_mlp* h, double* ms, int64_t* launches, int
   return AMCA_OK;
 }
 
+// Device rows in place: one launch, no copies and no workspace.
 amca_status amca_mlp_forward_device(amca_mlp* h, int64_t n, const float* dX, float* dT) {
   if (!h || n < 1 || !dX || !dT) return mlp_fail(AMCA_ERR_INVALID, "bad arguments");
-  const int chunk = 1 << 20;
-  MLP_TRY(ensure_cap(h, (int)std::min<int64_t>(n, chunk)));
-  for (int64_t r = 0; r < n; r += chunk) {
-    const int m = (int)std::min<int64_t>(chunk, n - r);
-    MLP_HIP(hipMemcpyAsync(h->X, dX + r * kIn, sizeof(float) * kIn * m, hipMemcpyDeviceToDevice,
-                           h->stream));
-    MLP_TRY(forward(h, m, false));
-    MLP_HIP(hipMemcpyAsync(dT + r, h->T, sizeof(float) * m, hipMemcpyDeviceToDevice, h->stream));
-  }
+  MLP_TRY(infer(h, n, dX, dT));
   MLP_HIP(hipStreamSynchronize(h->stream));
   return AMCA_OK;
 }
 
-// amca_mlp_forward_device's kernels with the activations in the device's copy
-// of `scratch` and the caller's rows read and written in place: no hipMalloc,
-// no hipFree, no staging copies.  Every buffer element a layer reads was written
-// by the layer before it in the same call, so nothing needs clearing.
 amca_status amca_mlp_forward_device_noalloc(amca_mlp* h, int64_t n, const float* dX, float* dT) {
   if (!h || n < 1 || !dX || !dT) return mlp_fail(AMCA_ERR_INVALID, "bad arguments");
-  if (n > kNoAllocRows)
+  if (n > AMCA_MLP_NOALLOC_MAX_ROWS)
     return mlp_fail(AMCA_ERR_INVALID, "n = " + std::to_string(n) +
                                           " rows exceeds the no-allocation maximum of " +
-                                          std::to_string(kNoAllocRows) + " rows per call");
+                                          std::to_string(AMCA_MLP_NOALLOC_MAX_ROWS) +
+                                          " rows per call");
   int dev = -1;
   MLP_HIP(hipGetDevice(&dev));
-  if (dev != h->device || !h->noalloc_act)
+  if (dev != h->device)
     return mlp_fail(AMCA_ERR_INVALID, "make the network's device (" + std::to_string(h->device) +
                                           ") current before the call");
-  __bf16* a0 = h->noalloc_act;
-  __bf16* a1 = h->noalloc_act + (size_t)kNoAllocRows * kHid;
-  __bf16* const act[4] = {a0, a1, a0, a1};
-  MLP_TRY(forward_rows(h, (int)n, dX, act, dT, false));
+  MLP_TRY(infer(h, n, dX, dT));
   MLP_HIP(hipStreamSynchronize(h->stream));
   return AMCA_OK;
 }
@@ -885,20 +888,33 @@ __global__ void k_denorm(const float* __restrict__ t, int m, amca_surrogate_desc
 // in every row of A and scales its output by -1/log2(e) before adding b5.  The
 // biases of layers 2..4 are loaded into the accumulators before the first
 // MFMA, so those layers add no bias either.
-// Inputs and weights round to BF16 as in the layered path; the activations
-// round to BF16 as scaled values, which differ from the layered path's in the
-// last BF16 place.
+// Inputs and weights round to BF16; the activations round to BF16 as scaled
+// values.  kRows keeps the unscaled form z sigmoid(z) instead (one multiply
+// more per activation), which rounds the activations where training does.
 
 constexpr int kFusedWaves = 8;
 constexpr int kWtStride = kHid + 8;  // bf16 per LDS row (padding spreads the banks)
 
-struct FusedLds {
+struct alignas(16) FusedLds {
   __bf16 wt[3][kHid][kWtStride];  // layers 2..4: wt[l][out][16*ks + 8*g + ii]
   __bf16 w1t[kHid][8];            // layer 1: W1[k][out] for k < 5, zero above
   float b[4][kHid];               // biases of layers 1..4, times -log2(e)
   __bf16 w5[8][2][8];             // W5 in BF16, as the A fragment of k-step ks, lane group g
   float b5;
 };
+
+// FusedLds as every work-group copies it into LDS, kept in device memory and
+// rewritten when the parameters change, and the biases without the scaling for
+// kRows.  Building it from the FP32 parameters in every work-group (a
+// transposing gather of 50 K values, each rounded) cost more than a small call.
+struct FusedImage {
+  FusedLds lds;
+  float raw_b[4][kHid];
+};
+static_assert(offsetof(FusedLds, b) % 16 == 0 && sizeof(FusedLds::b) % 16 == 0 &&
+                  offsetof(FusedImage, raw_b) % 16 == 0,
+              "the image is copied in 16-byte pieces");
+size_t fused_image_bytes() { return sizeof(FusedImage); }
 
 constexpr float kNegLog2e = -1.4426950408889634f;
 constexpr float kNegLn2 = -0.6931471805599453f;  // -1/log2(e)
@@ -912,39 +928,95 @@ __device__ __forceinline__ int fused_feature(int ks, int g, int ii) {
 __device__ __forceinline__ int fused_w(int l) { return l == 0 ? 0 : 768 + (l - 1) * 16512; }
 __device__ __forceinline__ int fused_b(int l) { return l == 0 ? 640 : fused_w(l) + kHid * kHid; }
 
-__device__ __forceinline__ void fused_load(const float* __restrict__ p, FusedLds& L) {
-  for (int q = threadIdx.x; q < 3 * kHid * kHid; q += blockDim.x) {
-    const int l = q / (kHid * kHid), out = (q / kHid) % kHid, kk = q % kHid;
-    const int in = fused_feature(kk >> 4, (kk >> 3) & 1, kk & 7);
-    L.wt[l][out][kk] = (__bf16)p[fused_w(l + 1) + in * kHid + out];
+// parameter i into its places in the image
+__device__ __forceinline__ void pack_param(FusedImage& I, int i, float v) {
+  FusedLds& L = I.lds;
+  if (i < kIn * kHid) {
+    L.w1t[i % kHid][i / kHid] = (__bf16)v;
+    return;
   }
-  for (int q = threadIdx.x; q < kHid * 8; q += blockDim.x) {
-    const int out = q / 8, k = q % 8;
-    L.w1t[out][k] = (__bf16)(k < kIn ? p[k * kHid + out] : 0.0f);
-  }
-  for (int q = threadIdx.x; q < 4 * kHid; q += blockDim.x)
-    L.b[q / kHid][q % kHid] = kNegLog2e * p[fused_b(q / kHid) + q % kHid];
   const int w5 = fused_b(3) + kHid;
-  for (int q = threadIdx.x; q < kHid; q += blockDim.x) {
-    const int ks = q >> 4, g = (q >> 3) & 1, ii = q & 7;
-    L.w5[ks][g][ii] = (__bf16)p[w5 + fused_feature(ks, g, ii)];
+  if (i >= w5) {
+    const int in = i - w5;
+    if (in == kHid) {
+      L.b5 = v;
+    } else {
+      const int r = in & 15;  // in = 16 ks + 8 (ii / 4) + 4 g + ii % 4
+      L.w5[in >> 4][(r >> 2) & 1][4 * (r >> 3) + (r & 3)] = (__bf16)v;
+    }
+    return;
   }
-  if (threadIdx.x == 0) L.b5 = p[w5 + kHid];
+  int l = 0, q = i - fused_b(0);
+  if (q >= kHid) {
+    l = 1 + (q - kHid) / (kHid * kHid + kHid);
+    q = i - fused_w(l);
+  } else {
+    q += kHid * kHid;  // a bias of layer 1, in the place of the other layers' biases
+  }
+  if (q >= kHid * kHid) {
+    I.raw_b[l][q - kHid * kHid] = v;
+    L.b[l][q - kHid * kHid] = kNegLog2e * v;
+    return;
+  }
+  const int in = q / kHid, out = q % kHid, r = in & 15;
+  L.wt[l - 1][out][16 * (in >> 4) + 8 * ((r >> 2) & 1) + 4 * (r >> 3) + (r & 3)] = (__bf16)v;
+}
+
+__global__ void __launch_bounds__(kThreads) k_pack(const float* __restrict__ p,
+                                                   FusedImage* __restrict__ img) {
+  const int i = blockIdx.x * kThreads + threadIdx.x;
+  if (i < fused_b(3) + 2 * kHid + 1) pack_param(*img, i, p[i]);
+  // the k rows above the five inputs
+  if (i < kHid)
+    for (int k = kIn; k < 8; k++) img->lds.w1t[i][k] = (__bf16)0.0f;
+}
+
+hipError_t launch_pack(const float* p, FusedImage* img, hipStream_t st) {
+  const int n = Layout().total;
+  hipLaunchKernelGGL(k_pack, dim3((n + kThreads - 1) / kThreads), dim3(kThreads), 0, st, p, img);
+  return hipGetLastError();
+}
+
+template <bool kScaled>
+__device__ __forceinline__ void fused_load(const FusedImage* __restrict__ img, FusedLds& L) {
+  constexpr int kPieces = (int)((sizeof(FusedLds) + 15) / 16);
+  constexpr int kPer = (kPieces + 64 * kFusedWaves - 1) / (64 * kFusedWaves);
+  constexpr int kB0 = (int)(offsetof(FusedLds, b) / 16), kB1 = kB0 + (int)(sizeof(L.b) / 16);
+  const uint4* src = reinterpret_cast<const uint4*>(img);
+  const uint4* raw = reinterpret_cast<const uint4*>(&img->raw_b[0][0]) - kB0;
+  uint4* dst = reinterpret_cast<uint4*>(&L);
+  uint4 v[kPer];
+#pragma unroll
+  for (int x = 0; x < kPer; x++) {
+    const int q = threadIdx.x + x * 64 * kFusedWaves;
+    v[x] = make_uint4(0u, 0u, 0u, 0u);
+    if (q < kPieces) v[x] = (!kScaled && q >= kB0 && q < kB1) ? raw[q] : src[q];
+  }
+#pragma unroll
+  for (int x = 0; x < kPer; x++) {
+    const int q = threadIdx.x + x * 64 * kFusedWaves;
+    if (q < kPieces) dst[q] = v[x];
+  }
   __syncthreads();
 }
 
 // Chunk ks of the epilogue: a' = y / (1 + 2^y) of the eight accumulator
 // registers 8(ks%2).. of tile ks/2, rounded to BF16, into the next layer's B
 // operand bop[ks]; kFirst: y = -log2(e) acc + bias (layer 1), else y = acc.
-template <bool kFirst>
+// Unscaled: a = z / (1 + 2^(-log2(e) z)), z = acc + bias (layer 1) or acc.
+template <bool kFirst, bool kScaled>
 __device__ __forceinline__ void fused_epi_chunk(const floatx16* acc, const float* bias, int g,
                                                 int ks, bf16x8* bop) {
   const int t = ks >> 1, s = ks & 1;
 #pragma unroll
   for (int ii = 0; ii < 8; ii++) {
     float y = acc[t][8 * s + ii];
-    if (kFirst) y = fmaf(y, kNegLog2e, bias[fused_feature(ks, g, ii)]);
-    bop[ks][ii] = (__bf16)(y * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(y)));
+    if (kFirst) {
+      const float b = bias[fused_feature(ks, g, ii)];
+      y = kScaled ? fmaf(y, kNegLog2e, b) : y + b;
+    }
+    const float e = __builtin_amdgcn_exp2f(kScaled ? y : kNegLog2e * y);
+    bop[ks][ii] = (__bf16)(y * __builtin_amdgcn_rcpf(1.0f + e));
   }
 }
 
@@ -954,7 +1026,7 @@ __device__ __forceinline__ void fused_epi_chunk(const floatx16* acc, const float
 // start at the layer's bias (register 4q+j of tile ot holds output feature
 // 32 ot + 8 q + 4 g + j); the weight fragments of k-step ks+1 are read from
 // LDS while those of k-step ks feed the MFMAs.
-template <bool kFirstEpi>
+template <bool kFirstEpi, bool kScaled>
 __device__ __forceinline__ void fused_phase(const FusedLds& L, int l, int r, int g,
                                             floatx16* accP, const bf16x8* bopP,
                                             const floatx16* accQ, bf16x8* bopQ) {
@@ -986,7 +1058,7 @@ __device__ __forceinline__ void fused_phase(const FusedLds& L, int l, int r, int
 #pragma unroll
     for (int ot = 0; ot < 4; ot++)
       accP[ot] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[ks & 1][ot], bopP[ks], accP[ot], 0, 0, 0);
-    fused_epi_chunk<kFirstEpi>(accQ, L.b[0], g, ks, bopQ);
+    fused_epi_chunk<kFirstEpi, kScaled>(accQ, L.b[0], g, ks, bopQ);
     // LDS reads first, then each MFMA followed by a share of the epilogue
     __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
 #pragma unroll
@@ -1001,7 +1073,7 @@ __device__ __forceinline__ void fused_phase(const FusedLds& L, int l, int r, int
 // Layer 5 of half P (8 MFMAs, A = W5 in every row, so every accumulator
 // register of lane L holds the output of row L % 32), optionally interleaved
 // with the last epilogue of half Q.
-template <bool kEpi>
+template <bool kEpi, bool kScaled>
 __device__ __forceinline__ float fused_out(const FusedLds& L, int g, const bf16x8* bopP,
                                            const floatx16* accQ, bf16x8* bopQ) {
   floatx16 acc;
@@ -1012,20 +1084,21 @@ __device__ __forceinline__ float fused_out(const FusedLds& L, int g, const bf16x
     const bf16x8 a = *reinterpret_cast<const bf16x8*>(&L.w5[ks][g][0]);
     acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bopP[ks], acc, 0, 0, 0);
     if (kEpi) {
-      fused_epi_chunk<false>(accQ, nullptr, g, ks, bopQ);
+      fused_epi_chunk<false, kScaled>(accQ, nullptr, g, ks, bopQ);
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x002, 40, 0);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
-  return fmaf(acc[0], kNegLn2, L.b5);
+  return kScaled ? fmaf(acc[0], kNegLn2, L.b5) : acc[0] + L.b5;
 }
 
 // Network output (the training target scale) of the 64 rows whose inputs the
 // lanes hold in x[0..4] (lane L: row L of the group), returned in lane L.
 // Half X is rows 0..31, half Y rows 32..63; each runs the whole network, and
 // the MFMAs of one half overlap the SiLU epilogue of the other.
+template <bool kScaled>
 __device__ __forceinline__ float fused_rows(const FusedLds& L, const float* x) {
   const int lane = threadIdx.x & 63, g = lane >> 5, r = lane & 31;
   floatx16 accX[4], accY[4];
@@ -1052,36 +1125,42 @@ __device__ __forceinline__ float fused_rows(const FusedLds& L, const float* x) {
     accY[ot] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, by, accY[ot], 0, 0, 0);
   }
 #pragma unroll
-  for (int ks = 0; ks < 8; ks++) fused_epi_chunk<true>(accX, L.b[0], g, ks, bopX);
+  for (int ks = 0; ks < 8; ks++) fused_epi_chunk<true, kScaled>(accX, L.b[0], g, ks, bopX);
   // hidden layers 2..4
-  fused_phase<true>(L, 0, r, g, accX, bopX, accY, bopY);
-  fused_phase<false>(L, 0, r, g, accY, bopY, accX, bopX);
-  fused_phase<false>(L, 1, r, g, accX, bopX, accY, bopY);
-  fused_phase<false>(L, 1, r, g, accY, bopY, accX, bopX);
-  fused_phase<false>(L, 2, r, g, accX, bopX, accY, bopY);
-  fused_phase<false>(L, 2, r, g, accY, bopY, accX, bopX);
-  const float tx = fused_out<true>(L, g, bopX, accY, bopY);
-  const float ty = fused_out<false>(L, g, bopY, nullptr, nullptr);
+  fused_phase<true, kScaled>(L, 0, r, g, accX, bopX, accY, bopY);
+  fused_phase<false, kScaled>(L, 0, r, g, accY, bopY, accX, bopX);
+  fused_phase<false, kScaled>(L, 1, r, g, accX, bopX, accY, bopY);
+  fused_phase<false, kScaled>(L, 1, r, g, accY, bopY, accX, bopX);
+  fused_phase<false, kScaled>(L, 2, r, g, accX, bopX, accY, bopY);
+  fused_phase<false, kScaled>(L, 2, r, g, accY, bopY, accX, bopX);
+  const float tx = fused_out<true, kScaled>(L, g, bopX, accY, bopY);
+  const float ty = fused_out<false, kScaled>(L, g, bopY, nullptr, nullptr);
   return g == 0 ? tx : ty;
 }
 
-// mode 0: rows of X (n x 5) -> T (network output); mode 1: lattice points ->
-// temperatures (from_target) into out
+// Bound by the SiLU epilogue's two transcendentals per activation (rows in and
+// out are 24 bytes against 99 840 flop).  Every inference call runs here: rows
+// that went through one tiled GEMM per layer, the activations through memory,
+// took 1417 us for 1 000 003 rows and 95 us for 300 (five launches); in this
+// kernel 154 us (646 TFLOP/s) and 23.5 us.
+// 64-row groups over the work-groups: group gr goes to work-group gr % gridDim,
+// so that a call of a few hundred rows spreads over as many CUs instead of
+// filling one work-group's eight waves.
 template <int kMode>
 __global__ void __launch_bounds__(64 * kFusedWaves)
-k_mlp_fused(const float* __restrict__ p, long long n, const float* __restrict__ X,
+k_mlp_fused(const FusedImage* __restrict__ img, long long n, const float* __restrict__ X,
             float* __restrict__ out, amca_surrogate_desc d, amca_scan s, SurLattice g) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
   FusedLds& L = *reinterpret_cast<FusedLds*>(lds_raw);
-  fused_load(p, L);
+  fused_load<kMode != kRows>(img, L);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const long long groups = (n + 63) / 64;
-  for (long long gr = (long long)blockIdx.x * kFusedWaves + wave; gr < groups;
+  for (long long gr = blockIdx.x + (long long)wave * gridDim.x; gr < groups;
        gr += (long long)gridDim.x * kFusedWaves) {
     const long long row = gr * 64 + lane;
     float x[kIn] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     if (row < n) {
-      if (kMode == 0) {
+      if (kMode != kLattice) {
 #pragma unroll
         for (int q = 0; q < kIn; q++) x[q] = X[row * kIn + q];
       } else {
@@ -1091,42 +1170,46 @@ k_mlp_fused(const float* __restrict__ p, long long n, const float* __restrict__ 
         inputs(d, s, g.xi0 + i * g.dxi + s.x_start, g.y0 + j * g.dy, g.z0 + k * g.dz, 0.0, x);
       }
     }
-    const float t = fused_rows(L, x);
-    if (row < n) out[row] = kMode == 0 ? t : (float)from_target(d, (double)t);
+    const float t = fused_rows<kMode != kRows>(L, x);
+    if (row < n) out[row] = kMode != kLattice ? t : (float)from_target(d, (double)t);
   }
 }
 
-hipError_t launch_fused(int mode, const float* p, long long n, const float* X, float* out,
-                        const amca_surrogate_desc& d, const amca_scan& s, const SurLattice& g,
-                        hipStream_t st) {
-  const size_t lds = sizeof(FusedLds);
-  long long blocks = (n + 64 * kFusedWaves - 1) / (64 * kFusedWaves);
-  if (blocks > 1024) blocks = 1024;
-  if (blocks < 1) blocks = 1;
-  if (mode == 0) {
-    hipError_t e = hipFuncSetAttribute((const void*)k_mlp_fused<0>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+hipError_t fused_setup() {
+  for (const void* f : {(const void*)k_mlp_fused<kRowsScaled>, (const void*)k_mlp_fused<kLattice>,
+                        (const void*)k_mlp_fused<kRows>}) {
+    const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             (int)sizeof(FusedLds));
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_mlp_fused<0>, dim3((unsigned)blocks), dim3(64 * kFusedWaves), lds, st, p,
-                       n, X, out, d, s, g);
-  } else {
-    hipError_t e = hipFuncSetAttribute((const void*)k_mlp_fused<1>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_mlp_fused<1>, dim3((unsigned)blocks), dim3(64 * kFusedWaves), lds, st, p,
-                       n, X, out, d, s, g);
   }
+  return hipSuccess;
+}
+
+// One work-group per CU at most (its weights fill two thirds of the LDS, so
+// more would only load them again when a CU comes free).
+hipError_t launch_fused(FusedMode mode, const FusedImage* img, int cus, long long n, const float* X,
+                        float* out, const amca_surrogate_desc& d, const amca_scan& s,
+                        const SurLattice& g, hipStream_t st) {
+  const dim3 grid((unsigned)std::max(1LL, std::min((n + 63) / 64, (long long)cus)));
+  const dim3 block(64 * kFusedWaves);
+  const size_t lds = sizeof(FusedLds);
+  if (mode == kRowsScaled)
+    hipLaunchKernelGGL(k_mlp_fused<kRowsScaled>, grid, block, lds, st, img, n, X, out, d, s, g);
+  else if (mode == kLattice)
+    hipLaunchKernelGGL(k_mlp_fused<kLattice>, grid, block, lds, st, img, n, X, out, d, s, g);
+  else
+    hipLaunchKernelGGL(k_mlp_fused<kRows>, grid, block, lds, st, img, n, X, out, d, s, g);
   return hipGetLastError();
 }
 
 // launch_fused, bracketed by HIP events on the handle's stream when timing is
 // on (the launch is waited for and its duration added to the totals)
-hipError_t launch_fused_timed(amca_mlp* h, int mode, long long n, const float* X, float* out,
+hipError_t launch_fused_timed(amca_mlp* h, FusedMode mode, long long n, const float* X, float* out,
                               const amca_surrogate_desc& d, const amca_scan& s,
                               const SurLattice& g) {
-  if (!h->timing) return launch_fused(mode, h->params, n, X, out, d, s, g, h->stream);
+  if (!h->timing) return launch_fused(mode, h->image, h->cus, n, X, out, d, s, g, h->stream);
   hipError_t e = hipEventRecord(h->ev[0], h->stream);
-  if (e == hipSuccess) e = launch_fused(mode, h->params, n, X, out, d, s, g, h->stream);
+  if (e == hipSuccess) e = launch_fused(mode, h->image, h->cus, n, X, out, d, s, g, h->stream);
   if (e == hipSuccess) e = hipEventRecord(h->ev[1], h->stream);
   if (e == hipSuccess) e = hipEventSynchronize(h->ev[1]);
   float ms = 0.0f;
@@ -1155,7 +1238,7 @@ const char* surrogate_error() { return g_mlp_error.c_str(); }
 amca_status surrogate_eval_lattice(amca_mlp* h, const amca_surrogate_desc& d, const amca_scan& s,
                                    const SurLattice& g, float* out) {
   const long long total = (long long)g.nxi * g.ny * g.nz;
-  MLP_HIP(launch_fused_timed(h, 1, total, nullptr, out, d, s, g));
+  MLP_HIP(launch_fused_timed(h, kLattice, total, nullptr, out, d, s, g));
   MLP_HIP(hipStreamSynchronize(h->stream));
   return AMCA_OK;
 }
@@ -1215,7 +1298,7 @@ amca_status amca_surrogate_eval_lattice(amca_mlp* h, const amca_surrogate_desc* 
 amca_status amca_surrogate_eval(amca_mlp* h, const amca_surrogate_desc* d, const amca_scan* s,
                                 int32_t n, const double* xyzt, double* Ts, double* Tfe) {
   if (!h || !d || !s || n < 1 || !xyzt || !Ts || !Tfe) return mlp_fail(AMCA_ERR_INVALID, "bad arguments");
-  MLP_TRY(ensure_cap(h, n));
+  MLP_TRY(ensure_rows(h, n));
   double *dp = nullptr, *dfe = nullptr;
   MLP_HIP(hipMalloc(&dp, sizeof(double) * 4 * n));
   MLP_HIP(hipMalloc(&dfe, sizeof(double) * n));
@@ -1225,7 +1308,7 @@ amca_status amca_surrogate_eval(amca_mlp* h, const amca_surrogate_desc* d, const
     if (hipMemcpy(dp, xyzt, sizeof(double) * 4 * n, hipMemcpyHostToDevice) != hipSuccess) { st = mlp_fail(AMCA_ERR_HIP, "copy"); break; }
     hipLaunchKernelGGL(k_eval_points, dim3((n + 255) / 256), dim3(256), 0, h->stream, *d, *s, n, dp,
                        h->X, dfe);
-    if ((st = forward(h, n, false)) != AMCA_OK) break;
+    if ((st = infer(h, n, h->X, h->T)) != AMCA_OK) break;
     if (hipMemcpyAsync(t.data(), h->T, sizeof(float) * n, hipMemcpyDeviceToHost, h->stream) != hipSuccess ||
         hipMemcpyAsync(Tfe, dfe, sizeof(double) * n, hipMemcpyDeviceToHost, h->stream) != hipSuccess ||
         hipStreamSynchronize(h->stream) != hipSuccess) { st = mlp_fail(AMCA_ERR_HIP, "readback"); break; }
