@@ -2,14 +2,12 @@
 // the gfx950 matrix cores (v_mfma_f32_32x32x16_bf16) and FP32 accumulation.
 //
 // Inference is one kernel, k_mlp_fused: the weights sit in LDS and a wave
-// carries 64 rows through the whole network in registers.  In training every
-// layer, forward and backward, is one call of a tiled GEMM
-//   C[M x N] = epilogue( opA(A)[M x K] * opB(B)[K x N] )
-// with A and B read from FP32 or BF16 memory, optionally transposed, rounded
-// to BF16 when staged into LDS, and an epilogue that adds the bias and applies
-// SiLU (forward), multiplies by SiLU' (backward), or accumulates atomically
-// (weight gradients, split over the batch).  A work-group of 4 waves owns a
-// 128 x 128 block of C; each wave owns 32 rows and four 32 x 32 MFMA tiles.
+// carries 64 rows through the whole network in registers.  A training step is
+// two: k_train takes 64 rows per work-group through the forward and backward
+// passes and leaves the work-group's share of the weight gradients, k_reduce
+// adds the shares and applies Adam.  Both read the weights as bf16 images in
+// the order the matrix instructions take them (NetImage), which whatever
+// changes the parameters rewrites.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -30,7 +28,6 @@ namespace mlpk {
 
 constexpr int kIn = 5, kHid = 128, kLayers = 5;
 constexpr int kBM = 128, kBN = 128, kBK = 32;
-constexpr int kWgradRows = 128;  // batch rows per work-group of a weight-gradient GEMM
 constexpr int kPad = 8;  // bf16 elements of padding per LDS row
 constexpr int kThreads = 256;
 
@@ -53,108 +50,48 @@ struct Layout {
   }
 };
 
-enum Epi : int {
-  kEpiStore = 0,     // C = acc (+ bias)
-  kEpiBiasSilu = 1,  // Z = acc + bias (FP32), Aout = bf16(silu(Z))
-  kEpiDSilu = 2,     // C = acc * silu'(Z)
-  kEpiAtomic = 3,    // C += acc (atomic)
-};
-
-struct EpiArgs {
-  float* C;          // output (FP32), row stride ldc
-  int ldc;
-  const float* bias; // per column, or null
-  float* Z;          // kEpiBiasSilu: pre-activation out; kEpiDSilu: pre-activation in
-  __bf16* Aout;      // kEpiBiasSilu: activation out (BF16), row stride ldc
-  float* colsum;     // kEpiAtomic with opB = B: column sums of B over the block's K
-                     // range (FP32, before rounding) added atomically, or null
-};
-
 // v_rcp_f32 (1 ulp) in place of the IEEE divide sequence: the result is
 // rounded to bf16 or feeds an fp32 gradient, far coarser than the reciprocal.
-__device__ __forceinline__ float silu(float z) { return z * __builtin_amdgcn_rcpf(1.0f + __expf(-z)); }
-__device__ __forceinline__ float dsilu(float z) {
-  const float s = __builtin_amdgcn_rcpf(1.0f + __expf(-z));
-  return s * (1.0f + z * (1.0f - s));
+__device__ __forceinline__ float sigmoid(float z) {
+  return __builtin_amdgcn_rcpf(1.0f + __expf(-z));
 }
 
-template <typename T>
-__device__ __forceinline__ float to_f(T v) { return (float)v; }
-
-// C = epi(opA(A) * opB(B)).  opA(A)[m][k] = TrA ? A[k*lda + m] : A[m*lda + k];
-// opB(B)[k][n] = TrB ? B[n*ldb + k] : B[k*ldb + n].  Out-of-range elements
-// stage as zero.  Grid: (ceil(N/128), ceil(M/128), ksplit); block z covers
-// K range [z*kchunk, (z+1)*kchunk).
-template <typename TA, typename TB, bool TrA, bool TrB, int E>
+// C = opA(A) * opB(B), operands rounded to BF16 when staged into LDS: the matrix
+// layout check behind amca_mlp_gemm_selftest.  opA(A)[m][k] = TrA ? A[k*lda + m] :
+// A[m*lda + k]; opB(B)[k][n] = TrB ? B[n*ldb + k] : B[k*ldb + n].  A work-group of
+// 4 waves owns a 128 x 128 block of C (ldc = N), each wave 32 rows and four
+// 32 x 32 MFMA tiles; elements outside the matrices stage as zero.
+template <bool TrA, bool TrB>
 __global__ void __launch_bounds__(kThreads)
-k_gemm(const TA* __restrict__ A, int lda, const TB* __restrict__ B, int ldb, int M, int N, int K,
-       int kchunk, EpiArgs e) {
+k_gemm(const float* __restrict__ A, int lda, const float* __restrict__ B, int ldb, int M, int N,
+       int K, float* __restrict__ C) {
   __shared__ __bf16 As[kBM][kBK + kPad];
   __shared__ __bf16 Bs[kBN][kBK + kPad];  // n-major: Bs[n][k]
   const int m0 = blockIdx.y * kBM, n0 = blockIdx.x * kBN;
-  const int kbeg = blockIdx.z * kchunk;
-  const int kend = min(K, kbeg + kchunk);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   floatx16 acc[4];
 #pragma unroll
   for (int t = 0; t < 4; t++)
 #pragma unroll
     for (int i = 0; i < 16; i++) acc[t][i] = 0.0f;
-  // column sum of B (thread t stages column t % kBN of every B tile when !TrB)
-  constexpr bool kColsum = E == kEpiAtomic && !TrB;
-  float cs = 0.0f;
-
-  for (int k0 = kbeg; k0 < kend; k0 += kBK) {
-    // stage A (128 x 32) and B (32 x 128): 4096 elements each, 16 per thread.
-    // Every load is issued before any is used: an element outside the matrix
-    // (or the block's K range) loads element 0 and stages as zero.
-    float va[(kBM * kBK) / kThreads], vb[(kBN * kBK) / kThreads];
-#pragma unroll
-    for (int q = 0; q < (kBM * kBK) / kThreads; q++) {
-      const int idx = threadIdx.x + q * kThreads;
-      int mm, kk;
-      if (TrA) {  // consecutive threads walk m (contiguous in memory)
-        mm = idx % kBM;
-        kk = idx / kBM;
-      } else {
-        kk = idx % kBK;
-        mm = idx / kBK;
-      }
-      const int gm = m0 + mm, gk = k0 + kk;
-      const bool in = gm < M && gk < kend;
-      const size_t o = in ? (TrA ? (size_t)gk * lda + gm : (size_t)gm * lda + gk) : 0;
-      va[q] = to_f(A[o]);
-      if (!in) va[q] = 0.0f;
-    }
-#pragma unroll
-    for (int q = 0; q < (kBN * kBK) / kThreads; q++) {
-      const int idx = threadIdx.x + q * kThreads;
-      int nn, kk;
-      if (TrB) {
-        kk = idx % kBK;
-        nn = idx / kBK;
-      } else {
-        nn = idx % kBN;
-        kk = idx / kBN;
-      }
-      const int gn = n0 + nn, gk = k0 + kk;
-      const bool in = gn < N && gk < kend;
-      const size_t o = in ? (TrB ? (size_t)gn * ldb + gk : (size_t)gk * ldb + gn) : 0;
-      vb[q] = to_f(B[o]);
-      if (!in) vb[q] = 0.0f;
-    }
+  for (int k0 = 0; k0 < K; k0 += kBK) {
 #pragma unroll
     for (int q = 0; q < (kBM * kBK) / kThreads; q++) {
       const int idx = threadIdx.x + q * kThreads;
       const int mm = TrA ? idx % kBM : idx / kBK, kk = TrA ? idx / kBM : idx % kBK;
-      As[mm][kk] = (__bf16)va[q];
+      const int gm = m0 + mm, gk = k0 + kk;
+      const bool in = gm < M && gk < K;
+      const size_t o = in ? (TrA ? (size_t)gk * lda + gm : (size_t)gm * lda + gk) : 0;
+      As[mm][kk] = (__bf16)(in ? A[o] : 0.0f);
     }
 #pragma unroll
     for (int q = 0; q < (kBN * kBK) / kThreads; q++) {
       const int idx = threadIdx.x + q * kThreads;
       const int nn = TrB ? idx / kBK : idx % kBN, kk = TrB ? idx % kBK : idx / kBN;
-      if (kColsum) cs += vb[q];
-      Bs[nn][kk] = (__bf16)vb[q];
+      const int gn = n0 + nn, gk = k0 + kk;
+      const bool in = gn < N && gk < K;
+      const size_t o = in ? (TrB ? (size_t)gn * ldb + gk : (size_t)gk * ldb + gn) : 0;
+      Bs[nn][kk] = (__bf16)(in ? B[o] : 0.0f);
     }
     __syncthreads();
     // two MFMA k-steps of 16: lane holds A[row = lane%32][k = (lane/32)*8 ..+8]
@@ -175,81 +112,16 @@ k_gemm(const TA* __restrict__ A, int lda, const TB* __restrict__ B, int ldb, int
     }
     __syncthreads();
   }
-  if (kColsum && e.colsum) {
-    static_assert(kThreads % kBN == 0, "a thread stages one column of B");
-    const int gn = n0 + (int)(threadIdx.x % kBN);
-    if (blockIdx.y == 0 && gn < N) atomicAdd(&e.colsum[gn], cs);
-  }
-  // D layout: element i of lane l is row (i/4)*8 + (l/32)*4 + i%4, column l%32.
-  // kEpiDSilu reads the pre-activations of the whole tile before using any.
-  float zin[4][16];
-  if (E == kEpiDSilu) {
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-#pragma unroll
-      for (int i = 0; i < 16; i++) {
-        const int m = m0 + wave * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3);
-        const int n = n0 + t * 32 + (lane & 31);
-        const bool in = m < M && n < N;
-        zin[t][i] = e.Z[in ? (size_t)m * e.ldc + n : 0];
-      }
-    }
-  }
+  // D layout: element i of lane l is row (i/4)*8 + (l/32)*4 + i%4, column l%32
 #pragma unroll
   for (int t = 0; t < 4; t++) {
 #pragma unroll
     for (int i = 0; i < 16; i++) {
       const int m = m0 + wave * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3);
       const int n = n0 + t * 32 + (lane & 31);
-      if (m >= M || n >= N) continue;
-      float v = acc[t][i];
-      const size_t o = (size_t)m * e.ldc + n;
-      if (E == kEpiStore) {
-        if (e.bias) v += e.bias[n];
-        e.C[o] = v;
-      } else if (E == kEpiBiasSilu) {
-        const float z = v + (e.bias ? e.bias[n] : 0.0f);
-        if (e.Z) e.Z[o] = z;
-        e.Aout[o] = (__bf16)silu(z);
-      } else if (E == kEpiDSilu) {
-        e.C[o] = v * dsilu(zin[t][i]);
-      } else {
-        atomicAdd(&e.C[o], v);
-      }
+      if (m < M && n < N) C[(size_t)m * N + n] = acc[t][i];
     }
   }
-}
-
-// dT = 2 (T - Y) / M (the gradient of the mean squared error), loss += sum (T - Y)^2
-__global__ void k_mse(const float* __restrict__ T, const float* __restrict__ Y, int M,
-                      float* __restrict__ dT, float* __restrict__ loss) {
-  __shared__ float s[kThreads];
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  float r = 0.0f;
-  if (i < M) {
-    r = T[i] - Y[i];
-    dT[i] = 2.0f * r / (float)M;
-  }
-  s[threadIdx.x] = r * r;
-  __syncthreads();
-  for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-    if (threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) atomicAdd(loss, s[0]);
-}
-
-__global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
-                       float* __restrict__ v, int n, float lr, float b1, float b2, float eps,
-                       float c1, float c2) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gi = g[i];
-  const float mi = b1 * m[i] + (1.0f - b1) * gi;
-  const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  p[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
 }
 
 }  // namespace mlpk
@@ -261,19 +133,34 @@ enum FusedMode : int {
   kLattice = 1,     // lattice points of (d, s, g) -> temperatures, the same rounding
   kRows = 2,        // rows of X -> network output, activations rounded as they are
 };
-struct FusedImage;
+struct NetImage;
+size_t net_image_bytes();
 hipError_t fused_setup();
-hipError_t launch_pack(const float* p, FusedImage* img, hipStream_t st);
-hipError_t launch_fused(FusedMode mode, const FusedImage* img, int cus, long long n, const float* X,
+hipError_t launch_pack(const float* p, NetImage* img, hipStream_t st);
+// training (defined at the end of the kernels): one 64-row group per work-group
+// and pass, at most one work-group per CU
+constexpr int kTrainRows = 64;
+constexpr int kPartStride = 50440;  // floats of one work-group's gradient share (16-byte rows)
+struct Adam {
+  float *m, *v;  // moments, or null: k_reduce leaves the gradients alone
+  float lr, c1, c2;
+};
+hipError_t launch_train(const float* p, NetImage* img, int blocks, int n, const float* X,
+                        const float* Y, float* part, float* part_loss, hipStream_t st);
+hipError_t launch_reduce(int blocks, const float* part, const float* part_loss, float* p,
+                         float* grads, float* loss, const Adam& adam, NetImage* img,
+                         hipStream_t st);
+hipError_t launch_fused(FusedMode mode, const NetImage* img, int cus, long long n, const float* X,
                         float* out, const amca_surrogate_desc& d, const amca_scan& s,
                         const SurLattice& g, hipStream_t st);
 hipError_t launch_fused_timed(amca_mlp* h, FusedMode mode, long long n, const float* X, float* out,
                               const amca_surrogate_desc& d, const amca_scan& s,
                               const SurLattice& g);
-size_t fused_image_bytes();
 }  // namespace mlpk
 
 using namespace mlpk;
+
+constexpr int kLossSteps = 4096;  // steps whose losses stay on the device between copies
 
 struct amca_mlp {
   hipStream_t stream = nullptr;
@@ -281,8 +168,8 @@ struct amca_mlp {
   int cus = 256;            // its compute units
   Layout lay;
   float* params = nullptr;  // FP32 master copy
-  FusedImage* image = nullptr;  // the same weights in k_mlp_fused's order (repacked whenever
-                                // the parameters change)
+  NetImage* image = nullptr;  // the same weights in the kernels' order (rewritten whenever
+                              // the parameters change)
   float* grads = nullptr;
   float* adam_m = nullptr;
   float* adam_v = nullptr;
@@ -292,13 +179,12 @@ struct amca_mlp {
   float* X = nullptr;            // [rows_cap][5]
   float* Y = nullptr;            // [rows_cap]
   float* T = nullptr;            // outputs [rows_cap]
-  // per-batch work buffers of training
-  int cap = 0;
-  float* Z[4] = {};              // pre-activations [cap][128]
-  __bf16* Aact[4] = {};          // activations [cap][128]
-  float* dT = nullptr;           // [cap]
-  float* dZ[2] = {};             // ping-pong [cap][128]
-  float* loss = nullptr;
+  // training: the work-groups' gradient shares and losses, and a stretch of
+  // per-step losses
+  int part_cap = 0;              // work-groups
+  float* part = nullptr;         // [part_cap][kPartStride]
+  float* part_loss = nullptr;    // [part_cap]
+  float* loss = nullptr;         // [kLossSteps]
   // device-resident training set (amca_surrogate_sample)
   float* setX = nullptr;
   float* setY = nullptr;
@@ -374,29 +260,23 @@ amca_status ensure_rows(amca_mlp* h, int n) {
   return AMCA_OK;
 }
 
-amca_status ensure_cap(amca_mlp* h, int n) {
-  MLP_TRY(ensure_rows(h, n));
-  if (n <= h->cap) return AMCA_OK;
+// work-groups of a training pass over n rows, their shares allocated
+amca_status train_blocks(amca_mlp* h, int n, int* blocks) {
+  *blocks = std::min((n + kTrainRows - 1) / kTrainRows, h->cus);
+  if (*blocks <= h->part_cap) return AMCA_OK;
   MLP_HIP(hipStreamSynchronize(h->stream));
-  h->cap = 0;
-  mlp_release(h, h->dT);
-  for (int l = 0; l < 4; l++) {
-    mlp_release(h, h->Z[l]);
-    mlp_release(h, h->Aact[l]);
+  h->part_cap = 0;
+  for (float** p : {&h->part, &h->part_loss}) {
+    mlp_release(h, *p);
+    *p = nullptr;
   }
-  for (int q = 0; q < 2; q++) mlp_release(h, h->dZ[q]);
-  const size_t c = (size_t)n;
-  MLP_TRY(mlp_alloc(h, &h->dT, c));
-  for (int l = 0; l < 4; l++) {
-    MLP_TRY(mlp_alloc(h, &h->Z[l], c * kHid));
-    MLP_TRY(mlp_alloc(h, &h->Aact[l], c * kHid));
-  }
-  for (int q = 0; q < 2; q++) MLP_TRY(mlp_alloc(h, &h->dZ[q], c * kHid));
-  h->cap = n;
+  MLP_TRY(mlp_alloc(h, &h->part, (size_t)*blocks * kPartStride));
+  MLP_TRY(mlp_alloc(h, &h->part_loss, (size_t)*blocks));
+  h->part_cap = *blocks;
   return AMCA_OK;
 }
 
-// the fused kernel's weights follow the parameters: on the network's stream
+// the weight images follow the parameters: on the network's stream
 // after whatever changed them
 amca_status repack(amca_mlp* h) {
   MLP_HIP(launch_pack(h->params, h->image, h->stream));
@@ -407,82 +287,6 @@ amca_status repack(amca_mlp* h) {
 amca_status infer(amca_mlp* h, long long n, const float* X, float* T) {
   MLP_HIP(launch_fused(kRows, h->image, h->cus, n, X, T, amca_surrogate_desc{}, amca_scan{},
                        SurLattice{}, h->stream));
-  return AMCA_OK;
-}
-
-template <typename TA, typename TB, bool TrA, bool TrB, int E>
-hipError_t gemm(hipStream_t s, const TA* A, int lda, const TB* B, int ldb, int M, int N, int K,
-                const EpiArgs& e, int ksplit = 1) {
-  const int kchunk = ((K + ksplit - 1) / ksplit + kBK - 1) / kBK * kBK;
-  const int kz = (K + kchunk - 1) / kchunk;
-  dim3 grid((N + kBN - 1) / kBN, (M + kBM - 1) / kBM, kz);
-  hipLaunchKernelGGL((k_gemm<TA, TB, TrA, TrB, E>), grid, dim3(kThreads), 0, s, A, lda, B, ldb, M,
-                     N, K, kchunk, e);
-  return hipGetLastError();
-}
-
-// forward of the n rows in h->X, keeping the activations and pre-activations
-// for a backward pass
-amca_status forward(amca_mlp* h, int n) {
-  const Layout& L = h->lay;
-  hipStream_t s = h->stream;
-  for (int l = 0; l < 4; l++) {
-    EpiArgs e{nullptr, kHid, h->params + L.b[l], h->Z[l], h->Aact[l]};
-    if (l == 0)
-      MLP_HIP((gemm<float, float, false, false, kEpiBiasSilu>(s, h->X, kIn, h->params + L.w[0],
-                                                               kHid, n, kHid, kIn, e)));
-    else
-      MLP_HIP((gemm<__bf16, float, false, false, kEpiBiasSilu>(s, h->Aact[l - 1], kHid,
-                                                                h->params + L.w[l], kHid, n, kHid,
-                                                                kHid, e)));
-  }
-  EpiArgs e{h->T, 1, h->params + L.b[4], nullptr, nullptr};
-  MLP_HIP((gemm<__bf16, float, false, false, kEpiStore>(s, h->Aact[3], kHid, h->params + L.w[4], 1,
-                                                         n, 1, kHid, e)));
-  return AMCA_OK;
-}
-
-// gradients of the mean squared error over n rows (X, Y on the device) into h->grads
-amca_status backward(amca_mlp* h, int n) {
-  const Layout& L = h->lay;
-  hipStream_t s = h->stream;
-  MLP_HIP(hipMemsetAsync(h->grads, 0, sizeof(float) * L.total, s));
-  MLP_HIP(hipMemsetAsync(h->loss, 0, sizeof(float), s));
-  hipLaunchKernelGGL(k_mse, dim3((n + kThreads - 1) / kThreads), dim3(kThreads), 0, s, h->T, h->Y,
-                     n, h->dT, h->loss);
-  MLP_HIP(hipGetLastError());
-  // weight gradients: one 128 x 128 tile per layer, split over the batch in
-  // chunks of kWgradRows rows so that the split fills the chip; the bias
-  // gradient (column sums of dZ) is taken while dZ is staged
-  const int ksplit = std::max(1, (n + kWgradRows - 1) / kWgradRows);
-  // layer 5: dW5 = A4^T dT, db5 = sum dT, dZ4 = (dT W5^T) * silu'(Z4)
-  {
-    EpiArgs e{h->grads + L.w[4], 1, nullptr, nullptr, nullptr, h->grads + L.b[4]};
-    MLP_HIP((gemm<__bf16, float, true, false, kEpiAtomic>(s, h->Aact[3], kHid, h->dT, 1, kHid, 1, n,
-                                                           e, ksplit)));
-    EpiArgs d{h->dZ[0], kHid, nullptr, h->Z[3], nullptr};
-    MLP_HIP((gemm<float, float, false, true, kEpiDSilu>(s, h->dT, 1, h->params + L.w[4], 1, n, kHid,
-                                                         1, d)));
-  }
-  int cur = 0;
-  for (int l = 3; l >= 0; l--) {
-    float* dz = h->dZ[cur];
-    // dW_l = A_{l-1}^T dZ_l (A_{-1} = X), db_l = sum dZ_l
-    EpiArgs e{h->grads + L.w[l], kHid, nullptr, nullptr, nullptr, h->grads + L.b[l]};
-    if (l == 0)
-      MLP_HIP((gemm<float, float, true, false, kEpiAtomic>(s, h->X, kIn, dz, kHid, kIn, kHid, n, e,
-                                                            ksplit)));
-    else
-      MLP_HIP((gemm<__bf16, float, true, false, kEpiAtomic>(s, h->Aact[l - 1], kHid, dz, kHid, kHid,
-                                                             kHid, n, e, ksplit)));
-    if (l > 0) {
-      // dZ_{l-1} = (dZ_l W_l^T) * silu'(Z_{l-1})
-      EpiArgs d{h->dZ[cur ^ 1], kHid, nullptr, h->Z[l - 1], nullptr};
-      MLP_HIP((gemm<float, float, false, true, kEpiDSilu>(s, dz, kHid, h->params + L.w[l], kHid, n,
-                                                           kHid, kHid, d)));
-      cur ^= 1;
-    }
-  }
   return AMCA_OK;
 }
 
@@ -520,14 +324,14 @@ amca_status amca_mlp_create(uint64_t seed, amca_mlp** out) {
       break;
     }
     unsigned char* img = nullptr;
-    if ((st = mlp_alloc(h, &img, fused_image_bytes())) != AMCA_OK) break;
-    h->image = reinterpret_cast<FusedImage*>(img);
+    if ((st = mlp_alloc(h, &img, net_image_bytes())) != AMCA_OK) break;
+    h->image = reinterpret_cast<NetImage*>(img);
     const int P = h->lay.total;
     if ((st = mlp_alloc(h, &h->params, P)) != AMCA_OK) break;
     if ((st = mlp_alloc(h, &h->grads, P)) != AMCA_OK) break;
     if ((st = mlp_alloc(h, &h->adam_m, P)) != AMCA_OK) break;
     if ((st = mlp_alloc(h, &h->adam_v, P)) != AMCA_OK) break;
-    if ((st = mlp_alloc(h, &h->loss, 1)) != AMCA_OK) break;
+    if ((st = mlp_alloc(h, &h->loss, kLossSteps)) != AMCA_OK) break;
     // He-uniform weights for SiLU layers, zero biases
     std::mt19937_64 rng(seed);
     std::vector<float> p(P, 0.0f);
@@ -538,7 +342,8 @@ amca_status amca_mlp_create(uint64_t seed, amca_mlp** out) {
     }
     if (hipMemcpy(h->params, p.data(), sizeof(float) * P, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemset(h->adam_m, 0, sizeof(float) * P) != hipSuccess ||
-        hipMemset(h->adam_v, 0, sizeof(float) * P) != hipSuccess) {
+        hipMemset(h->adam_v, 0, sizeof(float) * P) != hipSuccess ||
+        hipMemset(h->image, 0, net_image_bytes()) != hipSuccess) {  // its padding stays zero
       st = mlp_fail(AMCA_ERR_HIP, "upload");
       break;
     }
@@ -586,11 +391,15 @@ amca_status amca_mlp_forward(amca_mlp* h, int32_t n, const float* x5, float* t) 
 amca_status amca_mlp_gradients(amca_mlp* h, int32_t n, const float* x5, const float* y,
                                float* grads, float* loss) {
   if (!h || n < 1 || !x5 || !y) return mlp_fail(AMCA_ERR_INVALID, "bad arguments");
-  MLP_TRY(ensure_cap(h, n));
+  MLP_TRY(ensure_rows(h, n));
+  int blocks = 0;
+  MLP_TRY(train_blocks(h, n, &blocks));
   MLP_HIP(hipMemcpyAsync(h->X, x5, sizeof(float) * kIn * n, hipMemcpyHostToDevice, h->stream));
   MLP_HIP(hipMemcpyAsync(h->Y, y, sizeof(float) * n, hipMemcpyHostToDevice, h->stream));
-  MLP_TRY(forward(h, n));
-  MLP_TRY(backward(h, n));
+  MLP_HIP(launch_train(h->params, h->image, blocks, n, h->X, h->Y, h->part, h->part_loss,
+                       h->stream));
+  MLP_HIP(launch_reduce(blocks, h->part, h->part_loss, h->params, h->grads, h->loss, Adam{},
+                        h->image, h->stream));
   if (grads)
     MLP_HIP(hipMemcpyAsync(grads, h->grads, sizeof(float) * h->lay.total, hipMemcpyDeviceToHost,
                            h->stream));
@@ -601,38 +410,37 @@ amca_status amca_mlp_gradients(amca_mlp* h, int32_t n, const float* x5, const fl
   return AMCA_OK;
 }
 
-// One Adam step per batch over device-resident samples X[n][5], Y[n].
+// One Adam step per batch over device-resident samples X[n][5], Y[n], read in
+// place.  The losses stay on the device until kLossSteps of them are there or
+// the last step is queued, so no step waits for the host.
 amca_status amca_mlp_train_device(amca_mlp* h, int64_t n, const float* dX, const float* dY,
                                   int32_t batch, int32_t steps, float lr, uint64_t seed,
                                   float* loss_trace) {
   if (!h || n < batch || batch < 1 || steps < 0 || !dX || !dY)
     return mlp_fail(AMCA_ERR_INVALID, "bad arguments");
-  MLP_TRY(ensure_cap(h, batch));
+  int blocks = 0;
+  MLP_TRY(train_blocks(h, batch, &blocks));
   std::mt19937_64 rng(seed);
   const long long nb = n / batch;
   for (int it = 0; it < steps; it++) {
     const long long b = (long long)(rng() % (unsigned long long)nb);
-    MLP_HIP(hipMemcpyAsync(h->X, dX + (size_t)b * batch * kIn, sizeof(float) * kIn * batch,
-                           hipMemcpyDeviceToDevice, h->stream));
-    MLP_HIP(hipMemcpyAsync(h->Y, dY + (size_t)b * batch, sizeof(float) * batch,
-                           hipMemcpyDeviceToDevice, h->stream));
-    MLP_TRY(forward(h, batch));
-    MLP_TRY(backward(h, batch));
+    MLP_HIP(launch_train(h->params, h->image, blocks, batch, dX + (size_t)b * batch * kIn,
+                         dY + (size_t)b * batch, h->part, h->part_loss, h->stream));
     h->adam_t++;
     const float b1 = 0.9f, b2 = 0.999f;
-    const float c1 = 1.0f - std::pow(b1, (float)h->adam_t);
-    const float c2 = 1.0f - std::pow(b2, (float)h->adam_t);
-    hipLaunchKernelGGL(k_adam, dim3((h->lay.total + 255) / 256), dim3(256), 0, h->stream, h->params,
-                       h->grads, h->adam_m, h->adam_v, h->lay.total, lr, b1, b2, 1e-8f, c1, c2);
-    MLP_HIP(hipGetLastError());
-    if (loss_trace) {
-      float l = 0.0f;
-      MLP_HIP(hipMemcpyAsync(&l, h->loss, sizeof(float), hipMemcpyDeviceToHost, h->stream));
+    const Adam adam{h->adam_m, h->adam_v, lr, 1.0f - std::pow(b1, (float)h->adam_t),
+                    1.0f - std::pow(b2, (float)h->adam_t)};
+    const int slot = it % kLossSteps;
+    MLP_HIP(launch_reduce(blocks, h->part, h->part_loss, h->params, h->grads, h->loss + slot, adam,
+                          h->image, h->stream));
+    if (loss_trace && (slot == kLossSteps - 1 || it == steps - 1)) {
+      float* out = loss_trace + (it - slot);
+      MLP_HIP(hipMemcpyAsync(out, h->loss, sizeof(float) * (slot + 1), hipMemcpyDeviceToHost,
+                             h->stream));
       MLP_HIP(hipStreamSynchronize(h->stream));
-      loss_trace[it] = l / (float)batch;
+      for (int q = 0; q <= slot; q++) out[q] /= (float)batch;
     }
   }
-  MLP_TRY(repack(h));
   MLP_HIP(hipStreamSynchronize(h->stream));
   return AMCA_OK;
 }
@@ -709,13 +517,17 @@ extern "C" amca_status amca_mlp_gemm_selftest(int32_t M, int32_t N, int32_t K, i
     }
     (void)hipMemcpy(dA, A, sizeof(float) * M * K, hipMemcpyHostToDevice);
     (void)hipMemcpy(dB, B, sizeof(float) * K * N, hipMemcpyHostToDevice);
-    EpiArgs e{dC, N, nullptr, nullptr, nullptr};
     const int lda = trans_a ? M : K, ldb = trans_b ? K : N;
-    hipError_t r;
-    if (!trans_a && !trans_b) r = gemm<float, float, false, false, kEpiStore>(s, dA, lda, dB, ldb, M, N, K, e);
-    else if (trans_a && !trans_b) r = gemm<float, float, true, false, kEpiStore>(s, dA, lda, dB, ldb, M, N, K, e);
-    else if (!trans_a && trans_b) r = gemm<float, float, false, true, kEpiStore>(s, dA, lda, dB, ldb, M, N, K, e);
-    else r = gemm<float, float, true, true, kEpiStore>(s, dA, lda, dB, ldb, M, N, K, e);
+    const dim3 grid((N + kBN - 1) / kBN, (M + kBM - 1) / kBM), block(kThreads);
+    if (!trans_a && !trans_b)
+      hipLaunchKernelGGL((k_gemm<false, false>), grid, block, 0, s, dA, lda, dB, ldb, M, N, K, dC);
+    else if (trans_a && !trans_b)
+      hipLaunchKernelGGL((k_gemm<true, false>), grid, block, 0, s, dA, lda, dB, ldb, M, N, K, dC);
+    else if (!trans_a && trans_b)
+      hipLaunchKernelGGL((k_gemm<false, true>), grid, block, 0, s, dA, lda, dB, ldb, M, N, K, dC);
+    else
+      hipLaunchKernelGGL((k_gemm<true, true>), grid, block, 0, s, dA, lda, dB, ldb, M, N, K, dC);
+    const hipError_t r = hipGetLastError();
     if (r != hipSuccess || hipStreamSynchronize(s) != hipSuccess) {
       st = mlp_fail(AMCA_ERR_HIP, "gemm");
       break;
@@ -914,7 +726,19 @@ struct FusedImage {
 static_assert(offsetof(FusedLds, b) % 16 == 0 && sizeof(FusedLds::b) % 16 == 0 &&
                   offsetof(FusedImage, raw_b) % 16 == 0,
               "the image is copied in 16-byte pieces");
-size_t fused_image_bytes() { return sizeof(FusedImage); }
+
+// The hidden layers' weights as the B operands of k_train, 8 values per lane and
+// k-step: wf for the forward pass (k = input, column = output feature), wb for
+// the backward pass (k = output, column = input feature); w1f is layer 1, its k
+// rows above the five inputs zero.
+struct NetImage {
+  FusedImage f;
+  __bf16 wf[3][4][8][64][8];  // [layer][column tile][k-step][lane][k]
+  __bf16 wb[3][4][8][64][8];
+  __bf16 w1f[4][64][8];
+};
+static_assert(offsetof(NetImage, wf) % 16 == 0, "operands are read 16 bytes at a time");
+size_t net_image_bytes() { return sizeof(NetImage); }
 
 constexpr float kNegLog2e = -1.4426950408889634f;
 constexpr float kNegLn2 = -0.6931471805599453f;  // -1/log2(e)
@@ -928,11 +752,14 @@ __device__ __forceinline__ int fused_feature(int ks, int g, int ii) {
 __device__ __forceinline__ int fused_w(int l) { return l == 0 ? 0 : 768 + (l - 1) * 16512; }
 __device__ __forceinline__ int fused_b(int l) { return l == 0 ? 640 : fused_w(l) + kHid * kHid; }
 
-// parameter i into its places in the image
-__device__ __forceinline__ void pack_param(FusedImage& I, int i, float v) {
+// parameter i into its places in the images
+__device__ __forceinline__ void pack_param(NetImage& N, int i, float v) {
+  FusedImage& I = N.f;
   FusedLds& L = I.lds;
   if (i < kIn * kHid) {
-    L.w1t[i % kHid][i / kHid] = (__bf16)v;
+    const int in = i / kHid, out = i % kHid;
+    L.w1t[out][in] = (__bf16)v;
+    N.w1f[out >> 5][out & 31][in] = (__bf16)v;
     return;
   }
   const int w5 = fused_b(3) + kHid;
@@ -960,18 +787,17 @@ __device__ __forceinline__ void pack_param(FusedImage& I, int i, float v) {
   }
   const int in = q / kHid, out = q % kHid, r = in & 15;
   L.wt[l - 1][out][16 * (in >> 4) + 8 * ((r >> 2) & 1) + 4 * (r >> 3) + (r & 3)] = (__bf16)v;
+  N.wf[l - 1][out >> 5][in >> 4][((in >> 3) & 1) * 32 + (out & 31)][in & 7] = (__bf16)v;
+  N.wb[l - 1][in >> 5][out >> 4][((out >> 3) & 1) * 32 + (in & 31)][out & 7] = (__bf16)v;
 }
 
 __global__ void __launch_bounds__(kThreads) k_pack(const float* __restrict__ p,
-                                                   FusedImage* __restrict__ img) {
+                                                   NetImage* __restrict__ img) {
   const int i = blockIdx.x * kThreads + threadIdx.x;
   if (i < fused_b(3) + 2 * kHid + 1) pack_param(*img, i, p[i]);
-  // the k rows above the five inputs
-  if (i < kHid)
-    for (int k = kIn; k < 8; k++) img->lds.w1t[i][k] = (__bf16)0.0f;
 }
 
-hipError_t launch_pack(const float* p, FusedImage* img, hipStream_t st) {
+hipError_t launch_pack(const float* p, NetImage* img, hipStream_t st) {
   const int n = Layout().total;
   hipLaunchKernelGGL(k_pack, dim3((n + kThreads - 1) / kThreads), dim3(kThreads), 0, st, p, img);
   return hipGetLastError();
@@ -1175,6 +1001,8 @@ k_mlp_fused(const FusedImage* __restrict__ img, long long n, const float* __rest
   }
 }
 
+hipError_t train_setup();
+
 hipError_t fused_setup() {
   for (const void* f : {(const void*)k_mlp_fused<kRowsScaled>, (const void*)k_mlp_fused<kLattice>,
                         (const void*)k_mlp_fused<kRows>}) {
@@ -1182,23 +1010,24 @@ hipError_t fused_setup() {
                                              (int)sizeof(FusedLds));
     if (e != hipSuccess) return e;
   }
-  return hipSuccess;
+  return train_setup();
 }
 
 // One work-group per CU at most (its weights fill two thirds of the LDS, so
 // more would only load them again when a CU comes free).
-hipError_t launch_fused(FusedMode mode, const FusedImage* img, int cus, long long n, const float* X,
+hipError_t launch_fused(FusedMode mode, const NetImage* img, int cus, long long n, const float* X,
                         float* out, const amca_surrogate_desc& d, const amca_scan& s,
                         const SurLattice& g, hipStream_t st) {
   const dim3 grid((unsigned)std::max(1LL, std::min((n + 63) / 64, (long long)cus)));
   const dim3 block(64 * kFusedWaves);
   const size_t lds = sizeof(FusedLds);
+  const FusedImage* f = &img->f;
   if (mode == kRowsScaled)
-    hipLaunchKernelGGL(k_mlp_fused<kRowsScaled>, grid, block, lds, st, img, n, X, out, d, s, g);
+    hipLaunchKernelGGL(k_mlp_fused<kRowsScaled>, grid, block, lds, st, f, n, X, out, d, s, g);
   else if (mode == kLattice)
-    hipLaunchKernelGGL(k_mlp_fused<kLattice>, grid, block, lds, st, img, n, X, out, d, s, g);
+    hipLaunchKernelGGL(k_mlp_fused<kLattice>, grid, block, lds, st, f, n, X, out, d, s, g);
   else
-    hipLaunchKernelGGL(k_mlp_fused<kRows>, grid, block, lds, st, img, n, X, out, d, s, g);
+    hipLaunchKernelGGL(k_mlp_fused<kRows>, grid, block, lds, st, f, n, X, out, d, s, g);
   return hipGetLastError();
 }
 
@@ -1220,6 +1049,351 @@ hipError_t launch_fused_timed(amca_mlp* h, FusedMode mode, long long n, const fl
     h->fused_rows += n;
   }
   return e;
+}
+
+// ---------------------------------------------------------------------------
+// Training.  A work-group of four waves takes 64 rows through the network and
+// back.  Wave w owns the 32 features f = 32 w + lane % 32 of every layer, for
+// both 32-row tiles: with rows as M and features as N, its accumulators hold
+// rows 32 rt + 8 (i / 4) + 4 (lane / 32) + i % 4 of feature f, and silu'(z) of
+// every layer stays there (FP32) from the forward to the backward pass.
+// Activations and dZ go through LDS in two layouts: [row][feature], the A
+// operand of the next layer (or of dZ W^T), and [feature][row], the operands of
+// the weight gradients A^T dZ, whose k is the row.  The work-group's gradients
+// go to its own row of `part`; a work-group that takes more than one group of
+// rows starts each weight-gradient tile from what it left there.  Weights come
+// straight from L2 as matrix operands: every wave reads other tiles, so LDS
+// would not save a byte.  Operands round to BF16 at the matrix instructions, dZ
+// and the bias gradients are FP32 up to there, and the sums run in a fixed
+// order, so the gradients are the same on every run.
+//
+// Bound by the latency of its chain of layers (one work-group per CU, 13
+// barrier phases).  One GEMM launch per layer and direction, with the
+// activations, dZ and atomic gradient sums through memory, took 285 us per step
+// of 8192 rows; k_train and k_reduce take 40 us.
+struct TrainLds {
+  __bf16 act[kTrainRows][kHid + 8];      // [row][feature]: activations, then dZ
+  __bf16 at[4][kHid][kTrainRows + 8];    // [feature][row] of the four activations
+  __bf16 xt[32][kTrainRows + 8];         // [input][row], rows above the five inputs zero
+  __bf16 dzt[kHid][kTrainRows + 8];      // [feature][row] of dZ
+  float w5[kHid];                        // W5, rounded to BF16
+  float dT[kTrainRows];
+  float sum[2][4];
+};
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+
+// 32 values of feature f (both row tiles) into the two LDS layouts
+__device__ __forceinline__ void train_store(TrainLds& S, __bf16 (*t)[kTrainRows + 8], int f, int g,
+                                            const floatx16* v) {
+#pragma unroll
+  for (int rt = 0; rt < 2; rt++) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int row = 32 * rt + 8 * q + 4 * g;
+      bf16x4 x;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        x[j] = (__bf16)v[rt][4 * q + j];
+        S.act[row + j][f] = x[j];
+      }
+      *reinterpret_cast<bf16x4*>(&t[f][row]) = x;
+    }
+  }
+}
+
+// acc[rt] += S.act rows of tile rt times the 128 x 32 operand tile b
+__device__ __forceinline__ void train_mfma(const TrainLds& S, const bf16x8* __restrict__ b, int lane,
+                                           floatx16* acc) {
+  const int c = lane & 31, g = lane >> 5;
+  bf16x8 w[8];
+#pragma unroll
+  for (int ks = 0; ks < 8; ks++) w[ks] = b[64 * ks + lane];
+#pragma unroll
+  for (int ks = 0; ks < 8; ks++) {
+#pragma unroll
+    for (int rt = 0; rt < 2; rt++) {
+      const bf16x8 a = *reinterpret_cast<const bf16x8*>(&S.act[32 * rt + c][16 * ks + 8 * g]);
+      acc[rt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, w[ks], acc[rt], 0, 0, 0);
+    }
+  }
+}
+
+// A phase boundary of k_train.  The scheduling barrier keeps the next phase's
+// loads behind it: hoisted, the weights of every layer would sit in registers.
+__device__ __forceinline__ void train_sync() {
+  __syncthreads();
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+__device__ __forceinline__ float wave_sum_f(float v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
+
+__global__ void __launch_bounds__(kThreads, 1)
+k_train(const float* __restrict__ p, const NetImage* __restrict__ img, int n,
+        const float* __restrict__ X, const float* __restrict__ Y, float* __restrict__ part,
+        float* __restrict__ part_loss) {
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  TrainLds& S = *reinterpret_cast<TrainLds*>(lds_raw);
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  int c = lane & 31, g = lane >> 5, f = 32 * w + c;
+  const int off_w5 = fused_b(3) + kHid;
+  float* __restrict__ out = part + (size_t)blockIdx.x * kPartStride;
+  if (t < kHid) S.w5[t] = (float)(__bf16)p[off_w5 + t];
+  for (int q = t; q < 32 * (kTrainRows + 8); q += kThreads) (&S.xt[0][0])[q] = (__bf16)0.0f;
+  const float b5 = p[off_w5 + kHid], inv_n = 2.0f / (float)n;
+  const bf16x8 w1 = *reinterpret_cast<const bf16x8*>(&img->w1f[w][lane][0]);
+  float bias[4], db[4];
+#pragma unroll
+  for (int l = 0; l < 4; l++) {
+    bias[l] = p[fused_b(l) + f];
+    db[l] = 0.0f;
+  }
+  float dw5 = 0.0f, db5 = 0.0f, loss = 0.0f;
+  const int groups = (n + kTrainRows - 1) / kTrainRows;
+  for (int gr = blockIdx.x; gr < groups; gr += gridDim.x) {
+    const bool first = gr == (int)blockIdx.x;
+    const int base = gr * kTrainRows;
+    // opaque to the compiler, or it keeps every layer's weights and every
+    // address of the loop in registers across the groups, and spills
+    const NetImage* im = img;
+    asm volatile("" : "+s"(im), "+v"(c), "+v"(g), "+v"(f));
+    train_sync();  // xt cleared; the last group's reads done
+    // layer 1: K = 5 in one k-step of 16
+    bf16x8 xa[2];
+    floatx16 z[4][2];
+#pragma unroll
+    for (int rt = 0; rt < 2; rt++) {
+      const int r = base + 32 * rt + c;
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        float v = 0.0f;
+        if (j < kIn && g == 0 && r < n) v = X[(size_t)r * kIn + j];
+        xa[rt][j] = (__bf16)v;
+      }
+      if (w == 0 && g == 0)
+#pragma unroll
+        for (int j = 0; j < kIn; j++) S.xt[j][32 * rt + c] = xa[rt][j];
+#pragma unroll
+      for (int i = 0; i < 16; i++) z[0][rt][i] = bias[0];
+      z[0][rt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[rt], w1, z[0][rt], 0, 0, 0);
+    }
+    floatx16 a[2];
+#pragma unroll
+    for (int l = 0; l < 4; l++) {
+      if (l > 0) {
+#pragma unroll
+        for (int rt = 0; rt < 2; rt++)
+#pragma unroll
+          for (int i = 0; i < 16; i++) z[l][rt][i] = bias[l];
+        train_mfma(S, reinterpret_cast<const bf16x8*>(&im->wf[l - 1][w][0][0][0]), lane, z[l]);
+        train_sync();  // the layer's input is read
+      }
+#pragma unroll
+      for (int rt = 0; rt < 2; rt++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+          const float v = z[l][rt][i], sg = sigmoid(v);
+          a[rt][i] = v * sg;
+          z[l][rt][i] = sg * (1.0f + v * (1.0f - sg));  // silu'(z), all the way back needs
+        }
+      train_store(S, S.at[l], f, g, a);
+      train_sync();
+    }
+    // layer 5 and the loss: four threads per row, 32 features each
+    {
+      const int row = t >> 2, q = t & 3;
+      float s = 0.0f;
+#pragma unroll
+      for (int x = 0; x < 4; x++) {
+        const bf16x8 v = *reinterpret_cast<const bf16x8*>(&S.act[row][32 * q + 8 * x]);
+#pragma unroll
+        for (int j = 0; j < 8; j++) s = fmaf((float)v[j], S.w5[32 * q + 8 * x + j], s);
+      }
+      s += __shfl_xor(s, 1, 64);
+      s += __shfl_xor(s, 2, 64);
+      float r = 0.0f;
+      if (base + row < n) r = (s + b5) - Y[base + row];
+      if (q == 0) {
+        S.dT[row] = inv_n * r;  // the gradient of the mean squared error
+        db5 += inv_n * r;
+        loss += r * r;
+      }
+    }
+    train_sync();
+    // dW5 = A4^T dT: two threads per feature, 32 rows each
+    {
+      const int fe = t >> 1, h = t & 1;
+#pragma unroll
+      for (int x = 0; x < 4; x++) {
+        const bf16x8 v = *reinterpret_cast<const bf16x8*>(&S.at[3][fe][32 * h + 8 * x]);
+#pragma unroll
+        for (int j = 0; j < 8; j++) dw5 = fmaf((float)v[j], S.dT[32 * h + 8 * x + j], dw5);
+      }
+    }
+    // dZ4 = dT W5^T silu'(Z4)
+    const float w5 = S.w5[f];
+#pragma unroll
+    for (int rt = 0; rt < 2; rt++)
+#pragma unroll
+      for (int i = 0; i < 16; i++) {
+        const int row = 32 * rt + 8 * (i >> 2) + 4 * g + (i & 3);
+        a[rt][i] = S.dT[row] * w5 * z[3][rt][i];
+        db[3] += a[rt][i];
+      }
+    train_store(S, S.dzt, f, g, a);
+    train_sync();
+#pragma unroll
+    for (int l = 3; l >= 0; l--) {
+      // dW = A^T dZ: input tile w against the four output tiles (layer 1: the
+      // inputs against output tile w)
+      if (l > 0) {
+        bf16x8 av[4];
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++)
+          av[ks] = *reinterpret_cast<const bf16x8*>(&S.at[l - 1][f][16 * ks + 8 * g]);
+#pragma unroll
+        for (int ot = 0; ot < 4; ot++) {
+          float* o = out + fused_w(l) + (32 * w + 4 * g) * kHid + 32 * ot + c;
+          floatx16 acc;
+#pragma unroll
+          for (int i = 0; i < 16; i++)
+            acc[i] = first ? 0.0f : o[(8 * (i >> 2) + (i & 3)) * kHid];
+#pragma unroll
+          for (int ks = 0; ks < 4; ks++) {
+            const bf16x8 b =
+                *reinterpret_cast<const bf16x8*>(&S.dzt[32 * ot + c][16 * ks + 8 * g]);
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[ks], b, acc, 0, 0, 0);
+          }
+#pragma unroll
+          for (int i = 0; i < 16; i++) o[(8 * (i >> 2) + (i & 3)) * kHid] = acc[i];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        // dZ of the layer below
+#pragma unroll
+        for (int rt = 0; rt < 2; rt++)
+#pragma unroll
+          for (int i = 0; i < 16; i++) a[rt][i] = 0.0f;
+        train_mfma(S, reinterpret_cast<const bf16x8*>(&im->wb[l - 1][w][0][0][0]), lane, a);
+        train_sync();  // dZ is read
+#pragma unroll
+        for (int rt = 0; rt < 2; rt++)
+#pragma unroll
+          for (int i = 0; i < 16; i++) {
+            a[rt][i] *= z[l - 1][rt][i];
+            db[l - 1] += a[rt][i];
+          }
+        train_store(S, S.dzt, f, g, a);
+        train_sync();
+      } else {
+        floatx16 acc;
+        float* o = out + f;
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[i] = 0.0f;
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++) {
+          const bf16x8 av = *reinterpret_cast<const bf16x8*>(&S.xt[c][16 * ks + 8 * g]);
+          const bf16x8 b = *reinterpret_cast<const bf16x8*>(&S.dzt[f][16 * ks + 8 * g]);
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, b, acc, 0, 0, 0);
+        }
+        // inputs 0..3 are elements 0..3 of lane group 0, input 4 element 0 of group 1
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          if (g == 0 || i == 0) {
+            float* q = o + (4 * g + i) * kHid;
+            *q = (first ? 0.0f : *q) + acc[i];
+          }
+      }
+    }
+  }
+#pragma unroll
+  for (int l = 0; l < 4; l++) {
+    const float v = db[l] + __shfl_xor(db[l], 32, 64);
+    if (g == 0) out[fused_b(l) + f] = v;
+  }
+  dw5 += __shfl_xor(dw5, 1, 64);
+  if ((t & 1) == 0) out[off_w5 + (t >> 1)] = dw5;
+  loss = wave_sum_f(loss);
+  db5 = wave_sum_f(db5);
+  if (lane == 0) {
+    S.sum[0][w] = loss;
+    S.sum[1][w] = db5;
+  }
+  __syncthreads();
+  if (t == 0) {
+    part_loss[blockIdx.x] = (S.sum[0][0] + S.sum[0][1]) + (S.sum[0][2] + S.sum[0][3]);
+    out[off_w5 + kHid] = (S.sum[1][0] + S.sum[1][1]) + (S.sum[1][2] + S.sum[1][3]);
+  }
+}
+
+hipError_t train_setup() {
+  return hipFuncSetAttribute((const void*)k_train, hipFuncAttributeMaxDynamicSharedMemorySize,
+                             (int)sizeof(TrainLds));
+}
+
+// Gradient i = the sum of the work-groups' shares, each wave a quarter of them
+// in order; with Adam's moments the parameter and its places in the images
+// follow at once.  Bound by the read of the shares (26 MB for 8192 rows, mostly
+// from L2 and the memory-side cache).
+__global__ void __launch_bounds__(kThreads)
+k_reduce(int blocks, const float* __restrict__ part, const float* __restrict__ part_loss,
+         float* __restrict__ p, float* __restrict__ grads, float* __restrict__ loss, Adam adam,
+         NetImage* __restrict__ img) {
+  __shared__ float s_sum[kThreads / 64][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int i = blockIdx.x * 64 + lane;
+  const int total = fused_b(3) + 2 * kHid + 1;
+  float s = 0.0f;
+  if (i < total) {
+    const float* q = part + i;
+    int b = w;
+    for (; b + 28 < blocks; b += 32) {
+      float v[8];
+#pragma unroll
+      for (int x = 0; x < 8; x++) v[x] = q[(size_t)(b + 4 * x) * kPartStride];
+#pragma unroll
+      for (int x = 0; x < 8; x++) s += v[x];
+    }
+    for (; b < blocks; b += 4) s += q[(size_t)b * kPartStride];
+  }
+  s_sum[w][lane] = s;
+  if (blockIdx.x == 0 && w == 1) {
+    float l = 0.0f;
+    for (int b = lane; b < blocks; b += 64) l += part_loss[b];
+    l = wave_sum_f(l);
+    if (lane == 0) *loss = l;
+  }
+  __syncthreads();
+  if (w != 0 || i >= total) return;
+  const float gi = (s_sum[0][lane] + s_sum[1][lane]) + (s_sum[2][lane] + s_sum[3][lane]);
+  grads[i] = gi;
+  if (!adam.m) return;
+  const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
+  const float mi = b1 * adam.m[i] + (1.0f - b1) * gi;
+  const float vi = b2 * adam.v[i] + (1.0f - b2) * gi * gi;
+  adam.m[i] = mi;
+  adam.v[i] = vi;
+  const float v = p[i] - adam.lr * (mi / adam.c1) / (sqrtf(vi / adam.c2) + eps);
+  p[i] = v;
+  pack_param(*img, i, v);
+}
+
+hipError_t launch_train(const float* p, NetImage* img, int blocks, int n, const float* X,
+                        const float* Y, float* part, float* part_loss, hipStream_t st) {
+  hipLaunchKernelGGL(k_train, dim3(blocks), dim3(kThreads), sizeof(TrainLds), st, p, img, n, X, Y,
+                     part, part_loss);
+  return hipGetLastError();
+}
+
+hipError_t launch_reduce(int blocks, const float* part, const float* part_loss, float* p,
+                         float* grads, float* loss, const Adam& adam, NetImage* img,
+                         hipStream_t st) {
+  const int n = Layout().total;
+  hipLaunchKernelGGL(k_reduce, dim3((n + 63) / 64), dim3(kThreads), 0, st, blocks, part, part_loss,
+                     p, grads, loss, adam, img);
+  return hipGetLastError();
 }
 
 __global__ void k_eval_points(amca_surrogate_desc d, amca_scan s, int n, const double* __restrict__ p,
