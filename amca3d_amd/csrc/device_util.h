@@ -122,14 +122,14 @@ __device__ __forceinline__ void stage_flush_or(const WordStage& s, unsigned long
     if (s.key[i] >= 0) atomicOr(&words[s.key[i]], s.bits[i]);
 }
 
-// The 26 neighbour bits of interior cell (i, j, k) from word `kWord` of the
-// brick map, in slot order (k, j, i, centre skipped).  The 3x3x3 block spans
+// The 26 neighbour bits of interior cell (i, j, k) from the words load(brick), or
+// (brick_bits26) word `kWord` of the brick map, in slot order (k, j, i, centre skipped).  The 3x3x3 block spans
 // bricks bx0..bx1 (bx1 = bx0 or bx0 + 1) per axis: the 8 corner words are
 // loaded once and each of the 9 rows takes its 3 bits from the two x-adjacent
 // nibbles.
-template <int kWord, bool kCoherent>
-__device__ __forceinline__ unsigned brick_bits26(const DevParams& P, const unsigned long long* bm,
-                                                 int i, int j, int k) {
+template <class Load>
+__device__ __forceinline__ unsigned block_bits26(const DevParams& P, int i, int j, int k,
+                                                 Load&& load) {
   const int bx0 = (i - 1) >> 2, bx1 = (i + 1) >> 2;
   const int by0 = (j - 1) >> 2, by1 = (j + 1) >> 2;
   const int bz0 = (k - 1) >> 2, bz1 = (k + 1) >> 2;
@@ -139,8 +139,7 @@ __device__ __forceinline__ unsigned brick_bits26(const DevParams& P, const unsig
     const int bx = (q & 1) ? bx1 : bx0;
     const int by = (q & 2) ? by1 : by0;
     const int bz = (q & 4) ? bz1 : bz0;
-    const unsigned long long* p = bm + 2 * ((bz * P.nbY + by) * P.nbX + bx) + kWord;
-    w[q] = kCoherent ? ld_coherent(p) : *p;
+    w[q] = load((bz * P.nbY + by) * P.nbX + bx);
   }
   const int xs = (i - 1) & 3;  // first x of the block inside brick bx0
   unsigned m = 0;
@@ -169,6 +168,23 @@ __device__ __forceinline__ unsigned brick_bits26(const DevParams& P, const unsig
     }
   }
   return m;
+}
+template <int kWord, bool kCoherent>
+__device__ __forceinline__ unsigned brick_bits26(const DevParams& P, const unsigned long long* bm,
+                                                 int i, int j, int k) {
+  return block_bits26(P, i, j, k, [&](int b) {
+    const unsigned long long* p = bm + 2 * b + kWord;
+    return kCoherent ? ld_coherent(p) : *p;
+  });
+}
+// The neighbours that are liquid and claimed (both words of a brick in one load).
+__device__ __forceinline__ unsigned taken_bits26(const DevParams& P, const DevBuffers& B, int i,
+                                                 int j, int k) {
+  const ulonglong2* m = reinterpret_cast<const ulonglong2*>(B.bmap);
+  return block_bits26(P, i, j, k, [&](int b) {
+    const ulonglong2 u = m[b];
+    return u.x & u.y;
+  });
 }
 
 // ---- per-cell slots (brick-major, the claim words' order) -----------------
@@ -290,10 +306,10 @@ __device__ __forceinline__ void chunk_of(int n, int bid, int nb, int tile, int& 
 
 // Block index with the eight XCDs each owning a contiguous range: work-groups
 // are dispatched to XCDs round-robin, so block b runs on XCD b % 8.
-__device__ __forceinline__ int xcd_block() {
-  const int nb = gridDim.x;
-  if (nb & 7) return blockIdx.x;
-  return (blockIdx.x & 7) * (nb >> 3) + (blockIdx.x >> 3);
+__device__ __forceinline__ int xcd_of(int b, int nb) {
+  if (nb & 7) return b;
+  return (b & 7) * (nb >> 3) + (b >> 3);
 }
+__device__ __forceinline__ int xcd_block() { return xcd_of(blockIdx.x, gridDim.x); }
 
 }  // namespace amca

@@ -3,8 +3,8 @@
 // The reference keeps the grid as raw host arrays owned by
 // CellularAutomataManager (CellularAutomataManager.cpp:303-326) and one heap
 // Grain per solid cell.  Here the grid and the per-cell envelopes live in HBM
-// for the lifetime of the handle, a step is a fixed sequence of six kernel
-// launches that reads every scalar it needs from device memory, and the host
+// for the lifetime of the handle, a step is a fixed sequence of seven or twelve
+// kernel launches that reads every scalar it needs from device memory, and the host
 // only reads the counters back between batches of steps.
 #include <hip/hip_runtime.h>
 
@@ -23,6 +23,8 @@
 
 namespace {
 
+constexpr long long kFusedCells = 1ll << 24;
+
 thread_local std::string g_last_error;
 
 amca_status fail(amca_status st, const std::string& msg) {
@@ -40,7 +42,8 @@ amca_status fail(amca_status st, const std::string& msg) {
 enum KernelId {
   K_NUCLEATE = 0, K_CLAIM, K_RESOLVE, K_EMIT, K_TAIL, K_IDSCAN, K_COMPACT, K_CNT, K_COUNT
 };
-// named as the kernels are, so event times line up with a kernel trace
+// named as the kernels are, so event times line up with a kernel trace (the short
+// step's k_wake_claim counts as k_claim)
 const char* kKernelNames[K_COUNT] = {"k_nucleate", "k_claim",   "k_resolve", "k_emit",
                                      "k_tail",     "k_idscan",  "k_compact", "k_count"};
 
@@ -176,6 +179,15 @@ amca_status enqueue_step(amca_domain* d) {
   const amca::DevBuffers& B = d->B;
   hipStream_t s = d->stream;
   AMCA_TRY(timed(d, K_NUCLEATE, [&] { return amca::launch_nucleate(P, B, d->nuc_blocks, s); }));
+  if (P.fused) {
+    AMCA_TRY(timed(d, K_CLAIM, [&] { return amca::launch_wake_claim(P, B, s); }));
+    AMCA_TRY(timed(d, K_RESOLVE, [&] { return amca::launch_resolve(P, B, 0, P.cmp_blocks, s); }));
+    AMCA_TRY(timed(d, K_IDSCAN, [&] { return amca::launch_idscan(P, B, 0, P.cmp_blocks, s); }));
+    AMCA_TRY(timed(d, K_EMIT, [&] { return amca::launch_emit(P, B, 0, P.cmp_blocks, s); }));
+    AMCA_TRY(timed(d, K_CLAIM, [&] { return amca::launch_claim(P, B, 1, d->list_blocks, s); }));
+    AMCA_TRY(timed(d, K_TAIL, [&] { return amca::launch_tail(P, B, s); }));
+    return AMCA_OK;
+  }
   AMCA_TRY(timed(d, K_CNT, [&] { return amca::launch_count(P, B, d->cmp_blocks, s); }));
   AMCA_TRY(timed(d, K_COMPACT, [&] { return amca::launch_compact(P, B, d->cmp_blocks, s); }));
   for (int wave = 0; wave < 2; wave++) {
@@ -328,19 +340,20 @@ amca_status amca_domain_create(const amca_domain_desc* desc, int32_t orient_capa
   ALLOC(B.bmap, 2 * (size_t)nB);
   ALLOC(B.amap, (size_t)nB);
   ALLOC(B.rec, 64 * (size_t)nB);
-  ALLOC(B.sL, 64 * (size_t)nB);
-  ALLOC(B.skey, 64 * (size_t)nB);
+  ALLOC(B.wake, 64 * (size_t)nB);
+  ALLOC(B.inc, amca::kRing);
+  ALLOC(B.awk, (size_t)nB);
   ALLOC(B.genv, N);
   ALLOC(B.gco, N);
-  ALLOC(B.alist, N);
-  ALLOC(B.plist, N);
+  ALLOC(B.alist, 64 * (size_t)nB);
+  ALLOC(B.plist, 64 * (size_t)nB);
   ALLOC(B.cnt, N + 64);  // the id scan reads whole 16-byte groups past the last id
   ALLOC(B.coff, N);
   ALLOC(B.idtot, amca::kMaxIdsBlocks);
   ALLOC(B.cmptot, amca::kMaxBlocks);
   ALLOC(B.listW[0], N);
   ALLOC(B.listW[1], N);
-  ALLOC(B.masks, N);
+  ALLOC(B.masks, 64 * (size_t)nB);
   ALLOC(B.l2g, 9 * (size_t)std::max(orient_capacity, 1));
   ALLOC(B.lb_flag, (size_t)amca::kLbSites * amca::kMaxBlocks);
   ALLOC(B.lb_agg, (size_t)amca::kLbSites * amca::kMaxBlocks);
@@ -368,13 +381,23 @@ amca_status amca_domain_create(const amca_domain_desc* desc, int32_t orient_capa
   d->list_blocks = (int)std::max(8LL, std::min<long long>((want + 7) / 8 * 8, 16LL * cus));
   d->emit_blocks = (int)std::max(8LL, std::min<long long>((want + 7) / 8 * 8, std::min(16LL * cus, (long long)amca::kMaxBlocks)));
   d->nuc_blocks = 1;
-  // id scan and compaction: eight blocks per CU at most (each block's tiles
-  // run one after another), at least 32 K ids / 512 bricks per block
+  // id scan: eight blocks per CU at most (each block's tiles run one after
+  // another), at least 32 K ids per block
   d->ids_blocks = (int)std::max(1LL, std::min<long long>((P.N + 32767) / 32768,
                                                          std::min(8LL * cus, (long long)amca::kMaxIdsBlocks)));
   P.ids_blocks = d->ids_blocks;
-  d->cmp_blocks = (int)std::max(1LL, std::min<long long>((nB + 511) / 512,
+  // compaction and retirement: the 64-brick pieces of the grid over at most eight
+  // blocks per CU
+  d->cmp_blocks = (int)std::max(1LL, std::min<long long>((nB + 63) / 64,
                                                          std::min(8LL * cus, (long long)amca::kMaxBlocks)));
+  P.cmp_blocks = d->cmp_blocks;
+  // The short step (see plain_step.hip) for grids of up to kFusedCells whose grains
+  // grow at most a quarter of a cell per step (dt <= time_step_factor h / v), which
+  // keeps captures by wave 1's fresh envelopes rare: k_tail takes those with one
+  // work-group.  Whole runs, short against long form: 131x97x67 46 against 68 us a
+  // step, 256^3 114 against 135; at 512^3 k_tail's one work-group takes 730 us
+  // of 1050 (long form 347).
+  P.fused = P.N <= kFusedCells && desc->time_step_factor <= 0.25 ? 1 : 0;
   if (amca::env_int("AMCA_DOMAIN_GRAPH_STEPS", 0, 1024, &d->graph_steps) < 0) {
     delete d;
     return fail(AMCA_ERR_INVALID, "AMCA_DOMAIN_GRAPH_STEPS must be an integer in [0, 1024]");
@@ -806,7 +829,8 @@ amca_status batch_apply_schedule(amca_batch* b) {
   std::vector<int4> mn, ml, me, ms, mi, mc;
   build_map(order, nn, b->sched.interleave, mn);
   build_map(order, ni, b->sched.interleave, mi);
-  for (auto& m : mi) m.w = ne[m.x];  // the id scan sums the domain's k_resolve blocks
+  // the id scan sums the domain's k_resolve blocks (short step: of wave 0 only)
+  for (auto& m : mi) m.w = b->L.fused ? nc[m.x] : ne[m.x];
   build_map(order, nc, b->sched.interleave, mc);
   build_map(order, nl, b->sched.interleave, ml);
   build_map(order, ne, b->sched.interleave, me);
@@ -997,8 +1021,11 @@ amca_status amca_batch_create(amca_domain* const* doms, int32_t n, amca_batch** 
       if (hipStreamSynchronize(b->doms[i]->stream) != hipSuccess) { st = fail(AMCA_ERR_HIP, "sync"); break; }
       P[i] = b->doms[i]->P;
       B[i] = b->doms[i]->B;
+      b->L.fused = (i == 0 || b->L.fused) && P[i].fused;
     }
     if (st != AMCA_OK) break;
+    // one launch sequence for the batch: the short one if every domain takes it
+    for (auto& p : P) p.fused = b->L.fused;
     if (hipMalloc(&b->dP, sizeof(amca::DevParams) * n) != hipSuccess ||
         hipMalloc(&b->dB, sizeof(amca::DevBuffers) * n) != hipSuccess ||
         hipMalloc(&b->status, sizeof(int4) * n) != hipSuccess ||

@@ -29,6 +29,9 @@ struct DevParams {
   int nbX, nbY, nbZ;      // 4x4x4-cell bricks per axis of the liquid / claimed map
   FastDiv fdX, fdY;       // division by nbX and by nbY
   int ids_blocks;         // blocks of the id scan (k_idscan)
+  int cmp_blocks;         // blocks of k_count / k_compact, and of the retirement in k_resolve
+  int fused;              // the short step: k_wake_claim instead of k_count, k_compact and wave 0's
+                          // k_claim, wave 1's captures in k_tail
 };
 
 // Mutable scalars that live on the device, so that a whole step (or many
@@ -45,6 +48,10 @@ struct DevCounters {
   int site_sel;           // which site buffer holds the live sites
   int n_grains, n_orient;
   int nA_in, nA_out;      // active list lengths (input / survivors)
+  double S;               // growth since the last refresh step, the running step's included
+  int Sq;                 // S in kWakeUnits per cell, rounded down, at most kWakeLate
+  int force;              // the running step is a refresh step: every active grain is awake
+  int n_awake;            // length of wave 0's list
   int nW[2];              // capture-wave list lengths
   int n_sites;
   int step_nuc, step_cap, step_nA0;
@@ -59,6 +66,10 @@ struct DevCounters {
   // ids of wave 0's claiming grains (min, max), spread over 64 slots by k_claim
   // block so that blocks rarely meet at one address
   int claim_lo[64], claim_hi[64];
+  // wave 1: whether any of its grains claimed a cell, and its grains without a
+  // liquid neighbour, spread over 64 slots
+  int w1_claims;
+  int w1_ret[64];
 };
 
 struct StepLogRow {
@@ -69,12 +80,13 @@ struct StepLogRow {
   int n_sites;
 };
 
-// The grain in a cell's slot: its centre and (id, orientation).  The
-// half-diagonal L sits in an array of its own, since every step rewrites it
-// for each active grain while the rest stays as written at capture.
-struct alignas(32) SlotRec {
-  double x, y, z;
-  int id, o;
+// The grain in a cell's slot: its centre, its half-diagonal L before the growth
+// of step `stamp` and later ones, id and orientation: half a 128-byte line, all
+// that its tests, its children and its end read or write.
+struct alignas(64) SlotRec {
+  double x, y, z, L;
+  int id, o, stamp, pad;
+  double spare[2];
 };
 
 // Device buffers of one domain (all owned by the handle).
@@ -84,36 +96,53 @@ struct alignas(32) SlotRec {
 // (claim_index).  Per brick: two 64-bit words of the 1-bit maps, [2b] liquid
 // and [2b+1] claimed, and the active word (a grain whose cell has the bit set
 // is on the reference's active list).  Per slot: the grain occupying the cell
-// (record, L, id) and the claim word of the capture waves.  Steps read and
-// write only these: wave 0 walks the active slots in brick order, so
-// neighbouring entries share map words and record lines, and the lists of
-// waves >= 1 hold slots in grain-id order.  The reference's layouts
-// (cellGrainID_ / cellOrientationID_ on the ghosted grid, x fastest; records
-// by grain id) are materialized from the slots when a download asks for them.
+// (its record) and the claim word of the capture waves.  Steps read and write
+// only these: wave 0 walks the awake slots in brick order, so neighbouring
+// entries share map words, and the lists of waves >= 1 hold slots in grain-id
+// order.  The reference's layouts (cellGrainID_ / cellOrientationID_ on the
+// ghosted grid, x fastest; records by grain id) are materialized from the slots
+// when a download asks for them.
+//
+// Sleep.  Every active grain grows by the same increment in a step, so the growth
+// it needs to enclose its nearest liquid neighbour is known when it is tested:
+// the growth clock S (DevCounters) at which it can next capture goes to `wake`,
+// and until then a step does not touch it (about one active grain in five is
+// awake in a step).  Its L is worked out when it wakes, retires or is downloaded,
+// by adding the increments of the steps since `stamp` one by one, in order: the
+// additions of Grain::grow, so the same value to the bit.  The liquid set only
+// shrinks, so a sleeping grain can never capture earlier than its clock says.
+// At a refresh step (every kRefresh steps, or when S nears its range) all active
+// grains are awake and take their L anew, and S restarts from zero, so no replay
+// outlasts the ring of increments.
 struct DevBuffers {
   int* gid;               // cellGrainID_ [NG], materialized for downloads
   int* oid;               // cellOrientationID_ [NG], materialized for downloads
   int* claim;             // smallest claiming grain id per slot, INT_MAX when free [64 nB]
   unsigned long long* bmap;  // brick words: liquid, claimed [2 nB]
   unsigned long long* amap;  // brick words: active grains [nB]
-  SlotRec* rec;           // centre, id and orientation of the grain in each slot [64 nB]
-  double* sL;             // half-diagonal L of the grain in each slot [64 nB]
-  int* skey;              // grain id of each slot (the id of rec, packed alone) [64 nB]
+  SlotRec* rec;           // the grain in each slot [64 nB]
+  unsigned short* wake;   // growth clock (kWakeUnits per cell, rounded down) from which the
+                          // active grain in the slot may capture a cell [64 nB]
+  double* inc;            // growth increments of the last kRing steps, by step [kRing]
+  unsigned long long* awk;  // brick words: active grains awake in the running step [nB]
   double4* genv;          // envelope by grain id, materialized for downloads [N]
   int2* gco;              // grain -> (cell, orientation), materialized for downloads [N]
-  int* alist;             // wave-0 list: active slots in brick order [N]
+  int* alist;             // wave-0 list: awake slots in brick order (short step: one segment per
+                          // k_wake_claim block, from the block's first slot) [64 nB]
   int4* plist;            // wave-0 capturing grains: (id, slot, captured slots), one segment
-                          // per k_resolve block from its first list entry [N]
+                          // per k_resolve block from its first list entry [64 nB]
   unsigned char* cnt;     // captures per grain id, nonzero only inside a wave-0 step [N]
   int* coff;              // first child (wave-relative) per capturing grain id [N]
   unsigned* idtot;        // wave-0 captures per id-scan block [kMaxIdsBlocks]
-  unsigned* cmptot;       // active cells per compaction block [kMaxBlocks]
+  unsigned* cmptot;       // awake grains per compaction block [kMaxBlocks]
   int* listW[2];          // capture-wave lists (slots, in grain-id order) [N]
-  unsigned long long* masks;  // per wave entry: liquid bits | inside bits << 32 [N]
+  unsigned long long* masks;  // per wave entry: inside bits << 32 | grain id (wave 0) or liquid
+                              // bits (waves >= 1) [64 nB]
   int* site_cell[2];      // live nucleation sites, ascending cell, ping-pong
   double* site_dt[2];
   double* l2g;            // orientation table, 9 doubles per row
-  unsigned* lb_flag;      // look-back state: epoch<<2 | state   [kLbSites * kMaxBlocks]
+  unsigned* lb_flag;      // look-back state: epoch<<2 | state; from kStatBase the grains retired
+                          // per block [kLbSites * kMaxBlocks]
   unsigned long long* lb_agg;
   unsigned long long* lb_pref;
   StepLogRow* log;
@@ -126,6 +155,13 @@ constexpr int kMaxBlocks = 4096;  // blocks of a look-back kernel
 constexpr int kLbSites = 2;       // look-back arrays: [0] k_nucleate's look-back, [1] k_resolve's
                                   // per-block statistics (lb_agg, lb_pref at kStatBase + block)
 constexpr int kStatBase = kMaxBlocks;
+constexpr int kRefresh = 2048;    // most steps between refresh steps
+constexpr int kRing = 2 * kRefresh;  // growth increments kept
+// Wake clocks: 1/1024 of a cell (a step's growth is some thousandths to a fifth of
+// a cell, so rounding down wakes a grain about a step early at most); S is
+// restarted from kWakeSpan cells, within the 16 bits.
+constexpr int kWakeUnits = 1024, kWakeSpan = 60;
+constexpr int kWakeLate = 65534, kWakeNever = 65535;
 constexpr int kMaxIdsBlocks = 2048;  // blocks of the id scan (a k_resolve block keeps one count each)
 
 inline FastDiv make_fastdiv(unsigned d) {
@@ -147,10 +183,13 @@ hipError_t launch_claim(const DevParams& P, const DevBuffers& B, int wave, int b
 // k_resolve and k_emit with the same `blocks` (<= kMaxBlocks list chunks)
 hipError_t launch_resolve(const DevParams& P, const DevBuffers& B, int wave, int blocks,
                           hipStream_t s);
-// wave 0's list: the active slots in brick order (k_count: active cells per
+// wave 0's list: the awake slots in brick order (k_count: awake grains per
 // block of bricks, then k_compact over the same blocks)
 hipError_t launch_count(const DevParams& P, const DevBuffers& B, int blocks, hipStream_t s);
 hipError_t launch_compact(const DevParams& P, const DevBuffers& B, int blocks, hipStream_t s);
+// the short step's list and claims of wave 0 (P.cmp_blocks blocks, as its
+// k_resolve and k_emit of wave 0)
+hipError_t launch_wake_claim(const DevParams& P, const DevBuffers& B, hipStream_t s);
 // child offsets of a wave's capturing grains, an exclusive scan over their
 // ids (P.ids_blocks blocks; `nres` = blocks of the wave's k_resolve, whose
 // statistics words it reads)
@@ -174,6 +213,7 @@ struct BatchLaunch {
   const int4* map_ids;   // id-scan geometry
   const int4* map_cmp;   // compaction geometry (k_count and k_compact)
   int n_nuc, n_list, n_emit, n_one, n_ids, n_cmp;
+  int fused;             // every domain takes the short step
 };
 hipError_t launch_batch_step(const BatchLaunch& L, hipStream_t s);
 // out[d] = (finished, error, step & 0x7fffffff, step >> 31) for each of n domains

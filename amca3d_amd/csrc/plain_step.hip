@@ -12,16 +12,23 @@
 // neighbour takes it; new ids follow (parent id, neighbour slot) order; a grain
 // stays active iff one of its liquid neighbours is outside its envelope and not
 // taken by a smaller id of the same wave.  The kernels compute exactly that:
-//   k_count/k_compact: wave 0's list, the active slots in brick order;
+//   k_count/k_compact: wave 0's list, the awake slots in brick order: the active
+//                     grains that have grown enough to capture a cell (the
+//                     others sleep, see DevBuffers);
 //   k_claim         : per wave entry, liquid test of the 26 neighbours on the
 //                     1-bit liquid map, envelope tests, and an atomicMin of the
 //                     grain id into each enclosed neighbour's claim word;
-//   k_resolve       : per entry, captured / keep decisions from the claims;
-//                     capturing grains go to a parent list with their counts;
+//   k_resolve       : per entry, captured decisions from the claims; capturing
+//                     grains go to a parent list with their counts.  In wave 0
+//                     a second set of blocks retires the active grains, awake or
+//                     not, that have no liquid neighbour left;
 //   k_idscan        : first child of each capturing grain, a scan over ids;
 //   k_emit          : the child records and the next wave's list;
 //   k_tail          : waves >= 2 (rare) in one work-group, then the time advance.
 // Waves 0 and 1 each run k_claim, k_resolve, k_idscan and k_emit.
+// On small grids a step is bound by its launches (about 4.5 us each, whatever
+// they do), and two shorter forms hold: k_wake_claim makes wave 0's list and tests
+// it in one launch, and k_tail also takes wave 1's captures, which are rare.
 // Claims need no reset: every claimed cell is captured in the same wave and is
 // never liquid again.
 #include <hip/hip_runtime.h>
@@ -95,14 +102,6 @@ __global__ void k_init_grid(DevParams P, DevBuffers B) {
 // exceeds its critical value nucleates with the next orientation row and the
 // next grain id; a non-liquid site is dropped.  Ranks come from the look-back
 // scan, so ids follow cell order exactly as in the reference loop.
-
-// Index of slot q's record.  A 128-byte line holds four 32-byte records; with
-// this order (x-bit 1 and y-bit 0 of the lane exchanged) they are a 2 x 2
-// patch of cells in x and y rather than a row of four in x, which holds more
-// cells of a growth front per line on average.
-__device__ __forceinline__ long long rec_slot(long long q) {
-  return (q & ~6ll) | ((q & 2) << 1) | ((q & 4) >> 1);
-}
 
 // Whether ghosted cell c is liquid: its bit in the brick map (ghost cells
 // never have one).
@@ -179,15 +178,15 @@ __device__ __forceinline__ void nucleate_body(const DevParams& P, const DevBuffe
         cell_ijk(P, c, ci, cj, ck);
         const int id = ng0 + r;
         const long long q = claim_index(P, ci, cj, ck);
-        SlotRec r;
+        SlotRec r{};
         r.x = centre_coord(P.x0, P.h, ci);
         r.y = centre_coord(P.y0, P.h, cj);
         r.z = centre_coord(P.z0, P.h, ck);
         r.id = id;
         r.o = o;
-        B.rec[rec_slot(q)] = r;
-        B.sL[q] = 0.0;
-        B.skey[q] = id;
+        r.stamp = (int)ctr->step;  // L = 0, and it grows in this step
+        B.rec[q] = r;
+        B.wake[q] = 0;  // awake
         brick_clear(P, B.bmap, 0, ci, cj, ck);
         atomicOr(&B.amap[q >> 6], 1ull << (q & 63));
       }
@@ -203,6 +202,7 @@ __device__ __forceinline__ void nucleate_body(const DevParams& P, const DevBuffe
     for (int q = threadIdx.x; q < 64; q += kBlock) {
       ctr->claim_lo[q] = INT_MAX;
       ctr->claim_hi[q] = -1;
+      ctr->w1_ret[q] = 0;
     }
   if (threadIdx.x == 0 && bid == nblk - 1) {
     const int nn = (int)(run >> 32);
@@ -236,8 +236,18 @@ __device__ __forceinline__ void nucleate_body(const DevParams& P, const DevBuffe
     double maxV = 1e-10;
     if (nA > 0 && v > maxV) maxV = v;
     const double a = P.tsf * P.h / maxV;
-    ctr->dt = (P.max_dt < a) ? P.max_dt : a;
+    const double dt = (P.max_dt < a) ? P.max_dt : a;
+    ctr->dt = dt;
     ctr->v = v;
+    // Grain::grow's increment of this step, and the growth clock
+    const double inc = dt * v;
+    B.inc[ctr->step & (kRing - 1)] = inc;
+    const double S = ctr->S + inc;
+    const int force = ((ctr->step & (kRefresh - 1)) == 0 || S > kWakeSpan * P.h) ? 1 : 0;
+    ctr->force = force;
+    ctr->S = force ? 0.0 : S;
+    ctr->Sq = force ? 0 : (int)(S * (kWakeUnits / P.h));
+    ctr->w1_claims = 0;
     ctr->tickets[0] = 0u;
   }
 }
@@ -246,28 +256,61 @@ __device__ __forceinline__ void nucleate_body(const DevParams& P, const DevBuffe
 // capture waves
 
 // Waves 0 and 1 run as "list waves" over many work-groups: wave 0 over the
-// active slots in brick order (k_count / k_compact), wave 1 over the slots of
+// awake slots in brick order (k_count / k_compact), wave 1 over the slots of
 // wave 0's children in the order wave 0's k_emit wrote them (parent blocks in
 // brick order).  The processing order of a wave does not change its outcome
 // (claims are an atomicMin, each entry's decision depends only on the claim
 // words); its children are numbered by an exclusive scan over the capturing
 // grains' ids (k_idscan).
-__device__ __forceinline__ void list_wave(const DevBuffers& B, int wave, const int*& list,
-                                          int& n) {
+// wave_chunk: block blk's entries [lo, hi) of the wave's list.
+__device__ __forceinline__ void cmp_range(const DevParams& P, int blk, int nblk, long long& lo,
+                                          long long& hi);
+__device__ __forceinline__ void wave_chunk(const DevParams& P, const DevBuffers& B, int wave,
+                                           int blk, int nblk, const int*& list, int& lo, int& hi) {
   const DevCounters* ctr = B.ctr;
-  if (wave == 0) {
-    list = B.alist;
-    n = ctr->nA_in;
-  } else {
-    list = B.listW[0];
-    n = ctr->nW[0];
+  list = wave == 0 ? B.alist : B.listW[0];
+  if (wave == 0 && P.fused) {
+    long long blo, bhi;
+    cmp_range(P, blk, nblk, blo, bhi);
+    lo = (int)(64 * blo);
+    hi = lo + (int)B.cmptot[blk];
+    return;
   }
+  chunk_of(wave == 0 ? ctr->n_awake : ctr->nW[0], blk, nblk, kBlock, lo, hi);
+}
+
+// L brought up to step `end` (exclusive) from `stamp`: the steps' increments
+// added in order, four loads at a time in flight.
+__device__ __forceinline__ double grow_to(const DevBuffers& B, double L, int stamp, int end) {
+  int s = stamp;
+  for (; s + 4 <= end; s += 4) {
+    const double a = B.inc[s & (kRing - 1)], b = B.inc[(s + 1) & (kRing - 1)];
+    const double c = B.inc[(s + 2) & (kRing - 1)], d = B.inc[(s + 3) & (kRing - 1)];
+    L += a;
+    L += b;
+    L += c;
+    L += d;
+  }
+  for (; s < end; s++) L += B.inc[s & (kRing - 1)];
+  return L;
+}
+
+// The growth clock at which a grain of half-diagonal L, tested at clock S, can
+// reach a neighbour at distance dmin > L, rounded down.  The sums behind S and L
+// differ by at most kRefresh roundings of values below kWakeSpan cells (2048 * 60 *
+// 2^-53 h, 1.4e-11 h), and the conversion to clock units by parts in 1e15.
+__device__ __forceinline__ unsigned short wake_clock(const DevParams& P, double S, double L,
+                                                     double dmin) {
+  const double t = (S + (dmin - L) - 1e-9 * P.h) * (kWakeUnits / P.h);
+  if (t < (double)kWakeLate) return (unsigned short)(t > 0.0 ? (int)t : 0);
+  return (unsigned short)(t < __builtin_inf() ? kWakeLate : kWakeNever);
 }
 
 // Envelope tests of grain g (orientation o, envelope e) at cell (ci, cj, ck)
 // against its liquid neighbours lm: each neighbour inside the envelope gets an
 // atomicMin of g into its claim word and its claimed bit.  Returns the inside
-// bits (none when L == 0: such an envelope captures nothing).
+// bits (none when L == 0: such an envelope captures nothing); dmin is the
+// distance of the nearest liquid neighbour outside (infinity: there is none).
 //
 // inside_envelope's arithmetic, reorganised without changing a value: along
 // each axis the neighbour centres sit at three offsets from the envelope
@@ -277,8 +320,9 @@ __device__ __forceinline__ void list_wave(const DevBuffers& B, int wave, const i
 // (its leading 0.0 + p is p up to the sign of a zero, which fabs drops).
 __device__ __forceinline__ unsigned claim_tests(const DevParams& P, const DevBuffers& B, int g,
                                                 int o, int ci, int cj, int ck, unsigned lm,
-                                                const double4& e, WordStage* st) {
-  if (lm == 0 || e.w == 0) return 0u;
+                                                const double4& e, WordStage* st, double& dmin) {
+  dmin = __builtin_inf();
+  if (lm == 0) return 0u;
   double r[9];
   const double* rp = B.l2g + 9 * (size_t)o;
 #pragma unroll
@@ -321,7 +365,11 @@ __device__ __forceinline__ unsigned claim_tests(const DevParams& P, const DevBuf
         const double lx = sx + pz[dk + 1][0];
         const double ly = sy + pz[dk + 1][1];
         const double lz = sz + pz[dk + 1][2];
-        if ((fabs(lx) + fabs(ly)) + fabs(lz) <= e.w) im |= 1u << s;
+        const double d = (fabs(lx) + fabs(ly)) + fabs(lz);
+        if (d <= e.w && e.w != 0)
+          im |= 1u << s;
+        else
+          dmin = fmin(dmin, d);
       }
     }
   }
@@ -339,30 +387,107 @@ __device__ __forceinline__ unsigned claim_tests(const DevParams& P, const DevBuf
   return im;
 }
 
-// The active slots in brick order.  k_count leaves the active-cell count of
-// each block of bricks; k_compact block b starts from the sum of the counts of
-// the blocks before it, and each thread lists its own brick's active slots
-// (bricks in 256-brick tiles, one block scan per tile).  The list's length is
-// the active count.
+// Inclusive prefix sum over the 64 lanes of a wave (every lane must call it).
+__device__ __forceinline__ unsigned wave_incl(unsigned v) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const unsigned u = __shfl_up(v, d, 64);
+    if (lane >= d) v += u;
+  }
+  return v;
+}
+
+// The awake slots in brick order.  k_count finds them (a brick's active grains
+// whose wake clock has come) and leaves their word per brick and their number
+// per block of bricks; k_compact block b starts from the sum of the counts of
+// the blocks before it, and each thread lists its own brick's awake slots
+// (bricks in 256-brick tiles, one block scan per tile).  k_count takes one brick
+// per lane, whose 64 clocks are one line: a wave per brick, one slot per lane,
+// was bound by its 20 instructions per brick (64 us a step at 2.1 M bricks against
+// 20 us).
 __device__ __forceinline__ void cmp_range(const DevParams& P, int blk, int nblk, long long& lo,
                                           long long& hi) {
   const long long nB = (long long)P.nbX * P.nbY * P.nbZ;
-  const long long per = ((nB + nblk - 1) / nblk + kBlock - 1) / kBlock * kBlock;
+  const long long per = ((nB + nblk - 1) / nblk + 63) / 64 * 64;
   lo = (long long)blk * per < nB ? (long long)blk * per : nB;
   hi = lo + per < nB ? lo + per : nB;
 }
 
+// The bricks [lo, hi) of wave wv of block blk: a quarter of the block's, whole
+// 16-brick pieces.
+__device__ __forceinline__ void cmp_wave_range(const DevParams& P, int blk, int nblk, int wv,
+                                               long long& lo, long long& hi) {
+  long long blo, bhi;
+  cmp_range(P, blk, nblk, blo, bhi);
+  const long long per = ((bhi - blo + 63) / 64) * 16;
+  lo = blo + wv * per < bhi ? blo + wv * per : bhi;
+  hi = lo + per < bhi ? lo + per : bhi;
+}
+
+// Bits (0, 1) set where the halves of w are above those of s.
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ unsigned above2(unsigned w, u16x2 s) {
+  u16x2 x;
+  __builtin_memcpy(&x, &w, 4);
+  const u16x2 one = {1, 1};
+  x = __builtin_elementwise_min(__builtin_elementwise_sub_sat(x, s), one);
+  unsigned t;
+  __builtin_memcpy(&t, &x, 4);
+  return (t | (t >> 15)) & 3u;
+}
+
+// The awake ones of brick b's active grains `word`.
+__device__ __forceinline__ unsigned long long awake_bits(const DevBuffers& B, long long b,
+                                                         unsigned long long word,
+                                                         unsigned short Sq) {
+  if (!word) return 0ull;
+  const u16x2 s2 = {Sq, Sq};
+  const uint4* w = reinterpret_cast<const uint4*>(B.wake + 64 * b);
+  uint4 u[8];
+#pragma unroll
+  for (int i = 0; i < 8; i++) u[i] = w[i];
+  unsigned late[2] = {0u, 0u};
+#pragma unroll
+  for (int i = 0; i < 8; i++)
+    late[i >> 2] |= (above2(u[i].x, s2) | (above2(u[i].y, s2) << 2) | (above2(u[i].z, s2) << 4) |
+                     (above2(u[i].w, s2) << 6))
+                    << (8 * (i & 3));
+  return word & ~((unsigned long long)late[0] | ((unsigned long long)late[1] << 32));
+}
+
 __device__ __forceinline__ void count_body(const DevParams& P, const DevBuffers& B, int blk,
                                            int nblk) {
-  if (B.ctr->skip) return;
-  __shared__ unsigned long long s_sm[kBlock / 64];
+  const DevCounters* ctr = B.ctr;
+  if (ctr->skip) return;
+  __shared__ unsigned s_cnt[kBlock / 64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  // a refresh step wakes every active grain
+  const unsigned short Sq = (unsigned short)(ctr->force ? kWakeNever : ctr->Sq);
   long long lo, hi;
-  cmp_range(P, blk, nblk, lo, hi);
-  unsigned long long mine = 0;
-  for (long long b = lo + threadIdx.x; b < hi; b += kBlock) mine += __popcll(B.amap[b]);
-  unsigned long long tot;
-  block_scan_excl(mine, &tot, s_sm);
-  if (threadIdx.x == 0) B.cmptot[blk] = (unsigned)tot;
+  cmp_wave_range(P, blk, nblk, wv, lo, hi);
+  unsigned mine = 0;
+  // 64 bricks per round, one per lane, the next round's active words loaded ahead
+  unsigned long long next = lo + lane < hi ? B.amap[lo + lane] : 0ull;
+  for (long long base = lo; base < hi; base += 64) {
+    const long long b = base + lane;
+    const unsigned long long word = next;
+    next = b + 64 < hi ? B.amap[b + 64] : 0ull;
+    const unsigned long long mask = awake_bits(B, b, word, Sq);
+    if (b < hi) {
+      B.awk[b] = mask;
+      mine += (unsigned)__popcll(mask);
+    }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) mine += __shfl_xor(mine, o, 64);
+  if (lane == 0) s_cnt[wv] = mine;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    unsigned tot = 0;
+    for (int q = 0; q < kBlock / 64; q++) tot += s_cnt[q];
+    B.cmptot[blk] = tot;
+  }
 }
 
 __device__ __forceinline__ void compact_body(const DevParams& P, const DevBuffers& B, int blk,
@@ -375,9 +500,11 @@ __device__ __forceinline__ void compact_body(const DevParams& P, const DevBuffer
   for (int q = threadIdx.x; q < blk; q += kBlock) pre += B.cmptot[q];
   unsigned long long run;
   block_scan_excl(pre, &run, s_sm);
-  if (B.cmptot[blk] == 0u) return;
+  const unsigned own = B.cmptot[blk];
+  if (blk == nblk - 1 && threadIdx.x == 0) B.ctr->n_awake = (int)(run + own);
+  if (own == 0u) return;
   // Per tile of 256 bricks, one brick per thread: each thread puts its brick's
-  // active slots, lowest first, at the brick's position in its wave's stretch
+  // awake slots, lowest first, at the brick's position in its wave's stretch
   // of the output (a wave scan of the active counts; the totals of the waves
   // before come from LDS, double-buffered so that one barrier per tile
   // suffices).  A wave stages its stretch in LDS and writes it out coalesced;
@@ -389,7 +516,7 @@ __device__ __forceinline__ void compact_body(const DevParams& P, const DevBuffer
   int par = 0;
   for (long long base = lo; base < hi; base += kBlock, par ^= 1) {
     const long long b = base + threadIdx.x;
-    unsigned long long w = b < hi ? B.amap[b] : 0ull;
+    unsigned long long w = b < hi ? B.awk[b] : 0ull;
     const unsigned pop = (unsigned)__popcll(w);
     unsigned inc = pop;
 #pragma unroll
@@ -492,48 +619,45 @@ __device__ __forceinline__ unsigned long long claim_entry(const DevParams& P, co
                                                           int q, WordStage* st) {
   int ci, cj, ck;
   slot_ijk(P, q, ci, cj, ck);
-  const SlotRec r = B.rec[rec_slot(q)];
+  const SlotRec r = B.rec[q];
   const unsigned lm = brick_bits26<0, kCoherent>(P, B.bmap, ci, cj, ck);
+  double dmin;
   const unsigned im =
-      claim_tests(P, B, r.id, r.o, ci, cj, ck, lm, make_double4(r.x, r.y, r.z, B.sL[q]), st);
+      claim_tests(P, B, r.id, r.o, ci, cj, ck, lm, make_double4(r.x, r.y, r.z, r.L), st, dmin);
+  B.wake[q] = wake_clock(P, B.ctr->S, r.L, dmin);
   return ((unsigned long long)im << 32) | lm;
 }
 
-// A list wave's envelope tests, one entry per thread.  Wave 0 first grows
-// each active grain (Grain::grow, Grain.h:27, over the whole list as in
-// :521-538); wave 1's grains were created in this step and do not grow.
-// Neighbouring entries sit in the same bricks, so their map words and
-// records share cache lines.
-__device__ __forceinline__ void claim_body(const DevParams& P, const DevBuffers& B, int wave,
-                                           int blk, int nblk) {
+// The tests of list entries [lo, hi) by one block.
+__device__ __forceinline__ void claim_range(const DevParams& P, const DevBuffers& B, int wave,
+                                            int blk, const int* __restrict__ list, int lo, int hi) {
   const DevCounters* ctr = B.ctr;
-  if (ctr->skip) return;
-  // the id scan's per-block capture totals start from zero (k_resolve adds)
-  for (int q = blk * kBlock + threadIdx.x; q < P.ids_blocks; q += nblk * kBlock) B.idtot[q] = 0u;
-  const int* list;
-  int n;
-  list_wave(B, wave, list, n);
-  int lo, hi;
-  chunk_of(n, blk, nblk, kBlock, lo, hi);
   if (lo >= hi) return;
   // the claimed bits, staged per work-group
   __shared__ WordStage s_st;
   stage_init(s_st);
   __syncthreads();
   if (wave == 0) {
-    const double inc = ctr->dt * ctr->v;
+    const double S = ctr->S;
+    const bool force = ctr->force != 0;
+    const int end = (int)ctr->step + 1;
     int id_lo = INT_MAX, id_hi = -1;  // this block's claiming grains
     for (int t = lo + threadIdx.x; t < hi; t += kBlock) {
       const long long q = list[t];
       int i, j, k;
       slot_ijk(P, q, i, j, k);
-      const SlotRec r = B.rec[rec_slot(q)];
-      const double L = B.sL[q] + inc;
-      B.sL[q] = L;
+      const SlotRec r = B.rec[q];
+      const double L = grow_to(B, r.L, r.stamp, end);
+      if (force) {
+        B.rec[q].L = L;
+        B.rec[q].stamp = end;
+      }
       const unsigned lm = brick_bits26<0, false>(P, B.bmap, i, j, k);
+      double dmin;
       const unsigned im =
-          claim_tests(P, B, r.id, r.o, i, j, k, lm, make_double4(r.x, r.y, r.z, L), &s_st);
-      B.masks[t] = ((unsigned long long)im << 32) | lm;
+          claim_tests(P, B, r.id, r.o, i, j, k, lm, make_double4(r.x, r.y, r.z, L), &s_st, dmin);
+      B.wake[q] = wake_clock(P, S, L, dmin);
+      B.masks[t] = ((unsigned long long)im << 32) | (unsigned)r.id;
       if (im) {
         id_lo = min(id_lo, r.id);
         id_hi = max(id_hi, r.id);
@@ -561,14 +685,97 @@ __device__ __forceinline__ void claim_body(const DevParams& P, const DevBuffers&
       atomicMax(&B.ctr->claim_hi[blk & 63], s_hi);
     }
   } else {
-    for (int t = lo + threadIdx.x; t < hi; t += kBlock)
-      B.masks[t] = claim_entry<false>(P, B, list[t], &s_st);
+    // A grain without a liquid neighbour leaves the active map here.  Whether one
+    // with liquid neighbours stays is k_resolve's to say only if a grain of the
+    // wave claimed a cell: without claims all of them stay.
+    int ret = 0;
+    unsigned any = 0;
+    for (int t = lo + threadIdx.x; t < hi; t += kBlock) {
+      const int q = list[t];
+      const unsigned long long m = claim_entry<false>(P, B, q, &s_st);
+      B.masks[t] = m;
+      if ((unsigned)m == 0u) {
+        atomicAnd(&B.amap[q >> 6], ~(1ull << (q & 63)));
+        ret++;
+      }
+      any |= (unsigned)(m >> 32);
+    }
+    __shared__ int s_ret;
+    if (threadIdx.x == 0) s_ret = 0;
+    __syncthreads();
+    if (ret) atomicAdd(&s_ret, ret);
+    if (any) B.ctr->w1_claims = 1;
+    __syncthreads();
+    if (threadIdx.x == 0 && s_ret) atomicAdd(&B.ctr->w1_ret[blk & 63], s_ret);
   }
   __syncthreads();
   stage_flush_or(s_st, B.bmap);
 }
 
-// Captured slots and the keep bit of the grain in slot q at (ci, cj, ck) from
+// A list wave's envelope tests, one entry per thread: bound by the lines of the
+// awake grains' records, about 340 bytes an entry at 512^3 (88 us a step for 1.1 M
+// awake grains of 5.0 M active; all 5.0 M, packed closer, took 145).  Wave 0 first brings each
+// awake grain's L up to the running step (Grain::grow, Grain.h:27, over the whole
+// list as in :521-538: the sleeping grains' turns come when they wake); wave 1's
+// grains were created in this step and do not grow.  Both leave the clock at
+// which the grain wakes next.
+// Neighbouring entries sit in the same bricks, so their map words and
+// records share cache lines.
+__device__ __forceinline__ void claim_body(const DevParams& P, const DevBuffers& B, int wave,
+                                           int blk, int nblk) {
+  const DevCounters* ctr = B.ctr;
+  if (ctr->skip) return;
+  // the id scan's per-block capture totals start from zero (k_resolve adds)
+  for (int q = blk * kBlock + threadIdx.x; q < P.ids_blocks; q += nblk * kBlock) B.idtot[q] = 0u;
+  const int* list;
+  int lo, hi;
+  wave_chunk(P, B, wave, blk, nblk, list, lo, hi);
+  claim_range(P, B, wave, blk, list, lo, hi);
+}
+
+// The short step's wave 0 up to the claims in one launch: each block lists the
+// awake slots of its own bricks (256 per round, one per thread) in its segment of
+// alist and tests them.
+__device__ __forceinline__ void wake_claim_body(const DevParams& P, const DevBuffers& B, int blk,
+                                                int nblk) {
+  const DevCounters* ctr = B.ctr;
+  if (ctr->skip) return;
+  for (int q = blk * kBlock + threadIdx.x; q < P.ids_blocks; q += nblk * kBlock) B.idtot[q] = 0u;
+  __shared__ unsigned long long s_sm[kBlock / 64];
+  const unsigned short Sq = (unsigned short)(ctr->force ? kWakeNever : ctr->Sq);
+  long long blo, bhi;
+  cmp_range(P, blk, nblk, blo, bhi);
+  const int lo = (int)(64 * blo);
+  int hi = lo;
+  for (long long base = blo; base < bhi; base += kBlock) {
+    const long long b = base + threadIdx.x;
+    unsigned long long m = awake_bits(B, b, b < bhi ? B.amap[b] : 0ull, Sq);
+    unsigned long long tot;
+    int pos = hi + (int)block_scan_excl((unsigned long long)__popcll(m), &tot, s_sm);
+    while (m) {
+      B.alist[pos++] = (int)(64 * b) + __builtin_ctzll(m);
+      m &= m - 1;
+    }
+    hi += (int)tot;
+  }
+  if (threadIdx.x == 0) B.cmptot[blk] = (unsigned)(hi - lo);
+  __syncthreads();  // the block's list is complete
+  claim_range(P, B, 0, blk, B.alist, lo, hi);
+}
+
+// claim_index of neighbour (di, dj, dk) = cx[di + 1] + cy[dj + 1] + cz[dk + 1].
+__device__ __forceinline__ void claim_axes(const DevParams& P, int ci, int cj, int ck, unsigned* cx,
+                                           unsigned* cy, unsigned* cz) {
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    const unsigned x = (unsigned)(ci + d - 1), y = (unsigned)(cj + d - 1), z = (unsigned)(ck + d - 1);
+    cx[d] = 64u * (x >> 2) + (x & 3u);
+    cy[d] = 64u * (unsigned)P.nbX * (y >> 2) + ((y & 3u) << 2);
+    cz[d] = 64u * (unsigned)P.nbX * (unsigned)P.nbY * (z >> 2) + ((z & 3u) << 4);
+  }
+}
+
+// Captured slots and the keep bit of the grain in slot q (waves >= 1) at (ci, cj, ck) from
 // its masks m and the claimed bits cmask of its neighbours.  A liquid slot
 // nobody claimed in this wave needs no claim word (its claim is "none", larger
 // than any id); only claimed slots read theirs, all loads issued before any is
@@ -585,16 +792,9 @@ __device__ __forceinline__ unsigned resolve_bits(const DevParams& P, const DevBu
   unsigned keep = (lm & ~im & ~cm) ? 1u : 0u;
   const unsigned need = keep ? (cm & im) : cm;
   if (need == 0) return keep << 31;
-  g = B.skey[q];
-  // claim_index of neighbour (di, dj, dk) = cx[di + 1] + cy[dj + 1] + cz[dk + 1]
+  g = B.rec[q].id;
   unsigned cx[3], cy[3], cz[3];
-#pragma unroll
-  for (int d = 0; d < 3; d++) {
-    const unsigned x = (unsigned)(ci + d - 1), y = (unsigned)(cj + d - 1), z = (unsigned)(ck + d - 1);
-    cx[d] = 64u * (x >> 2) + (x & 3u);
-    cy[d] = 64u * (unsigned)P.nbX * (y >> 2) + ((y & 3u) << 2);
-    cz[d] = 64u * (unsigned)P.nbX * (unsigned)P.nbY * (z >> 2) + ((z & 3u) << 4);
-  }
+  claim_axes(P, ci, cj, ck, cx, cy, cz);
   int cl[26];
 #pragma unroll
   for (int s = 0; s < 26; s++) {
@@ -637,19 +837,166 @@ __device__ __forceinline__ unsigned resolve_entry(const DevParams& P, const DevB
   return r;
 }
 
-// Inclusive prefix sum over the 64 lanes of a wave (every lane must call it).
-__device__ __forceinline__ unsigned wave_incl(unsigned v) {
-  const int lane = threadIdx.x & 63;
+// Captured slots of a wave-0 entry: the enclosed neighbours whose claim word is
+// the grain's own id (every claim of the wave is in by now).
+__device__ __forceinline__ unsigned captured_bits(const DevParams& P, const DevBuffers& B,
+                                                  unsigned im, int ci, int cj, int ck, int g) {
+  unsigned cx[3], cy[3], cz[3];
+  claim_axes(P, ci, cj, ck, cx, cy, cz);
+  int cl[26];
 #pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const unsigned u = __shfl_up(v, d, 64);
-    if (lane >= d) v += u;
+  for (int s = 0; s < 26; s++) {
+    cl[s] = -1;
+    if ((im >> s) & 1u) {
+      int di, dj, dk;
+      slot_delta(s, di, dj, dk);
+      cl[s] = B.claim[cx[di + 1] + cy[dj + 1] + cz[dk + 1]];
+    }
   }
-  return v;
+  unsigned cap = 0;
+#pragma unroll
+  for (int s = 0; s < 26; s++)
+    if (cl[s] == g) cap |= 1u << s;
+  return cap;
 }
 
-// A list wave's decisions, over the same list chunks as its k_emit.  A grain
-// that does not stay active leaves the active map; a grain that captured
+// A brick index along one axis, kept on the grid: a neighbour beyond it only
+// touches ghost cells, so any brick may stand in for it.
+__device__ __forceinline__ int clamp_brick(int b, int n) { return b < 0 ? 0 : (b >= n ? n - 1 : b); }
+
+// The cells of brick (bx, by, bz) with a neighbour (of 26) that is liquid and
+// not claimed in this wave: a bitwise dilation along x, then y, then z.  Lane bits
+// are x (0, 1), y (2, 3), z (4, 5).
+__device__ __forceinline__ unsigned long long open_cells(const DevParams& P, const DevBuffers& B,
+                                                         int bx, int by, int bz) {
+  const ulonglong2* m = reinterpret_cast<const ulonglong2*>(B.bmap);
+  const int xs[3] = {clamp_brick(bx - 1, P.nbX), bx, clamp_brick(bx + 1, P.nbX)};
+  unsigned long long zz[3];
+#pragma unroll
+  for (int dz = 0; dz < 3; dz++) {
+    unsigned long long yy[3];
+#pragma unroll
+    for (int dy = 0; dy < 3; dy++) {
+      const int row = (clamp_brick(bz + dz - 1, P.nbZ) * P.nbY + clamp_brick(by + dy - 1, P.nbY)) * P.nbX;
+      unsigned long long w[3];
+#pragma unroll
+      for (int dx = 0; dx < 3; dx++) {
+        const ulonglong2 u = m[row + xs[dx]];
+        w[dx] = u.x & ~u.y;
+      }
+      const unsigned long long c = w[1];
+      yy[dy] = c | ((c & 0x7777777777777777ull) << 1) | ((c & 0xeeeeeeeeeeeeeeeeull) >> 1) |
+               ((w[0] >> 3) & 0x1111111111111111ull) | ((w[2] & 0x1111111111111111ull) << 3);
+    }
+    const unsigned long long c = yy[1];
+    zz[dz] = c | ((c & 0x0fff0fff0fff0fffull) << 4) | ((c & 0xfff0fff0fff0fff0ull) >> 4) |
+             ((yy[0] >> 12) & 0x000f000f000f000full) | ((yy[2] & 0x000f000f000f000full) << 12);
+  }
+  const unsigned long long c = zz[1];
+  return c | (c << 16) | (c >> 16) | (zz[0] >> 48) | (zz[2] << 48);
+}
+
+// Wave 0's end of activity.  A grain stays active iff at its turn in the sweep one
+// of its liquid neighbours is outside its envelope and not taken by a smaller
+// id: iff some neighbour that was liquid when the wave began carries no claim or
+// a claim above the grain's id (a neighbour inside its own envelope carries a
+// claim of at most its id).  That needs no envelope, so it covers sleeping and
+// awake grains alike, 64 cells at a time: only the active grains whose liquid
+// neighbours are all claimed are looked at one by one.  A grain that retires
+// takes its last growth; retired[blk] counts the block's.
+__device__ __forceinline__ void retire_body(const DevParams& P, const DevBuffers& B, int blk,
+                                            int nblk) {
+  const DevCounters* ctr = B.ctr;
+  if (ctr->skip) return;
+  // Each wave works on its own: 64 bricks per round, one per lane, their
+  // candidates to the wave's stage; the stage is worked off 64 at a time, so
+  // that the dependent loads of a candidate are paid by full waves.
+  constexpr int kStage = 1024;
+  __shared__ int s_q[kBlock / 64][kStage];
+  __shared__ int s_ret;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  if (threadIdx.x == 0) s_ret = 0;
+  __syncthreads();
+  int* st = s_q[wv];
+  const int end = (int)ctr->step + 1;
+  int ret = 0;
+  auto work = [&](int from, int n) {  // stage entries [from, from + n), n <= 64
+    bool gone = false;
+    if (lane < n) {
+      const int q = st[from + lane];
+      int i, j, k;
+      slot_ijk(P, q, i, j, k);
+      const unsigned cm = taken_bits26(P, B, i, j, k);
+      const SlotRec* r = &B.rec[q];
+      const int g = r->id, stamp = r->stamp;
+      const double L = r->L;
+      gone = true;
+      if (cm) {
+        unsigned cx[3], cy[3], cz[3];
+        claim_axes(P, i, j, k, cx, cy, cz);
+        int above = -1;
+#pragma unroll
+        for (int s = 0; s < 26; s++) {
+          if ((cm >> s) & 1u) {
+            int di, dj, dk;
+            slot_delta(s, di, dj, dk);
+            above = max(above, B.claim[cx[di + 1] + cy[dj + 1] + cz[dk + 1]]);
+          }
+        }
+        gone = above <= g;
+      }
+      if (gone) {
+        atomicAnd(&B.amap[q >> 6], ~(1ull << (q & 63)));
+        // its children of this step read L after this
+        B.rec[q].L = grow_to(B, L, stamp, end);
+        B.rec[q].stamp = end;
+      }
+    }
+    ret += gone ? 1 : 0;
+  };
+  long long lo, hi;
+  cmp_wave_range(P, blk, nblk, wv, lo, hi);
+  int pend = 0;
+  unsigned long long next = lo + lane < hi ? B.amap[lo + lane] : 0ull;
+  for (long long base = lo; base < hi; base += 64) {
+    const long long b = base + lane;
+    unsigned long long cand = next;
+    next = b + 64 < hi ? B.amap[b + 64] : 0ull;
+    if (cand) {
+      int bx, by, bz;
+      brick_xyz(P, b, bx, by, bz);
+      cand &= ~open_cells(P, B, bx, by, bz);
+    }
+    // candidates of up to 64 * 64 cells: as many as fit per pass
+    while (__ballot(cand != 0ull)) {
+      const unsigned pop = (unsigned)__popcll(cand);
+      const unsigned incl = wave_incl(pop);
+      int pos = pend + (int)(incl - pop);
+      while (cand && pos < kStage) {
+        st[pos++] = (int)(64 * b) + __builtin_ctzll(cand);
+        cand &= cand - 1;
+      }
+      pend = min(kStage, pend + (int)__shfl(incl, 63, 64));
+      // the wave's LDS operations complete in order
+      __builtin_amdgcn_wave_barrier();
+      while (pend >= 64) {
+        pend -= 64;
+        work(pend, 64);
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
+  work(0, pend);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) ret += __shfl_xor(ret, o, 64);
+  if (lane == 0 && ret) atomicAdd(&s_ret, ret);
+  __syncthreads();
+  if (threadIdx.x == 0) B.lb_flag[kStatBase + blk] = (unsigned)s_ret;
+}
+
+// A list wave's decisions, over the same list chunks as its k_emit.  A grain of
+// wave 1 that does not stay active leaves the active map (wave 0's are
+// retire_body's); a grain that captured
 // writes (id, slot, captured slots, first child in the block) to its block's
 // segment of the parent list, which starts at the block's first list entry,
 // and its capture count to the id-indexed count array.  Each block leaves
@@ -659,7 +1006,7 @@ __device__ __forceinline__ unsigned wave_incl(unsigned v) {
 __device__ __forceinline__ void resolve_body(const DevParams& P, const DevBuffers& B, int wave,
                                              int blk, int nblk) {
   const DevCounters* ctr = B.ctr;
-  if (ctr->skip) return;
+  if (ctr->skip || (wave == 1 && !ctr->w1_claims)) return;
   __shared__ unsigned long long s_pc;         // parents << 32 | children
   __shared__ int s_surv;
   __shared__ unsigned s_hist[kMaxIdsBlocks];  // captures per id-scan block
@@ -670,10 +1017,8 @@ __device__ __forceinline__ void resolve_body(const DevParams& P, const DevBuffer
   for (int q = threadIdx.x; q < P.ids_blocks; q += kBlock) s_hist[q] = 0u;
   __syncthreads();
   const int* list;
-  int n;
-  list_wave(B, wave, list, n);
   int lo, hi;
-  chunk_of(n, blk, nblk, kBlock, lo, hi);
+  wave_chunk(P, B, wave, blk, nblk, list, lo, hi);
   int4* __restrict__ seg = B.plist + lo;
   const IdRange ir = id_range(P, ctr, wave);
   const int lane = threadIdx.x & 63;
@@ -685,12 +1030,21 @@ __device__ __forceinline__ void resolve_body(const DevParams& P, const DevBuffer
     if (t < hi) {
       q = list[t];
       const unsigned long long m = B.masks[t];
-      if ((unsigned)m != 0u) {
-        int i, j, k;
-        slot_ijk(P, q, i, j, k);
-        r = resolve_bits<false>(P, B, q, m, brick_bits26<1, false>(P, B.bmap, i, j, k), i, j, k, g);
+      int i, j, k;
+      if (wave == 0) {
+        const unsigned im = (unsigned)(m >> 32);
+        if (im) {
+          g = (int)(unsigned)m;
+          slot_ijk(P, q, i, j, k);
+          r = captured_bits(P, B, im, i, j, k, g);
+        }
+      } else {
+        if ((unsigned)m != 0u) {
+          slot_ijk(P, q, i, j, k);
+          r = resolve_bits<false>(P, B, q, m, brick_bits26<1, false>(P, B.bmap, i, j, k), i, j, k, g);
+        }
+        if (!(r >> 31)) atomicAnd(&B.amap[q >> 6], ~(1ull << (q & 63)));
       }
-      if (!(r >> 31)) atomicAnd(&B.amap[q >> 6], ~(1ull << (q & 63)));
     }
     const unsigned long long keepm = __ballot(t < hi && (r >> 31));
     if (lane == 0 && keepm) atomicAdd(&s_surv, (int)__popcll(keepm));
@@ -730,12 +1084,12 @@ __device__ __forceinline__ void resolve_body(const DevParams& P, const DevBuffer
 // thread, one uint4 of counts), writes each capturing grain's first child
 // (wave-relative) and zeroes the counts it has read.  The last block also
 // turns the `nres` k_resolve blocks' child counts into each block's first
-// child, adds the wave's survivors to the active count, and publishes the
-// wave's children (the next id range and list length).
+// child, adds the wave's survivors to the active count (wave 0: the active
+// grains without those retired), and publishes the wave's children (the next id range and list length).
 __device__ __forceinline__ void idscan_body(const DevParams& P, const DevBuffers& B, int wave,
                                             int blk, int nres) {
   DevCounters* ctr = B.ctr;
-  if (ctr->skip) return;
+  if (ctr->skip || (wave == 1 && !ctr->w1_claims)) return;
   __shared__ unsigned long long s_sm[kBlock / 64];
   const int nblk = P.ids_blocks;
   const IdRange ir = id_range(P, ctr, wave);
@@ -810,7 +1164,13 @@ __device__ __forceinline__ void idscan_body(const DevParams& P, const DevBuffers
         off += c[x];
       }
     }
-    const unsigned long long svt = tot >> 32;
+    unsigned long long svt = tot >> 32;
+    if (wave == 0) {
+      unsigned long long gone = 0;
+      for (int q = threadIdx.x; q < P.cmp_blocks; q += kBlock) gone += B.lb_flag[kStatBase + q];
+      block_scan_excl(gone, &tot, s_sm);
+      svt = (unsigned long long)ctr->nA_in - tot;
+    }
     if (threadIdx.x == 0) {
       const unsigned long long nc = start + mine;
       const int gbase = ctr->n_grains;
@@ -835,15 +1195,15 @@ __device__ __forceinline__ void idscan_body(const DevParams& P, const DevBuffers
 __device__ __forceinline__ int write_child(const DevParams& P, const DevBuffers& B, int id, int ni,
                                            int nj, int nk, int o, const double4& env) {
   const long long q = claim_index(P, ni, nj, nk);
-  SlotRec r;
+  SlotRec r{};
   r.x = env.x;
   r.y = env.y;
   r.z = env.z;
+  r.L = env.w;
   r.id = id;
   r.o = o;
-  B.rec[rec_slot(q)] = r;
-  B.sL[q] = env.w;
-  B.skey[q] = id;
+  r.stamp = (int)B.ctr->step + 1;  // grows from the next step on
+  B.rec[q] = r;
   brick_clear(P, B.bmap, 0, ni, nj, nk);
   atomicOr(&B.amap[q >> 6], 1ull << (q & 63));
   return (int)q;
@@ -883,9 +1243,9 @@ __device__ __forceinline__ void emit_from(const DevParams& P, const DevBuffers& 
   }
 }
 
-// The envelope of the grain in slot q.
-__device__ __forceinline__ double4 slot_env(const DevBuffers& B, const SlotRec& r, long long q) {
-  return make_double4(r.x, r.y, r.z, B.sL[q]);
+// The envelope of a grain in the running step.
+__device__ __forceinline__ double4 slot_env(const DevBuffers& B, const SlotRec& r) {
+  return make_double4(r.x, r.y, r.z, grow_to(B, r.L, r.stamp, (int)B.ctr->step + 1));
 }
 
 // The children of the parent in slot qp.
@@ -894,8 +1254,8 @@ __device__ __forceinline__ void emit_children(const DevParams& P, const DevBuffe
                                               int pos0) {
   int ci, cj, ck;
   slot_ijk(P, qp, ci, cj, ck);
-  const SlotRec pr = B.rec[rec_slot(qp)];
-  emit_from(P, B, pr.o, slot_env(B, pr, qp), ci, cj, ck, cap, id0, kids, pos0);
+  const SlotRec pr = B.rec[qp];
+  emit_from(P, B, pr.o, slot_env(B, pr), ci, cj, ck, cap, id0, kids, pos0);
 }
 
 // A list wave's children, one per thread.  A capturing grain's children take
@@ -911,14 +1271,12 @@ __device__ __forceinline__ void emit_children(const DevParams& P, const DevBuffe
 __device__ __forceinline__ void emit_body(const DevParams& P, const DevBuffers& B, int wave,
                                           int blk, int nblk) {
   const DevCounters* ctr = B.ctr;
-  if (ctr->skip) return;
+  if (ctr->skip || (wave == 1 && !ctr->w1_claims)) return;
   constexpr int kStage = 1024;
   __shared__ int2 s_stage[kStage];
   const int* list;
-  int n;
-  list_wave(B, wave, list, n);
   int lo, hi;
-  chunk_of(n, blk, nblk, kBlock, lo, hi);
+  wave_chunk(P, B, wave, blk, nblk, list, lo, hi);
   const int np = (int)(B.lb_agg[kStatBase + blk] >> 32);
   if (np == 0) return;
   const int cb = (int)B.lb_pref[kStatBase + blk];
@@ -953,8 +1311,8 @@ __device__ __forceinline__ void emit_body(const DevParams& P, const DevBuffers& 
         const int q = pp.y;
         int ci, cj, ck;
         slot_ijk(P, q, ci, cj, ck);
-        const SlotRec pr = B.rec[rec_slot(q)];
-        const double4 e = slot_env(B, pr, q);
+        const SlotRec pr = B.rec[q];
+        const double4 e = slot_env(B, pr);
         double r[9];
         const double* rp = B.l2g + 9 * (size_t)pr.o;
 #pragma unroll
@@ -977,12 +1335,76 @@ __device__ __forceinline__ void emit_body(const DevParams& P, const DevBuffers& 
 // of the step: time_ += dT_, iStep_++, liquid count (:650-659).
 constexpr int kTailBlock = 1024;
 
+// Wave 1's captures in the short step (k_resolve, k_idscan and k_emit of the list
+// wave, by one work-group): wave 1's list is in its parents' brick order, so its
+// capturing grains' children are numbered by a scan over the wave's id range.
+__device__ __forceinline__ void tail_wave1(const DevParams& P, const DevBuffers& B, int n,
+                                           unsigned long long* s_sm) {
+  DevCounters* ctr = B.ctr;
+  const int* list = B.listW[0];
+  unsigned long long kept = 0;
+  for (int i = threadIdx.x; i < n; i += kTailBlock) {
+    const int q = list[i];
+    // nothing here changes the maps or the claims, so plain loads do
+    const unsigned r = resolve_entry<false>(P, B, q, B.masks[i]);
+    const unsigned cap = r & 0x3ffffffu;
+    kept += r >> 31;
+    B.masks[i] = cap;
+    if (cap) B.cnt[B.rec[q].id] = (unsigned char)__builtin_popcount(cap);
+  }
+  unsigned long long surv;
+  block_scan_excl(kept, &surv, s_sm);
+  __threadfence_block();
+  __syncthreads();
+  const int lo = ctr->w1_lo, hi = lo + ctr->w1_n, gbase = ctr->n_grains;
+  unsigned long long run = 0;
+  for (int base = lo; base < hi; base += kTailBlock) {
+    const int g = base + threadIdx.x;
+    const unsigned c = g < hi ? B.cnt[g] : 0u;
+    unsigned long long tot;
+    const unsigned long long off = run + block_scan_excl(c, &tot, s_sm);
+    if (c) {
+      B.coff[g] = (int)off;
+      B.cnt[g] = 0;
+    }
+    run += tot;
+  }
+  __threadfence_block();
+  __syncthreads();
+  for (int i = threadIdx.x; i < n; i += kTailBlock) {
+    const unsigned cap = (unsigned)B.masks[i];
+    if (!cap) continue;
+    const int q = list[i];
+    const int c0 = B.coff[B.rec[q].id];
+    emit_children(P, B, q, cap, gbase + c0, B.listW[1], c0);
+  }
+  __threadfence_block();
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const int nc = (int)run;
+    ctr->n_grains = gbase + nc;
+    ctr->nA_out += (int)surv;
+    ctr->nW[1] = nc;
+    ctr->step_cap += nc;
+    if (nc > 0 && ctr->max_wave < 2) ctr->max_wave = 2;
+    if (nc > 0 && ctr->step_wave < 2) ctr->step_wave = 2;
+  }
+  __syncthreads();
+}
+
 __device__ __forceinline__ void tail_body(const DevParams& P, const DevBuffers& B) {
   DevCounters* ctr = B.ctr;
   if (ctr->skip) return;
   __shared__ unsigned long long s_sm[kTailBlock / 64];
   __shared__ int s_n, s_gbase, s_sbase;
   const int n_wave1 = ctr->nW[0];  // wave-0 captures, before wave 2 reuses the slot
+  if (P.fused && ctr->w1_claims) {
+    tail_wave1(P, B, n_wave1, s_sm);
+  } else if (!ctr->w1_claims && threadIdx.x < 64) {
+    // wave 1 claimed nothing: its grains with a liquid neighbour stay active
+    const int ret = (int)wave_sum((unsigned long long)ctr->w1_ret[threadIdx.x]);
+    if (threadIdx.x == 0) ctr->nA_out += n_wave1 - ret;
+  }
   int wave = 2;
   while (true) {
     const int in = (wave - 1) & 1;
@@ -1101,13 +1523,20 @@ __global__ void __launch_bounds__(kBlock) k_nucleate(DevParams P, DevBuffers B) 
 __global__ void __launch_bounds__(kBlock) k_claim(DevParams P, DevBuffers B, int wave) {
   claim_body(P, B, wave, xcd_block(), gridDim.x);
 }
-__global__ void __launch_bounds__(kBlock) k_resolve(DevParams P, DevBuffers B, int wave) {
-  resolve_body(P, B, wave, xcd_block(), gridDim.x);
+// the first `nres` blocks decide the wave's captures; in wave 0 the others retire
+__global__ void __launch_bounds__(kBlock) k_resolve(DevParams P, DevBuffers B, int wave, int nres) {
+  if ((int)blockIdx.x < nres)
+    resolve_body(P, B, wave, xcd_of(blockIdx.x, nres), nres);
+  else
+    retire_body(P, B, xcd_of(blockIdx.x - nres, P.cmp_blocks), P.cmp_blocks);
 }
 __global__ void __launch_bounds__(kBlock) k_emit(DevParams P, DevBuffers B, int wave) {
   emit_body(P, B, wave, xcd_block(), gridDim.x);
 }
 __global__ void __launch_bounds__(kTailBlock) k_tail(DevParams P, DevBuffers B) { tail_body(P, B); }
+__global__ void __launch_bounds__(kBlock) k_wake_claim(DevParams P, DevBuffers B) {
+  wake_claim_body(P, B, xcd_block(), gridDim.x);
+}
 __global__ void __launch_bounds__(kBlock) k_count(DevParams P, DevBuffers B) {
   count_body(P, B, blockIdx.x, gridDim.x);
 }
@@ -1134,10 +1563,12 @@ __global__ void k_materialize(DevParams P, DevBuffers B) {
       continue;
     }
     const long long q = claim_index(P, i, j, k);
-    const SlotRec r = B.rec[rec_slot(q)];
+    const SlotRec r = B.rec[q];
     B.gid[c] = r.id;
     B.oid[c] = r.o;
-    B.genv[r.id] = make_double4(r.x, r.y, r.z, B.sL[q]);
+    double L = r.L;
+    if ((B.amap[q >> 6] >> (q & 63)) & 1ull) L = grow_to(B, L, r.stamp, (int)B.ctr->step);
+    B.genv[r.id] = make_double4(r.x, r.y, r.z, L);
     B.gco[r.id] = make_int2((int)c, r.o);
   }
 }
@@ -1157,9 +1588,15 @@ __global__ void __launch_bounds__(kBlock) kb_claim(const DevParams* Ps, const De
   claim_body(Ps[m.x], Bs[m.x], wave, m.y, m.z);
 }
 __global__ void __launch_bounds__(kBlock) kb_resolve(const DevParams* Ps, const DevBuffers* Bs,
-                                                     const int4* map, int wave) {
-  const int4 m = map[blockIdx.x];
-  resolve_body(Ps[m.x], Bs[m.x], wave, m.y, m.z);
+                                                     const int4* map, int nres,
+                                                     const int4* map_cmp, int wave) {
+  if ((int)blockIdx.x < nres) {
+    const int4 m = map[blockIdx.x];
+    resolve_body(Ps[m.x], Bs[m.x], wave, m.y, m.z);
+  } else {
+    const int4 m = map_cmp[blockIdx.x - nres];
+    retire_body(Ps[m.x], Bs[m.x], m.y, m.z);
+  }
 }
 __global__ void __launch_bounds__(kBlock) kb_emit(const DevParams* Ps, const DevBuffers* Bs,
                                                   const int4* map, int wave) {
@@ -1180,6 +1617,11 @@ __global__ void __launch_bounds__(kBlock) kb_count(const DevParams* Ps, const De
                                                    const int4* map) {
   const int4 m = map[blockIdx.x];
   count_body(Ps[m.x], Bs[m.x], m.y, m.z);
+}
+__global__ void __launch_bounds__(kBlock) kb_wake_claim(const DevParams* Ps, const DevBuffers* Bs,
+                                                        const int4* map) {
+  const int4 m = map[blockIdx.x];
+  wake_claim_body(Ps[m.x], Bs[m.x], m.y, m.z);
 }
 __global__ void __launch_bounds__(kBlock) kb_idscan(const DevParams* Ps, const DevBuffers* Bs,
                                                     const int4* map, int wave) {
@@ -1203,12 +1645,24 @@ hipError_t launch_batch_status(const BatchLaunch& L, int n, int4* out, hipStream
 }
 
 hipError_t launch_batch_step(const BatchLaunch& L, hipStream_t s) {
+  if (L.fused) {
+    hipLaunchKernelGGL(kb_nucleate, dim3(L.n_nuc), dim3(kBlock), 0, s, L.P, L.B, L.map_nuc);
+    hipLaunchKernelGGL(kb_wake_claim, dim3(L.n_cmp), dim3(kBlock), 0, s, L.P, L.B, L.map_cmp);
+    hipLaunchKernelGGL(kb_resolve, dim3(2 * L.n_cmp), dim3(kBlock), 0, s, L.P, L.B, L.map_cmp, L.n_cmp,
+                       L.map_cmp, 0);
+    hipLaunchKernelGGL(kb_idscan, dim3(L.n_ids), dim3(kBlock), 0, s, L.P, L.B, L.map_ids, 0);
+    hipLaunchKernelGGL(kb_emit, dim3(L.n_cmp), dim3(kBlock), 0, s, L.P, L.B, L.map_cmp, 0);
+    hipLaunchKernelGGL(kb_claim, dim3(L.n_list), dim3(kBlock), 0, s, L.P, L.B, L.map_list, 1);
+    hipLaunchKernelGGL(kb_tail, dim3(L.n_one), dim3(kTailBlock), 0, s, L.P, L.B, L.map_one);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL(kb_nucleate, dim3(L.n_nuc), dim3(kBlock), 0, s, L.P, L.B, L.map_nuc);
   hipLaunchKernelGGL(kb_count, dim3(L.n_cmp), dim3(kBlock), 0, s, L.P, L.B, L.map_cmp);
   hipLaunchKernelGGL(kb_compact, dim3(L.n_cmp), dim3(kBlock), 0, s, L.P, L.B, L.map_cmp);
   for (int wave = 0; wave < 2; wave++) {
     hipLaunchKernelGGL(kb_claim, dim3(L.n_list), dim3(kBlock), 0, s, L.P, L.B, L.map_list, wave);
-    hipLaunchKernelGGL(kb_resolve, dim3(L.n_emit), dim3(kBlock), 0, s, L.P, L.B, L.map_emit, wave);
+    hipLaunchKernelGGL(kb_resolve, dim3(L.n_emit + (wave == 0 ? L.n_cmp : 0)), dim3(kBlock), 0, s,
+                       L.P, L.B, L.map_emit, L.n_emit, L.map_cmp, wave);
     hipLaunchKernelGGL(kb_idscan, dim3(L.n_ids), dim3(kBlock), 0, s, L.P, L.B, L.map_ids, wave);
     hipLaunchKernelGGL(kb_emit, dim3(L.n_emit), dim3(kBlock), 0, s, L.P, L.B, L.map_emit, wave);
   }
@@ -1236,7 +1690,8 @@ hipError_t launch_claim(const DevParams& P, const DevBuffers& B, int wave, int b
 
 hipError_t launch_resolve(const DevParams& P, const DevBuffers& B, int wave, int blocks,
                           hipStream_t s) {
-  hipLaunchKernelGGL(k_resolve, dim3(blocks), dim3(kBlock), 0, s, P, B, wave);
+  hipLaunchKernelGGL(k_resolve, dim3(blocks + (wave == 0 ? P.cmp_blocks : 0)), dim3(kBlock), 0, s, P,
+                     B, wave, blocks);
   return hipGetLastError();
 }
 
@@ -1253,6 +1708,11 @@ hipError_t launch_count(const DevParams& P, const DevBuffers& B, int blocks, hip
 
 hipError_t launch_compact(const DevParams& P, const DevBuffers& B, int blocks, hipStream_t s) {
   hipLaunchKernelGGL(k_compact, dim3(blocks), dim3(kBlock), 0, s, P, B);
+  return hipGetLastError();
+}
+
+hipError_t launch_wake_claim(const DevParams& P, const DevBuffers& B, hipStream_t s) {
+  hipLaunchKernelGGL(k_wake_claim, dim3(P.cmp_blocks), dim3(kBlock), 0, s, P, B);
   return hipGetLastError();
 }
 
