@@ -578,24 +578,27 @@ amca_status amca_domain_download(amca_domain* d, int32_t* orient, int32_t* grain
   const size_t NG = (size_t)d->P.NG;
   amca::DevCounters c;
   AMCA_TRY(read_counters(d, &c));
-  // the grain-ID fields and the records by id, materialized from the slots
-  if (orient || grain || env) {
+  // the grain-ID fields, materialized from the slots
+  if (orient || grain) {
     HIP_TRY(amca::launch_materialize(d->P, d->B, d->stream));
     HIP_TRY(hipStreamSynchronize(d->stream));
   }
   if (orient) HIP_TRY(hipMemcpy(orient, d->B.oid, sizeof(int32_t) * NG, hipMemcpyDeviceToHost));
   if (grain) HIP_TRY(hipMemcpy(grain, d->B.gid, sizeof(int32_t) * NG, hipMemcpyDeviceToHost));
   if (env) {
-    // grain records by id, scattered to their cells
-    std::memset(env, 0, sizeof(double) * 4 * NG);
-    const size_t ng = (size_t)std::max(c.n_grains, 0);
-    if (ng > 0) {
-      std::vector<double> ge(4 * ng);
-      std::vector<int32_t> gc(2 * ng);
-      HIP_TRY(hipMemcpy(ge.data(), d->B.genv, sizeof(double) * 4 * ng, hipMemcpyDeviceToHost));
-      HIP_TRY(hipMemcpy(gc.data(), d->B.gco, sizeof(int32_t) * 2 * ng, hipMemcpyDeviceToHost));
-      for (size_t g = 0; g < ng; g++)
-        std::memcpy(env + 4 * (size_t)gc[2 * g], &ge[4 * g], sizeof(double) * 4);
+    // laid out by cell on the device, a piece of 64 MB at a time (the host's
+    // memset and scatter of the records took longer than the run of a small grid)
+    const size_t piece = std::min<size_t>(NG, (size_t)1 << 21);
+    double4* buf = nullptr;
+    const auto release = on_scope_exit([&] {
+      if (buf) (void)hipFree(buf);
+    });
+    HIP_TRY(hipMalloc(&buf, sizeof(double4) * piece));
+    for (size_t c0 = 0; c0 < NG; c0 += piece) {
+      const int n = (int)std::min(piece, NG - c0);
+      HIP_TRY(amca::launch_cell_env(d->P, d->B, (long long)c0, n, buf, d->stream));
+      HIP_TRY(hipMemcpyAsync(env + 4 * c0, buf, sizeof(double4) * n, hipMemcpyDeviceToHost, d->stream));
+      HIP_TRY(hipStreamSynchronize(d->stream));
     }
   }
   if (n_sites) *n_sites = c.n_sites;

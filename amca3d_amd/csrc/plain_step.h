@@ -197,6 +197,9 @@ hipError_t launch_idscan(const DevParams& P, const DevBuffers& B, int wave, int 
                          hipStream_t s);
 // gid / oid on the ghosted grid, genv / gco by grain id, from the slots
 hipError_t launch_materialize(const DevParams& P, const DevBuffers& B, hipStream_t s);
+// envelopes by cell of the n ghosted cells from c0 on
+hipError_t launch_cell_env(const DevParams& P, const DevBuffers& B, long long c0, int n, double4* out,
+                           hipStream_t s);
 hipError_t launch_emit(const DevParams& P, const DevBuffers& B, int wave, int blocks,
                        hipStream_t s);
 hipError_t launch_tail(const DevParams& P, const DevBuffers& B, hipStream_t s);

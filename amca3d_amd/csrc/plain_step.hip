@@ -1573,6 +1573,25 @@ __global__ void k_materialize(DevParams P, DevBuffers B) {
   }
 }
 
+// Envelopes by cell, ghosted cells [c0, c0 + n): the grain's centre and L, zeros
+// where there is none.
+__global__ void k_cell_env(DevParams P, DevBuffers B, long long c0, int n, double4* out) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  double4 e = make_double4(0.0, 0.0, 0.0, 0.0);
+  int i, j, k;
+  cell_ijk(P, (int)(c0 + t), i, j, k);
+  if (i >= 1 && i <= P.nx && j >= 1 && j <= P.ny && k >= 1 && k <= P.nz &&
+      !(B.bmap[brick_word(P, i, j, k)] & brick_bit(i, j, k))) {
+    const long long q = claim_index(P, i, j, k);
+    const SlotRec r = B.rec[q];
+    double L = r.L;
+    if ((B.amap[q >> 6] >> (q & 63)) & 1ull) L = grow_to(B, L, r.stamp, (int)B.ctr->step);
+    e = make_double4(r.x, r.y, r.z, L);
+  }
+  out[t] = e;
+}
+
 // ---------------------------------------------------------------------------
 // batched kernels: block b serves domain map[b].x as its block map[b].y of
 // map[b].z (the per-domain launch geometry of the single-domain kernels)
@@ -1727,6 +1746,12 @@ hipError_t launch_materialize(const DevParams& P, const DevBuffers& B, hipStream
   if (blocks > 16384) blocks = 16384;
   if (blocks < 1) blocks = 1;
   hipLaunchKernelGGL(k_materialize, dim3((unsigned)blocks), dim3(256), 0, s, P, B);
+  return hipGetLastError();
+}
+
+hipError_t launch_cell_env(const DevParams& P, const DevBuffers& B, long long c0, int n, double4* out,
+                           hipStream_t s) {
+  hipLaunchKernelGGL(k_cell_env, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, P, B, c0, n, out);
   return hipGetLastError();
 }
 

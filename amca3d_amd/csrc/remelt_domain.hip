@@ -69,8 +69,6 @@ struct amca_remelt {
   std::vector<double> site_dts;
   std::vector<double> euler;                  // Euler angles of every row, 3 per row
   size_t grain_cap = 0;  // records genv/gco can hold
-  std::vector<int32_t> host_tag;
-  std::vector<double> host_par;
   std::vector<double> node_xyz;
   // per-kernel event timing (off by default)
   bool timing = false;
@@ -443,72 +441,167 @@ amca_status amca_remelt_destroy(amca_remelt* d) {
 
 namespace {
 
+// device memory of one call, freed on every return
+struct DeviceTemp {
+  void* p = nullptr;
+  ~DeviceTemp() {
+    if (p) (void)hipFree(p);
+  }
+  hipError_t get(size_t bytes) { return hipMalloc(&p, std::max<size_t>(bytes, 16)); }
+};
+
 // tag_voxels on the device: one thread per CA cell (ghosts included), the
 // arithmetic of the host mapper (voxel_math.h), so tags and parametric
-// coordinates equal the host's bit for bit
+// coordinates equal the host's bit for bit; *any is set when a cell has an element
 __global__ void k_map_voxels(amca_vox::MeshView M, amca_vox::VoxelGrid G,
                              const int* __restrict__ bin_start, const int* __restrict__ bin_elems,
                              long long NG, double tol, int max_iter, int32_t* __restrict__ tag,
-                             double* __restrict__ par) {
+                             double* __restrict__ par, int* any) {
   const long long stride = (long long)gridDim.x * blockDim.x;
+  int found = 0;
   for (long long v = (long long)blockIdx.x * blockDim.x + threadIdx.x; v < NG; v += stride) {
     double pc[3];
     const int e = amca_vox::tag_voxel(M, G, bin_start, bin_elems, v, tol, max_iter, pc);
     tag[v] = e;
     for (int q = 0; q < 3; q++) par[3 * v + q] = e >= 0 ? pc[q] : -2.0;
+    found |= e >= 0 ? 1 : 0;
   }
+  if (__syncthreads_or(found) && threadIdx.x == 0 &&
+      !__hip_atomic_load(any, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+    __hip_atomic_store(any, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// map_voxels on the device: the plan (search box, bins) on the host, the
-// per-cell search in k_map_voxels; results copied into host vectors.
-// Returns false when no cell found an element.
+// map_voxels on the device into tag[NG], par[3 NG] (device memory): the plan
+// (search box, bins) on the host, the per-cell search in k_map_voxels.  any:
+// whether a cell found an element.
 amca_status map_voxels_device(const amca_host::FeMesh& mesh, const amca_host::VoxelMapParams& vp,
-                              std::vector<int32_t>& tag, std::vector<double>& par, bool& any) {
+                              int32_t* tag, double* par, hipStream_t s, bool& any) {
   amca_host::VoxelPlan plan;
   amca_host::plan_voxels(mesh, vp, plan);
   const amca_vox::VoxelGrid& G = plan.grid;
   const long long NG = (long long)G.nxG * G.nyG * G.nzG;
   if (plan.bin_elems.empty()) plan.bin_elems.push_back(0);  // a valid pointer; no bin reads it
-  double* dxyz = nullptr;
-  int *dbs = nullptr, *dbe = nullptr;
-  int32_t* dtag = nullptr;
-  double* dpar = nullptr;
-  amca_status st = AMCA_OK;
-  auto hip = [&](hipError_t e, const char* what) {
-    if (e != hipSuccess && st == AMCA_OK) st = rm_fail(AMCA_ERR_HIP, std::string(what) + ": " +
-                                                              hipGetErrorString(e));
-    return e == hipSuccess;
-  };
-  if (hip(hipMalloc(&dxyz, sizeof(double) * mesh.xyz.size()), "voxel map alloc") &&
-      hip(hipMalloc(&dbs, sizeof(int) * plan.bin_start.size()), "voxel map alloc") &&
-      hip(hipMalloc(&dbe, sizeof(int) * plan.bin_elems.size()), "voxel map alloc") &&
-      hip(hipMalloc(&dtag, sizeof(int32_t) * (size_t)NG), "voxel map alloc") &&
-      hip(hipMalloc(&dpar, sizeof(double) * 3 * (size_t)NG), "voxel map alloc") &&
-      hip(hipMemcpy(dxyz, mesh.xyz.data(), sizeof(double) * mesh.xyz.size(),
-                    hipMemcpyHostToDevice), "voxel map upload") &&
-      hip(hipMemcpy(dbs, plan.bin_start.data(), sizeof(int) * plan.bin_start.size(),
-                    hipMemcpyHostToDevice), "voxel map upload") &&
-      hip(hipMemcpy(dbe, plan.bin_elems.data(), sizeof(int) * plan.bin_elems.size(),
-                    hipMemcpyHostToDevice), "voxel map upload")) {
-    const amca_vox::MeshView mv{dxyz, mesh.fnx, mesh.fny, mesh.fnz};
-    long long blocks = (NG + 255) / 256;
-    if (blocks > 65536) blocks = 65536;
-    hipLaunchKernelGGL(k_map_voxels, dim3((unsigned)blocks), dim3(256), 0, 0, mv, G, dbs, dbe, NG,
-                       vp.tol, vp.max_iter, dtag, dpar);
-    tag.resize((size_t)NG);
-    par.resize(3 * (size_t)NG);
-    if (hip(hipGetLastError(), "k_map_voxels") &&
-        hip(hipMemcpy(tag.data(), dtag, sizeof(int32_t) * (size_t)NG, hipMemcpyDeviceToHost),
-            "voxel map readback"))
-      hip(hipMemcpy(par.data(), dpar, sizeof(double) * 3 * (size_t)NG, hipMemcpyDeviceToHost),
-          "voxel map readback");
+  DeviceTemp dxyz, dbs, dbe, dany;
+  RM_HIP(dxyz.get(sizeof(double) * mesh.xyz.size()));
+  RM_HIP(dbs.get(sizeof(int) * plan.bin_start.size()));
+  RM_HIP(dbe.get(sizeof(int) * plan.bin_elems.size()));
+  RM_HIP(dany.get(sizeof(int)));
+  int found = 0;
+  RM_HIP(hipMemcpyAsync(dxyz.p, mesh.xyz.data(), sizeof(double) * mesh.xyz.size(),
+                        hipMemcpyHostToDevice, s));
+  RM_HIP(hipMemcpyAsync(dbs.p, plan.bin_start.data(), sizeof(int) * plan.bin_start.size(),
+                        hipMemcpyHostToDevice, s));
+  RM_HIP(hipMemcpyAsync(dbe.p, plan.bin_elems.data(), sizeof(int) * plan.bin_elems.size(),
+                        hipMemcpyHostToDevice, s));
+  RM_HIP(hipMemcpyAsync(dany.p, &found, sizeof(int), hipMemcpyHostToDevice, s));
+  const amca_vox::MeshView mv{static_cast<double*>(dxyz.p), mesh.fnx, mesh.fny, mesh.fnz};
+  long long blocks = (NG + 255) / 256;
+  if (blocks > 65536) blocks = 65536;
+  hipLaunchKernelGGL(k_map_voxels, dim3((unsigned)blocks), dim3(256), 0, s, mv, G,
+                     static_cast<int*>(dbs.p), static_cast<int*>(dbe.p), NG, vp.tol, vp.max_iter,
+                     tag, par, static_cast<int*>(dany.p));
+  RM_HIP(hipGetLastError());
+  RM_HIP(hipMemcpyAsync(&found, dany.p, sizeof(int), hipMemcpyDeviceToHost, s));
+  RM_HIP(hipStreamSynchronize(s));
+  any = found != 0;
+  return AMCA_OK;
+}
+
+// ---- boxes for the active box (amca_remelt_set_fe) --------------------------
+// Per element the box of its cells; per frame the union over the elements with a
+// hot node (at or above Tm - hot_margin), and the union over the elements with a
+// node whose void state can change between frames.  On the host these loops and
+// the copies of the voxel map down and up again were most of the call (72 ms at
+// 400 x 160 x 80 cells and 100 frames).
+
+__global__ void k_box_clear(long long n, int* __restrict__ b) {
+  const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q < n) b[q] = (q % 6) < 3 ? INT_MAX : INT_MIN;
+}
+
+__global__ void k_elem_boxes(amca::RmParams P, const int32_t* __restrict__ tag, int* ebox) {
+  const long long stride = (long long)gridDim.x * blockDim.x;
+  for (long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x; c < P.NG; c += stride) {
+    const int e = tag[c];
+    if (e < 0) continue;
+    const int k = (int)c / P.nxyG, r = (int)c - k * P.nxyG, j = r / P.nxG, i = r - j * P.nxG;
+    int* b = ebox + 6 * (size_t)e;
+    const int v[3] = {i, j, k};
+    // most cells change nothing: a plain read first (a stale one only costs an atomic)
+    for (int a = 0; a < 3; a++) {
+      if (v[a] < b[a]) atomicMin(&b[a], v[a]);
+      if (v[a] > b[3 + a]) atomicMax(&b[3 + a], v[a]);
+    }
   }
-  for (void* ptr : {(void*)dxyz, (void*)dbs, (void*)dbe, (void*)dtag, (void*)dpar})
-    if (ptr) (void)hipFree(ptr);
-  any = false;
-  if (st == AMCA_OK)
-    for (long long v = 0; v < NG && !any; v++) any = tag[(size_t)v] >= 0;
-  return st;
+}
+
+// a node near the void temperature in some frame may change between void and
+// material: the field is void_temp where a frame is at or below it, and is
+// compared with void_temp + 1e-5
+__global__ void k_void_nodes(const double* __restrict__ frames, int n_frames, int nodes,
+                             double void_temp, unsigned char* __restrict__ out) {
+  const int n = blockIdx.x * blockDim.x + threadIdx.x;
+  if (n >= nodes) return;
+  const double nm = void_temp + 0.00001;
+  bool maybe = false, always = true;
+  for (int f = 0; f < n_frames; f++) {
+    const double v = frames[(size_t)f * nodes + n];
+    maybe |= !(v > nm + 1e-6);
+    always &= v <= void_temp;
+  }
+  out[n] = maybe && !always ? 1 : 0;
+}
+
+// box blockIdx.y: the union of the boxes of the elements with a marked node --
+// frame blockIdx.y's nodes at or above `hot`, or with `mark` the marked ones
+__global__ void __launch_bounds__(256)
+k_union_boxes(amca::RmParams P, const double* __restrict__ frames, double hot,
+              const unsigned char* __restrict__ mark, const int* __restrict__ ebox,
+              int* __restrict__ out) {
+  const int ncx = P.fnx - 1, ncy = P.fny - 1, nxy = P.fnx * P.fny;
+  const long long ne = (long long)ncx * ncy * (P.fnz - 1);
+  const double* v = frames + (size_t)blockIdx.y * P.nodes;
+  int lo[3] = {INT_MAX, INT_MAX, INT_MAX}, hi[3] = {INT_MIN, INT_MIN, INT_MIN};
+  for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < ne;
+       e += (long long)gridDim.x * blockDim.x) {
+    const int ei = (int)(e % ncx), ej = (int)((e / ncx) % ncy), ek = (int)(e / ((long long)ncx * ncy));
+    const int n0 = nxy * ek + P.fnx * ej + ei;
+    const int nid[8] = {n0, n0 + 1, n0 + P.fnx, n0 + P.fnx + 1, n0 + nxy, n0 + nxy + 1,
+                        n0 + nxy + P.fnx, n0 + nxy + P.fnx + 1};
+    bool any = false;
+#pragma unroll
+    for (int m = 0; m < 8; m++) any |= mark ? mark[nid[m]] != 0 : v[nid[m]] >= hot;
+    if (!any) continue;
+    const int* b = ebox + 6 * e;
+    for (int a = 0; a < 3; a++) {
+      lo[a] = min(lo[a], b[a]);
+      hi[a] = max(hi[a], b[3 + a]);
+    }
+  }
+  __shared__ int s_b[6];
+  if (threadIdx.x < 6) s_b[threadIdx.x] = threadIdx.x < 3 ? INT_MAX : INT_MIN;
+  __syncthreads();
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    for (int o = 32; o > 0; o >>= 1) {
+      lo[a] = min(lo[a], __shfl_xor(lo[a], o, 64));
+      hi[a] = max(hi[a], __shfl_xor(hi[a], o, 64));
+    }
+    if ((threadIdx.x & 63) == 0) {
+      atomicMin(&s_b[a], lo[a]);
+      atomicMax(&s_b[3 + a], hi[a]);
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < 6) {
+    int* q = out + 6 * (size_t)blockIdx.y + threadIdx.x;
+    if (threadIdx.x < 3 && s_b[threadIdx.x] < INT_MAX) atomicMin(q, s_b[threadIdx.x]);
+    if (threadIdx.x >= 3 && s_b[threadIdx.x] > INT_MIN) atomicMax(q, s_b[threadIdx.x]);
+  }
+}
+
+unsigned grid_for(long long n, int cap = 65536) {
+  return (unsigned)std::max(1LL, std::min<long long>((n + 255) / 256, cap));
 }
 
 }  // namespace
@@ -534,8 +627,22 @@ amca_status amca_remelt_set_fe(amca_remelt* d, int32_t fnx, int32_t fny, int32_t
   vp.tol = d->desc.tolerance;
   vp.max_iter = d->desc.max_iterations;
   bool any = false;
-  RM_TRY(map_voxels_device(mesh, vp, d->host_tag, d->host_par, any));
-  if (!any) return rm_fail(AMCA_ERR_INVALID, "no CA cell lies in the FE mesh");
+  // a new map next to the one in use, which stays if the mesh holds no cell
+  int32_t* tag = nullptr;
+  double* par = nullptr;
+  RM_TRY(d->alloc(&tag, (size_t)P.NG));
+  amca_status st = d->alloc(&par, 3 * (size_t)P.NG);
+  if (st == AMCA_OK) st = map_voxels_device(mesh, vp, tag, par, d->stream, any);
+  if (st == AMCA_OK && !any) st = rm_fail(AMCA_ERR_INVALID, "no CA cell lies in the FE mesh");
+  if (st != AMCA_OK) {
+    d->release(tag);
+    d->release(par);
+    return st;
+  }
+  d->release(d->B.tag);
+  d->release(d->B.par);
+  d->B.tag = tag;
+  d->B.par = par;
   P.fnx = fnx;
   P.fny = fny;
   P.fnz = fnz;
@@ -547,96 +654,50 @@ amca_status amca_remelt_set_fe(amca_remelt* d, int32_t fnx, int32_t fny, int32_t
   d->release((void*)d->B.frame_time);
   d->release(d->B.theta);
   d->release(const_cast<int*>(d->B.frame_hot));
+  d->B.frames = d->B.frame_time = nullptr;
+  d->B.theta = nullptr;
+  d->B.frame_hot = nullptr;
+  d->fe_ready = false;  // until all of it is set
   double *fr = nullptr, *ft = nullptr, *th = nullptr;
   int* fh = nullptr;
-  const size_t ne = (size_t)(fnx - 1) * (fny - 1) * (fnz - 1);
   RM_TRY(d->alloc(&fr, nodes * (size_t)n_frames));
   RM_TRY(d->alloc(&ft, (size_t)n_frames));
   RM_TRY(d->alloc(&th, nodes));
   RM_TRY(d->alloc(&fh, 6 * (size_t)n_frames));
-  // For the active box: the cell box of the elements around each node, then
-  // per frame the union over its hot nodes (at or above Tm - hot_margin), and
-  // the union over nodes whose void state can change between frames.
+  RM_HIP(hipMemcpyAsync(fr, frame_theta, sizeof(double) * nodes * n_frames, hipMemcpyHostToDevice, d->stream));
   {
-    std::vector<int32_t> box(6 * ne);
-    for (size_t e = 0; e < ne; e++) {
-      box[6 * e + 0] = box[6 * e + 1] = box[6 * e + 2] = INT_MAX;
-      box[6 * e + 3] = box[6 * e + 4] = box[6 * e + 5] = INT_MIN;
-    }
-    for (int c = 0; c < P.NG; c++) {
-      const int e = d->host_tag[c];
-      if (e < 0) continue;
-      const int k = c / P.nxyG, j = (c % P.nxyG) / P.nxG, i = (c % P.nxyG) % P.nxG;
-      int32_t* b = &box[6 * (size_t)e];
-      b[0] = std::min(b[0], i);
-      b[1] = std::min(b[1], j);
-      b[2] = std::min(b[2], k);
-      b[3] = std::max(b[3], i);
-      b[4] = std::max(b[4], j);
-      b[5] = std::max(b[5], k);
-    }
-    std::vector<int32_t> nbox(6 * nodes);
-    for (size_t n = 0; n < nodes; n++) {
-      nbox[6 * n + 0] = nbox[6 * n + 1] = nbox[6 * n + 2] = INT_MAX;
-      nbox[6 * n + 3] = nbox[6 * n + 4] = nbox[6 * n + 5] = INT_MIN;
-    }
-    const int ncx = fnx - 1, ncy = fny - 1;
-    for (size_t e = 0; e < ne; e++) {
-      const int32_t* b = &box[6 * e];
-      if (b[0] > b[3]) continue;
-      const int ei = (int)(e % ncx), ej = (int)((e / ncx) % ncy), ek = (int)(e / ((size_t)ncx * ncy));
-      for (int dk = 0; dk < 2; dk++)
-        for (int dj = 0; dj < 2; dj++)
-          for (int di = 0; di < 2; di++) {
-            int32_t* nb = &nbox[6 * (((size_t)(ek + dk) * fny + (ej + dj)) * fnx + (ei + di))];
-            for (int a = 0; a < 3; a++) {
-              nb[a] = std::min(nb[a], b[a]);
-              nb[3 + a] = std::max(nb[3 + a], b[3 + a]);
-            }
-          }
-    }
-    auto add = [](int32_t* dst, const int32_t* b) {
-      if (b[0] > b[3]) return;
-      for (int a = 0; a < 3; a++) {
-        dst[a] = std::min(dst[a], b[a]);
-        dst[3 + a] = std::max(dst[3 + a], b[3 + a]);
-      }
+    const long long ne = (long long)(fnx - 1) * (fny - 1) * (fnz - 1);
+    DeviceTemp ebox, mark, vbox;
+    RM_HIP(ebox.get(sizeof(int) * 6 * (size_t)ne));
+    RM_HIP(mark.get(nodes));
+    RM_HIP(vbox.get(sizeof(int) * 6));
+    int* eb = static_cast<int*>(ebox.p);
+    int* vb = static_cast<int*>(vbox.p);
+    unsigned char* mk = static_cast<unsigned char*>(mark.p);
+    const auto clear = [&](long long n, int* b) {
+      hipLaunchKernelGGL(k_box_clear, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, d->stream, n, b);
     };
-    const double hot = P.Tm - P.hot_margin;
-    const double nm = P.void_temp + 0.00001;
-    std::vector<int32_t> fhot(6 * (size_t)n_frames);
-    std::vector<unsigned char> maybe_void(nodes, 0), always_void(nodes, 1);
-    for (int f = 0; f < n_frames; f++) {
-      int32_t* fb = &fhot[6 * (size_t)f];
-      fb[0] = fb[1] = fb[2] = INT_MAX;
-      fb[3] = fb[4] = fb[5] = INT_MIN;
-      const double* v = frame_theta + (size_t)f * nodes;
-      for (size_t n = 0; n < nodes; n++) {
-        if (v[n] >= hot) add(fb, &nbox[6 * n]);
-        // the field is void_temp where a frame is at or below it, and is
-        // compared with void_temp + 1e-5: a node near that value in some
-        // frame may change between void and material
-        if (!(v[n] > nm + 1e-6)) maybe_void[n] = 1;
-        if (!(v[n] <= P.void_temp)) always_void[n] = 0;
-      }
-    }
-    int32_t vb[6] = {INT_MAX, INT_MAX, INT_MAX, INT_MIN, INT_MIN, INT_MIN};
-    for (size_t n = 0; n < nodes; n++)
-      if (maybe_void[n] && !always_void[n]) add(vb, &nbox[6 * n]);
-    for (int a = 0; a < 6; a++) P.void_box[a] = vb[a];
-    RM_HIP(hipMemcpyAsync(fh, fhot.data(), sizeof(int32_t) * fhot.size(), hipMemcpyHostToDevice,
-                          d->stream));
+    clear(6 * ne, eb);
+    clear(6, vb);
+    clear(6LL * n_frames, fh);
+    hipLaunchKernelGGL(k_elem_boxes, dim3(grid_for(P.NG, 16384)), dim3(256), 0, d->stream, P, tag, eb);
+    hipLaunchKernelGGL(k_void_nodes, dim3((unsigned)((nodes + 255) / 256)), dim3(256), 0, d->stream,
+                       fr, n_frames, (int)nodes, P.void_temp, mk);
+    for (int f = 0; f < n_frames; f += 32768)  // frames on the grid's y axis (65535 at most)
+      hipLaunchKernelGGL(k_union_boxes, dim3(grid_for(ne, 64), std::min(32768, n_frames - f)),
+                         dim3(256), 0, d->stream, P, fr + (size_t)f * nodes, P.Tm - P.hot_margin,
+                         (const unsigned char*)nullptr, eb, fh + 6 * (size_t)f);
+    hipLaunchKernelGGL(k_union_boxes, dim3(grid_for(ne, 256)), dim3(256), 0, d->stream, P, fr, 0.0,
+                       mk, eb, vb);
+    RM_HIP(hipGetLastError());
+    RM_HIP(hipMemcpyAsync(P.void_box, vb, sizeof(int) * 6, hipMemcpyDeviceToHost, d->stream));
     RM_HIP(hipStreamSynchronize(d->stream));
   }
   std::vector<double> rel(n_frames);
   for (int f = 0; f < n_frames; f++) rel[f] = frame_time[f] - frame_time[0];  // inTimeOffset_
-  RM_HIP(hipMemcpyAsync(fr, frame_theta, sizeof(double) * nodes * n_frames, hipMemcpyHostToDevice, d->stream));
   RM_HIP(hipMemcpyAsync(ft, rel.data(), sizeof(double) * n_frames, hipMemcpyHostToDevice, d->stream));
   // thetaArray_ starts as theta_[1], the first frame
-  RM_HIP(hipMemcpyAsync(th, frame_theta, sizeof(double) * nodes, hipMemcpyHostToDevice, d->stream));
-  RM_HIP(hipMemcpyAsync(d->B.tag, d->host_tag.data(), sizeof(int32_t) * P.NG, hipMemcpyHostToDevice, d->stream));
-  RM_HIP(hipMemcpyAsync(d->B.par, d->host_par.data(), sizeof(double) * 3 * (size_t)P.NG,
-                        hipMemcpyHostToDevice, d->stream));
+  RM_HIP(hipMemcpyAsync(th, fr, sizeof(double) * nodes, hipMemcpyDeviceToDevice, d->stream));
   d->B.frames = fr;
   d->B.frame_time = ft;
   d->B.theta = th;
@@ -658,8 +719,10 @@ amca_status amca_remelt_set_fe(amca_remelt* d, int32_t fnx, int32_t fny, int32_t
 
 amca_status amca_remelt_voxel_map(amca_remelt* d, int32_t* tag, double* par) {
   if (!d || !d->fe_ready) return rm_fail(AMCA_ERR_INVALID, "FE mesh not set");
-  if (tag) std::memcpy(tag, d->host_tag.data(), sizeof(int32_t) * d->P.NG);
-  if (par) std::memcpy(par, d->host_par.data(), sizeof(double) * 3 * (size_t)d->P.NG);
+  RM_HIP(hipStreamSynchronize(d->stream));
+  if (tag) RM_HIP(hipMemcpy(tag, d->B.tag, sizeof(int32_t) * d->P.NG, hipMemcpyDeviceToHost));
+  if (par)
+    RM_HIP(hipMemcpy(par, d->B.par, sizeof(double) * 3 * (size_t)d->P.NG, hipMemcpyDeviceToHost));
   return AMCA_OK;
 }
 
@@ -706,14 +769,113 @@ amca_status amca_fe_map_voxels_device(int32_t nx, int32_t ny, int32_t nz, double
   for (int q = 0; q < 3; q++) vp.bin[q] = (bin && bin[q] > 0) ? bin[q] : 10;
   vp.tol = tolerance;
   vp.max_iter = max_iterations;
-  std::vector<int32_t> t;
-  std::vector<double> p;
+  const size_t NG = (size_t)(nx + 2) * (ny + 2) * (nz + 2);
+  DeviceTemp dtag, dpar;
+  RM_HIP(dtag.get(sizeof(int32_t) * NG));
+  RM_HIP(dpar.get(sizeof(double) * 3 * NG));
   bool any = false;
-  RM_TRY(map_voxels_device(mesh, vp, t, p, any));
-  std::memcpy(tag, t.data(), sizeof(int32_t) * t.size());
-  std::memcpy(par, p.data(), sizeof(double) * p.size());
+  RM_TRY(map_voxels_device(mesh, vp, static_cast<int32_t*>(dtag.p), static_cast<double*>(dpar.p), 0,
+                           any));
+  RM_HIP(hipMemcpy(tag, dtag.p, sizeof(int32_t) * NG, hipMemcpyDeviceToHost));
+  RM_HIP(hipMemcpy(par, dpar.p, sizeof(double) * 3 * NG, hipMemcpyDeviceToHost));
   return any ? AMCA_OK : rm_fail(AMCA_ERR_INVALID, "no CA cell lies in the FE mesh");
 }
+
+namespace {
+
+// ---- loading a state (amca_remelt_set_state) --------------------------------
+// The checks and the layout of a loaded state, from the caller's arrays as they
+// are: one upload of 9 bytes per cell and 8 per record, then kernels.  The host
+// loops over cells and records took 89 ms at 400 x 160 x 80 cells.
+
+// smallest key of a failed check, per pass: cell or record index, and what failed
+struct StateErr {
+  unsigned long long record_orient, cell, no_record, record_cell;  // ~0: none
+  unsigned long long grainless;
+};
+enum : unsigned { kBadOrient = 0, kBadGrain = 1, kShared = 2 };
+
+__device__ __forceinline__ bool state_interior(const amca::RmParams& P, long long c) {
+  const int k = (int)c / P.nxyG, r = (int)c - k * P.nxyG, j = r / P.nxG, i = r - j * P.nxG;
+  return !(i == 0 || j == 0 || k == 0 || i == P.nxG - 1 || j == P.nyG - 1 || k == P.nzG - 1);
+}
+
+__global__ void k_state_records(amca::RmParams P, int n_orient, int n_grains,
+                                const int* __restrict__ gcell, const int* __restrict__ gorient,
+                                int* __restrict__ owner, StateErr* err) {
+  const long long stride = (long long)gridDim.x * blockDim.x;
+  for (long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x; g < n_grains; g += stride) {
+    owner[g] = INT_MAX;
+    if (gorient[g] < 0 || gorient[g] >= n_orient)
+      atomicMin(&err->record_orient, (unsigned long long)g);
+    if (gcell[g] < 0 || gcell[g] >= P.NG) atomicMin(&err->record_cell, (unsigned long long)g);
+  }
+}
+
+// the first cell of every record, the cells' own checks and the grainless count
+__global__ void __launch_bounds__(256)
+k_state_cells(amca::RmParams P, int n_orient, int n_grains, const int* __restrict__ orient,
+              const int* __restrict__ grain, int* __restrict__ owner, StateErr* err) {
+  const long long stride = (long long)gridDim.x * blockDim.x;
+  unsigned less = 0;
+  for (long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x; c < P.NG; c += stride) {
+    if (!state_interior(P, c)) continue;
+    const int g = grain[c], o = orient[c];
+    if (o < -1 || o >= n_orient)
+      atomicMin(&err->cell, 4ull * (unsigned long long)c + kBadOrient);
+    else if (g >= n_grains)
+      atomicMin(&err->cell, 4ull * (unsigned long long)c + kBadGrain);
+    if (g < 0) {
+      less++;
+      if (o <= -1) atomicMin(&err->no_record, (unsigned long long)c);
+    } else if (g < n_grains) {
+      atomicMin(&owner[g], (int)c);
+    }
+  }
+  for (int o = 32; o > 0; o >>= 1) less += __shfl_xor(less, o, 64);
+  if ((threadIdx.x & 63) == 0 && less) atomicAdd(&err->grainless, (unsigned long long)less);
+}
+
+__global__ void k_state_shared(amca::RmParams P, int n_grains, const int* __restrict__ grain,
+                               const int* __restrict__ owner, StateErr* err) {
+  const long long stride = (long long)gridDim.x * blockDim.x;
+  for (long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x; c < P.NG; c += stride) {
+    if (!state_interior(P, c)) continue;
+    const int g = grain[c];
+    if (g >= 0 && g < n_grains && owner[g] != (int)c)
+      atomicMin(&err->cell, 4ull * (unsigned long long)c + kShared);
+  }
+}
+
+// retrieve_grain_information_before_simulation (:312-332): ghosts liquid, other
+// cells without an orientation take their grain's; grain records with the centre
+// reset to the cell centre and zero length (:282-300)
+__global__ void k_state_load(amca::RmParams P, amca::RmBuffers B, int n_grains,
+                             const int* __restrict__ orient, const int* __restrict__ grain,
+                             const unsigned char* __restrict__ melted,
+                             const int* __restrict__ gcell, const int* __restrict__ gorient) {
+  const long long stride = (long long)gridDim.x * blockDim.x;
+  const long long t0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  for (long long c = t0; c < P.NG; c += stride) {
+    int o = -1;
+    if (state_interior(P, c)) {
+      o = orient[c];
+      if (o <= -1) o = gorient[grain[c]];
+    }
+    B.oid[c] = o;
+    B.gid[c] = grain[c];
+    B.melted[c] = melted[c];
+  }
+  for (long long g = t0; g < n_grains; g += stride) {
+    const int c = gcell[g];
+    const int k = c / P.nxyG, r = c - k * P.nxyG, j = r / P.nxG, i = r - j * P.nxG;
+    B.genv[g] = make_double4(P.x0 + P.h * (i - 0.5), P.y0 + P.h * (j - 0.5), P.z0 + P.h * (k - 0.5),
+                             0.0);
+    B.gco[g] = make_int2(c, gorient[g]);
+  }
+}
+
+}  // namespace
 
 amca_status amca_remelt_set_state(amca_remelt* d, const int32_t* orient, const int32_t* grain,
                                   const uint8_t* melted, int32_t n_orient, int32_t n_grains,
@@ -723,77 +885,65 @@ amca_status amca_remelt_set_state(amca_remelt* d, const int32_t* orient, const i
   amca::RmParams& P = d->P;
   if (n_orient < 0 || n_orient > d->rows_pushed)
     return rm_fail(AMCA_ERR_INVALID, "push the loaded orientation rows before the state");
-  for (int g = 0; g < n_grains; g++)
-    if (grain_orient[g] < 0 || grain_orient[g] >= n_orient)
-      return rm_fail(AMCA_ERR_INVALID, "grain orientation out of range");
   // Every interior cell owns at most one grain record and no record is shared:
   // the device grows a record once per flagged cell, as the reference does when
   // each cell carries its own grain.  Records for grainless cells are added by
   // captures and nucleation, so the table needs n_grains + (grainless cells).
-  std::vector<uint8_t> owned((size_t)std::max(n_grains, 1), 0);
-  long long grainless = 0;
-  for (int c = 0; c < P.NG; c++) {
-    const int k = c / P.nxyG, j = (c % P.nxyG) / P.nxG, i = (c % P.nxyG) % P.nxG;
-    if (i == 0 || j == 0 || k == 0 || i == P.nxG - 1 || j == P.nyG - 1 || k == P.nzG - 1) continue;
-    const int g = grain[c];
-    if (orient[c] < -1 || orient[c] >= n_orient)
-      return rm_fail(AMCA_ERR_INVALID, "cell orientation out of range");
-    if (g < 0) {
-      grainless++;
-      continue;
-    }
-    if (g >= n_grains) return rm_fail(AMCA_ERR_INVALID, "cell grain id out of range");
-    if (owned[g]) return rm_fail(AMCA_ERR_INVALID, "a grain record is shared by two cells");
-    owned[g] = 1;
+  const size_t NG = (size_t)P.NG, ng = (size_t)n_grains;
+  const auto up = [](size_t b) { return (b + 255) / 256 * 256; };
+  const size_t cells = up(sizeof(int32_t) * NG), recs = up(sizeof(int32_t) * std::max<size_t>(ng, 1));
+  DeviceTemp tmp;
+  RM_HIP(tmp.get(2 * cells + up(NG) + 3 * recs + sizeof(StateErr)));
+  char* p = static_cast<char*>(tmp.p);
+  int* d_orient = reinterpret_cast<int*>(p);
+  int* d_grain = reinterpret_cast<int*>(p + cells);
+  unsigned char* d_melted = reinterpret_cast<unsigned char*>(p + 2 * cells);
+  int* d_gcell = reinterpret_cast<int*>(p + 2 * cells + up(NG));
+  int* d_gorient = reinterpret_cast<int*>(p + 2 * cells + up(NG) + recs);
+  int* d_owner = reinterpret_cast<int*>(p + 2 * cells + up(NG) + 2 * recs);
+  StateErr* d_err = reinterpret_cast<StateErr*>(p + 2 * cells + up(NG) + 3 * recs);
+  StateErr err{~0ull, ~0ull, ~0ull, ~0ull, 0ull};
+  hipStream_t s = d->stream;
+  RM_HIP(hipMemcpyAsync(d_err, &err, sizeof(err), hipMemcpyHostToDevice, s));
+  RM_HIP(hipMemcpyAsync(d_orient, orient, sizeof(int32_t) * NG, hipMemcpyHostToDevice, s));
+  RM_HIP(hipMemcpyAsync(d_grain, grain, sizeof(int32_t) * NG, hipMemcpyHostToDevice, s));
+  RM_HIP(hipMemcpyAsync(d_melted, melted, NG, hipMemcpyHostToDevice, s));
+  if (ng) {
+    RM_HIP(hipMemcpyAsync(d_gcell, grain_cell, sizeof(int32_t) * ng, hipMemcpyHostToDevice, s));
+    RM_HIP(hipMemcpyAsync(d_gorient, grain_orient, sizeof(int32_t) * ng, hipMemcpyHostToDevice, s));
   }
-  const size_t need = (size_t)n_grains + (size_t)grainless;
+  const dim3 grid(grid_for(P.NG, 16384)), block(256);
+  hipLaunchKernelGGL(k_state_records, dim3(grid_for(n_grains, 16384)), block, 0, s, P, n_orient,
+                     n_grains, d_gcell, d_gorient, d_owner, d_err);
+  hipLaunchKernelGGL(k_state_cells, grid, block, 0, s, P, n_orient, n_grains, d_orient, d_grain,
+                     d_owner, d_err);
+  hipLaunchKernelGGL(k_state_shared, grid, block, 0, s, P, n_grains, d_grain, d_owner, d_err);
+  RM_HIP(hipGetLastError());
+  RM_HIP(hipMemcpyAsync(&err, d_err, sizeof(err), hipMemcpyDeviceToHost, s));
+  RM_HIP(hipStreamSynchronize(s));
+  if (err.record_orient != ~0ull) return rm_fail(AMCA_ERR_INVALID, "grain orientation out of range");
+  if (err.cell != ~0ull)
+    return rm_fail(AMCA_ERR_INVALID, (err.cell & 3u) == kBadOrient ? "cell orientation out of range"
+                                     : (err.cell & 3u) == kBadGrain
+                                         ? "cell grain id out of range"
+                                         : "a grain record is shared by two cells");
+  if (err.no_record != ~0ull)
+    return rm_fail(AMCA_ERR_INVALID, "a cell without orientation has no grain record");
+  if (err.record_cell != ~0ull) return rm_fail(AMCA_ERR_INVALID, "grain cell out of range");
+  const size_t need = ng + (size_t)err.grainless;
   if (need > d->grain_cap) {
-    RM_HIP(hipStreamSynchronize(d->stream));
     d->release(d->B.genv);
     d->release(d->B.gco);
     d->B.genv = nullptr;
     d->B.gco = nullptr;
+    d->grain_cap = 0;
     RM_TRY(d->alloc(&d->B.genv, need));
     RM_TRY(d->alloc(&d->B.gco, need));
     d->grain_cap = need;
   }
-  // retrieve_grain_information_before_simulation (:312-332): ghosts liquid,
-  // other cells without an orientation take their grain's
-  std::vector<int32_t> o(orient, orient + P.NG);
-  const int nxG = P.nxG, nyG = P.nyG, nzG = P.nzG;
-  for (int c = 0; c < P.NG; c++) {
-    const int k = c / P.nxyG, j = (c % P.nxyG) / nxG, i = (c % P.nxyG) % nxG;
-    if (i == 0 || j == 0 || k == 0 || i == nxG - 1 || j == nyG - 1 || k == nzG - 1) {
-      o[c] = -1;
-      continue;
-    }
-    if (o[c] > -1) continue;
-    const int g = grain[c];
-    if (g < 0 || g >= n_grains)
-      return rm_fail(AMCA_ERR_INVALID, "a cell without orientation has no grain record");
-    o[c] = grain_orient[g];
-  }
-  // grain records: centre reset to the cell centre, zero length (:282-300)
-  std::vector<double> env(4 * (size_t)std::max(n_grains, 1));
-  std::vector<int32_t> co(2 * (size_t)std::max(n_grains, 1));
-  for (int g = 0; g < n_grains; g++) {
-    const int c = grain_cell[g];
-    if (c < 0 || c >= P.NG) return rm_fail(AMCA_ERR_INVALID, "grain cell out of range");
-    const int k = c / P.nxyG, j = (c % P.nxyG) / nxG, i = (c % P.nxyG) % nxG;
-    env[4 * (size_t)g + 0] = P.x0 + P.h * (i - 0.5);
-    env[4 * (size_t)g + 1] = P.y0 + P.h * (j - 0.5);
-    env[4 * (size_t)g + 2] = P.z0 + P.h * (k - 0.5);
-    env[4 * (size_t)g + 3] = 0.0;
-    co[2 * (size_t)g] = c;
-    co[2 * (size_t)g + 1] = grain_orient[g];
-  }
-  RM_HIP(hipMemcpyAsync(d->B.oid, o.data(), sizeof(int32_t) * P.NG, hipMemcpyHostToDevice, d->stream));
-  RM_HIP(hipMemcpyAsync(d->B.gid, grain, sizeof(int32_t) * P.NG, hipMemcpyHostToDevice, d->stream));
-  RM_HIP(hipMemcpyAsync(d->B.melted, melted, P.NG, hipMemcpyHostToDevice, d->stream));
-  if (n_grains > 0) {
-    RM_HIP(hipMemcpyAsync(d->B.genv, env.data(), sizeof(double) * 4 * n_grains, hipMemcpyHostToDevice, d->stream));
-    RM_HIP(hipMemcpyAsync(d->B.gco, co.data(), sizeof(int32_t) * 2 * n_grains, hipMemcpyHostToDevice, d->stream));
-  }
+  hipLaunchKernelGGL(k_state_load, grid, block, 0, s, P, d->B, n_grains, d_orient, d_grain, d_melted,
+                     d_gcell, d_gorient);
+  RM_HIP(hipGetLastError());
   amca::RmCounters c;
   RM_TRY(rm_counters(d, &c));
   c.n_grains = n_grains;
@@ -1180,6 +1330,18 @@ amca_status amca_remelt_get_counters(amca_remelt* d, amca_remelt_counters* out) 
   return AMCA_OK;
 }
 
+namespace {
+__global__ void k_split_pairs(long long n, const int2* __restrict__ in, int* __restrict__ x,
+                              int* __restrict__ y) {
+  const long long stride = (long long)gridDim.x * blockDim.x;
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+    const int2 v = in[i];
+    x[i] = v.x;
+    y[i] = v.y;
+  }
+}
+}  // namespace
+
 amca_status amca_remelt_download(amca_remelt* d, int32_t* orient, int32_t* grain, double* T,
                                  uint8_t* melted, uint8_t* cooling, int32_t grain_cap,
                                  double* genv, int32_t* gcell, int32_t* gorient, int32_t* n_grains) {
@@ -1197,12 +1359,15 @@ amca_status amca_remelt_download(amca_remelt* d, int32_t* orient, int32_t* grain
   if (m > 0) {
     if (genv) RM_HIP(hipMemcpy(genv, d->B.genv, sizeof(double) * 4 * m, hipMemcpyDeviceToHost));
     if (gcell || gorient) {
-      std::vector<int32_t> co(2 * m);
-      RM_HIP(hipMemcpy(co.data(), d->B.gco, sizeof(int32_t) * 2 * m, hipMemcpyDeviceToHost));
-      for (size_t g = 0; g < m; g++) {
-        if (gcell) gcell[g] = co[2 * g];
-        if (gorient) gorient[g] = co[2 * g + 1];
-      }
+      DeviceTemp split;  // cells, then orientations
+      RM_HIP(split.get(sizeof(int32_t) * 2 * m));
+      int* q = static_cast<int*>(split.p);
+      hipLaunchKernelGGL(k_split_pairs, dim3(grid_for((long long)m, 16384)), dim3(256), 0, d->stream,
+                         (long long)m, d->B.gco, q, q + m);
+      RM_HIP(hipGetLastError());
+      RM_HIP(hipStreamSynchronize(d->stream));
+      if (gcell) RM_HIP(hipMemcpy(gcell, q, sizeof(int32_t) * m, hipMemcpyDeviceToHost));
+      if (gorient) RM_HIP(hipMemcpy(gorient, q + m, sizeof(int32_t) * m, hipMemcpyDeviceToHost));
     }
   }
   return AMCA_OK;

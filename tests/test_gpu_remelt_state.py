@@ -1,0 +1,127 @@
+"""Loading a state into a coupled domain: every refusal with its message (the
+first failing cell's, in cell order), what a refused state leaves in place, and the
+layout of an accepted one, against a restatement here."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+NX, NY, NZ, H = 6, 5, 4, 2e-6
+
+
+def _domain(amca, rows=3):
+    from amca3d_amd.remelt import RemeltDomain
+    d = RemeltDomain(dict(nx=NX, ny=NY, nz=NZ, h=H, x0=1e-6, y0=2e-6, z0=3e-6, Tm=1600.0, Ts=1550.0,
+                          Tmin_nuc=1550.0, a1=-0.544e-4, a2=2.03e-4, a3=0.0, b1=1.0, b2=2.0, b3=3.0,
+                          trunc=1.7, time_step_factor=0.2, cutoff_factor=4.0, final_time=1.0,
+                          void_temperature=200.0, bin=(5, 5, 5), tolerance=1e-16, max_iterations=20,
+                          initial_melted=0), 64)
+    d.push_orientations(np.zeros((rows, 3)))
+    return d
+
+
+def _interior():
+    k, j, i = np.meshgrid(np.arange(1, NZ + 1), np.arange(1, NY + 1), np.arange(1, NX + 1),
+                          indexing="ij")
+    return ((k * (NY + 2) + j) * (NX + 2) + i).ravel().astype(np.int32)
+
+
+def _state(holes=0):
+    """Every interior cell with its own record, the last `holes` of them without one."""
+    ng = (NX + 2) * (NY + 2) * (NZ + 2)
+    cells = _interior()
+    n = len(cells) - holes
+    rng = np.random.default_rng(1)
+    ori = np.full(ng, 7, np.int32)      # ghost values are not looked at
+    gid = np.full(ng, -5, np.int32)
+    perm = rng.permutation(n).astype(np.int32)   # ids in no particular cell order
+    ori[cells] = rng.integers(0, 3, len(cells))
+    ori[cells[::4][: n // 4]] = -1                # these take their record's orientation
+    gid[cells[:n]] = perm
+    if holes:
+        ori[cells[n:]] = 1
+        gid[cells[n:]] = -1
+    gcell = np.empty(n, np.int32)
+    gcell[perm] = cells[:n]
+    return dict(ori=ori, gid=gid, melted=rng.integers(0, 2, ng).astype(np.uint8),
+                euler=np.zeros((3, 3)), grain_cell=gcell,
+                grain_orient=rng.integers(0, 3, n).astype(np.int32))
+
+
+@pytest.mark.parametrize("holes", [0, 9])
+def test_loaded_layout(amca, holes):
+    d = _domain(amca)
+    st = _state(holes)
+    d.set_state(st)
+    g = d.download()
+    cells = _interior()
+    ori = np.full_like(st["ori"], -1)
+    ori[cells] = np.where(st["ori"][cells] > -1, st["ori"][cells],
+                          st["grain_orient"][np.maximum(st["gid"][cells], 0)])
+    assert np.array_equal(g["ori"], ori)
+    assert np.array_equal(g["gid"], st["gid"])
+    assert np.array_equal(g["melted"], st["melted"])
+    assert np.array_equal(g["grain_cell"], st["grain_cell"])
+    assert np.array_equal(g["grain_orient"], st["grain_orient"])
+    c = st["grain_cell"].astype(np.int64)
+    k, r = c // ((NX + 2) * (NY + 2)), c % ((NX + 2) * (NY + 2))
+    j, i = r // (NX + 2), r % (NX + 2)
+    env = np.stack([1e-6 + H * (i - 0.5), 2e-6 + H * (j - 0.5), 3e-6 + H * (k - 0.5), 0.0 * i], 1)
+    assert np.array_equal(g["grain_env"], env)
+    d.close()
+
+
+CELLS = _interior()
+
+
+def _set(key, at, value):
+    def f(st):
+        st[key][at] = value
+    return f
+
+
+def _share(a, b):
+    def f(st):
+        st["gid"][CELLS[b]] = st["gid"][CELLS[a]]
+    return f
+
+
+@pytest.mark.parametrize("edits,message", [
+    ([_set("grain_orient", 5, 3)], "grain orientation out of range"),
+    ([_set("grain_orient", 0, -1)], "grain orientation out of range"),
+    ([_set("ori", CELLS[-1], 3)], "cell orientation out of range"),
+    ([_set("ori", CELLS[0], -2)], "cell orientation out of range"),
+    ([_set("gid", CELLS[11], NX * NY * NZ)], "cell grain id out of range"),
+    ([_share(3, 90)], "a grain record is shared by two cells"),
+    # the first failing cell decides: the shared record's second cell comes first here
+    ([_share(3, 10), _set("ori", CELLS[40], 9)], "a grain record is shared by two cells"),
+    ([_share(3, 50), _set("ori", CELLS[40], 9)], "cell orientation out of range"),
+    # in one cell: orientation before grain id
+    ([_set("gid", CELLS[11], 10 ** 6), _set("ori", CELLS[11], 3)], "cell orientation out of range"),
+    ([_set("gid", CELLS[7], -1), _set("ori", CELLS[7], -1)],
+     "a cell without orientation has no grain record"),
+    ([_set("grain_cell", 2, -1)], "grain cell out of range"),
+    ([_set("grain_cell", 2, (NX + 2) * (NY + 2) * (NZ + 2))], "grain cell out of range"),
+])
+def test_refusals(amca, edits, message):
+    from amca3d_amd import AmcaError
+    d = _domain(amca)
+    d.set_state(_state())
+    before = d.download()
+    st = _state()
+    for e in edits:
+        e(st)
+    with pytest.raises(AmcaError, match=message):
+        d.set_state(st)
+    after = d.download()
+    for f in ("ori", "gid", "melted", "grain_env", "grain_cell", "grain_orient"):
+        assert np.array_equal(before[f], after[f]), f
+    d.close()
+
+
+def test_rows_come_first(amca):
+    from amca3d_amd import AmcaError
+    d = _domain(amca, rows=2)
+    with pytest.raises(AmcaError, match="push the loaded orientation rows"):
+        d.set_state(_state())
+    d.close()
