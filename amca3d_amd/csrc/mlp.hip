@@ -276,10 +276,16 @@ amca_status train_blocks(amca_mlp* h, int n, int* blocks) {
   return AMCA_OK;
 }
 
-// the weight images follow the parameters: on the network's stream
-// after whatever changed them
-amca_status repack(amca_mlp* h) {
+// the parameters from host memory, Adam's moments from zero, and the weight
+// images, all on the network's stream and complete on return
+amca_status load_params(amca_mlp* h, const float* p) {
+  const size_t bytes = sizeof(float) * h->lay.total;
+  MLP_HIP(hipMemcpyAsync(h->params, p, bytes, hipMemcpyHostToDevice, h->stream));
+  MLP_HIP(hipMemsetAsync(h->adam_m, 0, bytes, h->stream));
+  MLP_HIP(hipMemsetAsync(h->adam_v, 0, bytes, h->stream));
+  h->adam_t = 0;
   MLP_HIP(launch_pack(h->params, h->image, h->stream));
+  MLP_HIP(hipStreamSynchronize(h->stream));
   return AMCA_OK;
 }
 
@@ -340,14 +346,13 @@ amca_status amca_mlp_create(uint64_t seed, amca_mlp** out) {
       std::uniform_real_distribution<float> U(-a, a);
       for (int i = 0; i < kFanIn[l] * kFanOut[l]; i++) p[h->lay.w[l] + i] = U(rng);
     }
-    if (hipMemcpy(h->params, p.data(), sizeof(float) * P, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemset(h->adam_m, 0, sizeof(float) * P) != hipSuccess ||
-        hipMemset(h->adam_v, 0, sizeof(float) * P) != hipSuccess ||
-        hipMemset(h->image, 0, net_image_bytes()) != hipSuccess) {  // its padding stays zero
+    // on the network's stream, which does not wait for the null stream; the image's
+    // padding stays zero
+    if (hipMemsetAsync(h->image, 0, net_image_bytes(), h->stream) != hipSuccess) {
       st = mlp_fail(AMCA_ERR_HIP, "upload");
       break;
     }
-    st = repack(h);
+    st = load_params(h, p.data());
   } while (0);
   if (st != AMCA_OK) {
     delete h;
@@ -364,11 +369,7 @@ amca_status amca_mlp_destroy(amca_mlp* h) {
 
 amca_status amca_mlp_set_params(amca_mlp* h, const float* p) {
   if (!h || !p) return mlp_fail(AMCA_ERR_INVALID, "null argument");
-  MLP_HIP(hipMemcpy(h->params, p, sizeof(float) * h->lay.total, hipMemcpyHostToDevice));
-  MLP_HIP(hipMemset(h->adam_m, 0, sizeof(float) * h->lay.total));
-  MLP_HIP(hipMemset(h->adam_v, 0, sizeof(float) * h->lay.total));
-  h->adam_t = 0;
-  return repack(h);
+  return load_params(h, p);
 }
 
 amca_status amca_mlp_get_params(amca_mlp* h, float* p) {

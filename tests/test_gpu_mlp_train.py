@@ -91,3 +91,23 @@ def test_adam_steps_and_loss_trace(amca):
     hip.close()
     m.close()
     ref.close()
+
+
+def test_training_right_after_create_repeats(amca):
+    """A network's first steps use the parameters it was created with (its setup is
+    complete when create or set_params returns), so two of a seed end the same."""
+    from amca3d_amd import surrogate as S
+    rng = np.random.default_rng(8)
+    X = rng.uniform(-1, 1, (256, 5)).astype(np.float32)
+    Y = rng.uniform(-1, 1, 256).astype(np.float32)
+    hip = _Hip()
+    dX, dY = hip.upload(X), hip.upload(Y)
+    first = None
+    for _ in range(20):
+        m = S.MLP(5)
+        assert S.lib().amca_mlp_train_device(m.h, 256, dX, dY, 256, 3, 1e-3, 9, None) == 0
+        p = m.params()
+        m.close()
+        first = p if first is None else first
+        np.testing.assert_array_equal(p.view(np.uint32), first.view(np.uint32))
+    hip.close()
