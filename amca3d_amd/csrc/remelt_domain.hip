@@ -350,6 +350,13 @@ amca_status amca_remelt_create(const amca_remelt_desc* desc, int32_t orient_capa
   P.final_time = desc->final_time;
   P.void_temp = desc->void_temperature;
   P.orient_cap = orient_capacity;
+  // A part takes the cells of every kRmParts-th of n blocks, each walking its 256
+  // threads through up to NG cells in strides of 256 n: at most
+  // 256 (NG / (256 n) + 1) (n / kRmParts + 1) cells, with n at most 16384 and at least
+  // 512 or NG / 256.
+  P.flist_cap = (int)std::min<long long>(
+      INT_MAX, NG / amca::kRmParts + NG / 512 + 256 * (16384 / amca::kRmParts + 3));
+  if (P.flist_cap > P.N) P.flist_cap = (int)P.N;  // one entry per interior cell
   P.window = 1;
   P.hot_margin = 1.0;
   P.sur_hot[0] = 1;
@@ -379,6 +386,8 @@ amca_status amca_remelt_create(const amca_remelt_desc* desc, int32_t orient_capa
   A(&B.par, 3 * ng);
   A(&B.claim, ng);
   A(&B.msk, ng);
+  A(&B.flist, (size_t)amca::kRmParts * P.flist_cap);
+  A(&B.clist, (size_t)P.N);
   A(&B.genv, nc);
   A(&B.gco, nc);
   d->grain_cap = nc;
@@ -405,6 +414,7 @@ amca_status amca_remelt_create(const amca_remelt_desc* desc, int32_t orient_capa
   (void)hipMemsetAsync(B.oid, 0xff, sizeof(int) * ng, d->stream);
   (void)hipMemsetAsync(B.melted, desc->initial_melted ? 1 : 0, ng, d->stream);
   (void)hipMemsetAsync(B.lb_flag, 0, sizeof(unsigned) * amca::kMaxBlocks, d->stream);
+  (void)hipMemsetAsync(B.rowcnt, 0, sizeof(int) * (size_t)P.nx * P.ny, d->stream);
   amca::RmCounters c{};
   for (int q = 0; q < 64; q++) c.min_t_keys[q] = ~0ull;
   c.last_step = -1;

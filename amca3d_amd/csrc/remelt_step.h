@@ -5,6 +5,8 @@
 
 namespace amca {
 
+constexpr int kRmParts = 8;  // parts of the flagged-cell list, by block of k_rm_nucleate_mint
+
 struct RmParams {
   int nx, ny, nz;
   int nxG, nyG, nzG;
@@ -20,6 +22,7 @@ struct RmParams {
   int fnx, fny, fnz, nodes, ncx, ncy;    // structured FE mesh
   int n_frames;
   int orient_cap;
+  int flist_cap;         // entries of a part of the flagged-cell list
   // temperature surrogate (sur = 1): moving-frame tables on a xi lattice of
   // spacing sur_dxi from sur_xi0; FE fallback within sur_band of Tm and in
   // elements whose nodes disagree with the surrogate by more than sur_resid
@@ -64,6 +67,7 @@ struct RmCounters {
   int skip, exhausted;
   int n_grains, n_orient, n_sites;
   int step_nuc, step_cap, step_fresh;
+  int n_flag[kRmParts];  // entries per part of the flagged-cell list
   int err;
   int log_cap;
   int n_fallback;      // cells of the running step that took the FE path
@@ -105,6 +109,10 @@ struct RmBuffers {
   double* par;            // parametric coordinates, 3 per cell [3*NG]
   int* claim;             // smallest claiming sweep key, INT_MAX when free [NG]
   unsigned* msk;          // per flagged cell: enclosed / captured neighbour slots [NG]
+  int* flist;             // the step's flagged cells that carry a grain, in no order
+                          // [kRmParts * flist_cap]
+  int2* clist;            // the step's captures: capturing cell; slot, rank among the cell's
+                          // fresh captures << 5, fresh << 10 [N]
   double4* genv;          // grain envelope by grain id [N]
   int2* gco;              // grain -> (cell, orientation) [N]
   const double* frames;   // nodal frames [n_frames * nodes]

@@ -18,7 +18,9 @@
 //                       (checkup_liquid_cell_neigh_to_growth, :485-542)
 //   k_rm_nucleate_mint  nucleation sites, remelting variant (:936-999), and in
 //                       the same launch the length cutoff and the minimum
-//                       flagged temperature (:656-727)
+//                       flagged temperature (:656-727), and the list of the
+//                       flagged cells (a few thousand of a box of some hundred
+//                       thousand) that the sweep works on
 //   k_rm_claim          dt = min(factor*h/v(minT), dT_FE); growth of every
 //                       flagged grain and claims on enclosed liquid neighbours
 //                       (single_integration_step, :544-652)
@@ -850,12 +852,12 @@ __device__ __forceinline__ void rm_nucleate_body(const RmParams& P, const RmBuff
 }
 
 // dt = min(dT_FE, min(factor*h/v(minT), dT_FE)) from the minimum flagged
-// temperature (every block of k_rm_claim computes it the same way)
+// temperature (the first wave of every block of k_rm_claim computes it)
 __device__ __forceinline__ double rm_step_dt(const RmParams& P, const RmCounters* ctr) {
   double minT = P.Tm;
-  unsigned long long key = ~0ull;
+  unsigned long long key = ctr->min_t_keys[threadIdx.x & 63];
 #pragma unroll
-  for (int q = 0; q < 64; q++) key = min(key, ctr->min_t_keys[q]);
+  for (int o = 32; o > 0; o >>= 1) key = min(key, (unsigned long long)__shfl_xor(key, o, 64));
   if (key != ~0ull) {
     const double m = dkey_inv(key);
     if (minT > m) minT = m;
@@ -871,11 +873,15 @@ __device__ __forceinline__ double rm_step_dt(const RmParams& P, const RmCounters
 __device__ __forceinline__ void rm_mint_body(const RmParams& P, const RmBuffers& B, int blk,
                                              int nblk) {
   RmCounters* ctr = B.ctr;
+  constexpr int kStage = 512;
   __shared__ unsigned long long s_min;
-  __shared__ int s_cnt;
+  __shared__ int s_cnt, s_n, s_base;
+  __shared__ int s_list[kStage];
+  int* part = B.flist + (size_t)(blk % kRmParts) * P.flist_cap;
   if (threadIdx.x == 0) {
     s_min = ~0ull;
     s_cnt = 0;
+    s_n = 0;
   }
   __syncthreads();
   unsigned long long mk = ~0ull;
@@ -899,6 +905,11 @@ __device__ __forceinline__ void rm_mint_body(const RmParams& P, const RmBuffers&
     cnt++;
     if (rm_ghost_ijk(P, i, j, k)) continue;
     if (g < 0) continue;
+    const int at = atomicAdd(&s_n, 1);
+    if (at < kStage)
+      s_list[at] = c;
+    else
+      part[atomicAdd(&ctr->n_flag[blk % kRmParts], 1)] = c;
     const double L = B.genv[g].w;
     if (!(L < P.cutoff)) B.genv[g].w = P.h;  // length reset (:688-694)
     if (Tc <= P.Ts) continue;
@@ -908,10 +919,14 @@ __device__ __forceinline__ void rm_mint_body(const RmParams& P, const RmBuffers&
   if (mk != ~0ull) atomicMin(&s_min, mk);
   if (cnt) atomicAdd(&s_cnt, cnt);
   __syncthreads();
+  const int staged = min(s_n, kStage);
   if (threadIdx.x == 0) {
     if (s_min != ~0ull) atomicMin(&ctr->min_t_keys[blk & 63], s_min);
     if (s_cnt) atomicAdd(&ctr->flagged_parts[blk & 63], s_cnt);
+    if (staged) s_base = atomicAdd(&ctr->n_flag[blk % kRmParts], staged);
   }
+  __syncthreads();
+  for (int q = threadIdx.x; q < staged; q += blockDim.x) part[s_base + q] = s_list[q];
 }
 
 // Nucleation at the sites (blocks 0 .. site_blocks-1) and the minimum flagged
@@ -927,7 +942,12 @@ __global__ void __launch_bounds__(kRmBlock) k_rm_nucleate_mint(RmParams P, RmBuf
     rm_mint_body(P, B, (int)blockIdx.x - site_blocks, (int)gridDim.x - site_blocks);
 }
 
-// The sweep kernels run one thread per interior cell of the box (i fastest).
+// The sweep kernels work on the list of flagged cells, half a wave per cell: lane
+// s (of 32) takes the cell's neighbour slot s.  One thread per cell of the box ran
+// its 26 neighbours one after the other in the few lanes that held a flagged cell
+// (k_rm_claim 16 us and k_rm_emit 13 us a step at 4.7 K flagged cells, 224 captures;
+// now 4.6 and 4.2).  The list's order does not matter: a claim is decided by
+// its sweep key, fresh ids by row.
 // Rows (i, j) keep the x-major sweep order: row r = (i - i0) * ny_box + (j - j0),
 // and per-row counts of fresh captures give each row its first new grain id.
 struct RmRows {
@@ -942,25 +962,46 @@ __device__ __forceinline__ RmRows rm_rows_of(const RmParams& P, const RmBox& b) 
 __device__ __forceinline__ RmRows rm_rows(const RmParams& P, const RmCounters* ctr) {
   return rm_rows_of(P, rm_step_box(ctr));
 }
-__device__ __forceinline__ void rm_cell_of(const RmRows& w, int q, int& i, int& j, int& k) {
-  const int exy = w.ex * w.ey;
-  k = w.k0 + q / exy;
-  const int rem = q - (k - w.k0) * exy;
-  j = w.j0 + rem / w.ex;
-  i = w.i0 + rem % w.ex;
+
+// The list of flagged cells lies in kRmParts parts, one counter each, so that the
+// blocks that build it rarely meet at one address (with one counter
+// k_rm_nucleate_mint took 3 us longer).  Entry q of all of them, as (part, place).
+struct RmList {
+  int start[kRmParts + 1];
+};
+__device__ __forceinline__ void rm_list(const RmCounters* ctr, RmList& l) {
+  l.start[0] = 0;
+#pragma unroll
+  for (int p = 0; p < kRmParts; p++) l.start[p + 1] = l.start[p] + ctr->n_flag[p];
+}
+__device__ __forceinline__ int rm_list_cell(const RmParams& P, const RmBuffers& B, const RmList& l,
+                                            int q) {
+  int p = 0;
+#pragma unroll
+  for (int x = 1; x < kRmParts; x++) p += q >= l.start[x] ? 1 : 0;
+  int s = 0;
+#pragma unroll
+  for (int x = 1; x < kRmParts; x++)
+    if (q >= l.start[x]) s = l.start[x];
+  return B.flist[(size_t)p * P.flist_cap + (q - s)];
 }
 
 constexpr unsigned kSlotBits = (1u << 26) - 1u;  // msk: captured slots; bits 26.. fresh count
+constexpr int kRmSub = 32;                       // lanes per flagged cell
 
 __global__ void __launch_bounds__(kRmBlock) k_rm_claim(RmParams P, RmBuffers B) {
   const RmCounters* ctr = B.ctr;
   if (ctr->skip) return;
-  const RmRows w = rm_rows(P, ctr);
-  const int total = w.ex * w.ey * w.ez;
-  // dt is the same for every thread: one thread per block evaluates it (three
-  // pow calls) for the rest
+  RmList lst;
+  rm_list(ctr, lst);
+  const int n = lst.start[kRmParts];
+  // dt is the same for every thread: one wave per block evaluates it (three pow
+  // calls) for the rest, whose first loads are under way meanwhile
   __shared__ double s_dt;
-  if (threadIdx.x == 0) s_dt = rm_step_dt(P, ctr);
+  if (threadIdx.x < 64) {
+    const double dt = rm_step_dt(P, ctr);
+    if (threadIdx.x == 0) s_dt = dt;
+  }
   __syncthreads();
   const double dt = s_dt, vts = P.vts;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -969,53 +1010,43 @@ __global__ void __launch_bounds__(kRmBlock) k_rm_claim(RmParams P, RmBuffers B) 
     B.ctr->step_cap = 0;
     B.ctr->step_fresh = 0;
   }
-  const int stride = gridDim.x * blockDim.x;
-  for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < total; q += stride) {
-    int i, j, k;
-    rm_cell_of(w, q, i, j, k);
-    if (k == w.k0) B.rowcnt[(i - w.i0) * w.ey + (j - w.j0)] = 0;
-    const int c = k * P.nxyG + j * P.nxG + i;
-    const unsigned char fl = B.flag[c];
-    const int g = B.gid[c];
-    if (!fl) continue;
-    if (g < 0) continue;
-    double4 e = B.genv[g];
-    const double Tc = B.T[c];
-    const int o = B.gco[g].y;
-    // neighbour state, loaded before any store or atomic
-    int no[26];
+  const int s = threadIdx.x & (kRmSub - 1);
+  int di, dj, dk;
+  slot_delta(s < 26 ? s : 0, di, dj, dk);
+  const int off = dk * P.nxyG + dj * P.nxG + di;
+  const int stride = gridDim.x * (kRmBlock / kRmSub);
+  const int first = (blockIdx.x * kRmBlock + threadIdx.x) / kRmSub;
+  for (int q = first; q - first < n; q += stride) {  // whole waves go round together
+    bool in = false;
+    int c = 0;
+    if (q < n) {
+      c = rm_list_cell(P, B, lst, q);
+      int i, j, k;
+      rm_ijk(P, c, i, j, k);
+      const int nb = c + off;
+      const int g = B.gid[c];
+      const double Tc = B.T[c];
+      const int no = s < 26 ? B.oid[nb] : 0;
+      const double Tn = s < 26 ? B.T[nb] : 0.0;
+      const double4 e = B.genv[g];
+      const int o = B.gco[g].y;
+      double r[9];
 #pragma unroll
-    for (int s = 0; s < 26; s++) no[s] = B.oid[c + P.off[s]];
-    double tn[26];
-#pragma unroll
-    for (int s = 0; s < 26; s++) tn[s] = no[s] > -1 ? 0.0 : B.T[c + P.off[s]];
-    const double vel = (Tc < P.Ts) ? vts : rm_velocity(P, Tc);
-    e.w = e.w + dt * vel;  // Grain::grow
-    B.genv[g].w = e.w;
-    double r[9];
-#pragma unroll
-    for (int x = 0; x < 9; x++) r[x] = B.l2g[9 * (size_t)o + x];
-    const int key = (i * P.nyG + j) * P.nzG + k;
-    unsigned m = 0;
-#pragma unroll
-    for (int s = 0; s < 26; s++) {
-      int di, dj, dk;
-      slot_delta(s, di, dj, dk);
-      const int nb = c + P.off[s];
-      if (no[s] > -1) continue;
-      const double Tn = tn[s];
-      if (Tn > P.Tm) continue;
-      if (!(Tn > -1.0)) continue;
-      if (rm_ghost_ijk(P, i + di, j + dj, k + dk)) continue;
-      const double gx = centre_coord(P.x0, P.h, i + di) - e.x;
-      const double gy = centre_coord(P.y0, P.h, j + dj) - e.y;
-      const double gz = centre_coord(P.z0, P.h, k + dk) - e.z;
-      if (inside_envelope(r, e.w, gx, gy, gz)) {
-        m |= 1u << s;
-        atomicMin(&B.claim[nb], key);
+      for (int x = 0; x < 9; x++) r[x] = B.l2g[9 * (size_t)o + x];
+      const double vel = (Tc < P.Ts) ? vts : rm_velocity(P, Tc);
+      const double L = e.w + dt * vel;  // Grain::grow
+      if (s == 0) B.genv[g].w = L;
+      if (s < 26 && no <= -1 && !(Tn > P.Tm) && Tn > -1.0 &&
+          !rm_ghost_ijk(P, i + di, j + dj, k + dk)) {
+        const double gx = centre_coord(P.x0, P.h, i + di) - e.x;
+        const double gy = centre_coord(P.y0, P.h, j + dj) - e.y;
+        const double gz = centre_coord(P.z0, P.h, k + dk) - e.z;
+        in = inside_envelope(r, L, gx, gy, gz);
+        if (in) atomicMin(&B.claim[nb], (i * P.nyG + j) * P.nzG + k);
       }
     }
-    B.msk[c] = m;
+    const unsigned long long m = __ballot(in);
+    if (s == 0 && q < n) B.msk[c] = (unsigned)(m >> (threadIdx.x & 32)) & kSlotBits;
   }
 }
 
@@ -1023,44 +1054,61 @@ __global__ void __launch_bounds__(kRmBlock) k_rm_resolve(RmParams P, RmBuffers B
   RmCounters* ctr = B.ctr;
   if (ctr->skip) return;
   const RmRows w = rm_rows(P, ctr);
-  const int total = w.ex * w.ey * w.ez;
-  const int stride = gridDim.x * blockDim.x;
-  for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < total; q += stride) {
-    int i, j, k;
-    rm_cell_of(w, q, i, j, k);
-    const int c = k * P.nxyG + j * P.nxG + i;
-    const unsigned char fl = B.flag[c];
-    const int g = B.gid[c];
-    unsigned m = B.msk[c];
-    if (!fl) continue;
-    if (g < 0) continue;
-    if (!m) continue;
-    const int key = (i * P.nyG + j) * P.nzG + k;
-    unsigned cap = 0;
-    int fresh = 0;
-    while (m) {
-      const int s = __builtin_ctz(m);
-      m &= m - 1;
-      const int nb = c + P.off[s];
-      if (B.claim[nb] == key) {
-        cap |= 1u << s;
-        if (B.gid[nb] < 0) fresh++;
+  RmList lst;
+  rm_list(ctr, lst);
+  const int n = lst.start[kRmParts];
+  const int s = threadIdx.x & (kRmSub - 1), half = threadIdx.x & 32;
+  int di, dj, dk;
+  slot_delta(s < 26 ? s : 0, di, dj, dk);
+  const int off = dk * P.nxyG + dj * P.nxG + di;
+  const int stride = gridDim.x * (kRmBlock / kRmSub);
+  const int first = (blockIdx.x * kRmBlock + threadIdx.x) / kRmSub;
+  for (int q = first; q - first < n; q += stride) {
+    bool hit = false, fresh = false;
+    int c = 0, i = 0, j = 0, k = 0;
+    if (q < n) {
+      c = rm_list_cell(P, B, lst, q);
+      const unsigned m = B.msk[c];
+      rm_ijk(P, c, i, j, k);
+      if ((m >> s) & 1u) {
+        const int nb = c + off;
+        hit = B.claim[nb] == (i * P.nyG + j) * P.nzG + k;
+        fresh = hit && B.gid[nb] < 0;
       }
     }
-    B.msk[c] = cap | ((unsigned)fresh << 26);
-    if (fresh) {
-      atomicAdd(&B.rowcnt[(i - w.i0) * w.ey + (j - w.j0)], fresh);
-      atomicAdd(&ctr->step_fresh, fresh);
+    const unsigned long long hm = __ballot(hit), fm = __ballot(fresh);
+    const unsigned cap = (unsigned)(hm >> half) & kSlotBits;
+    const unsigned fr = (unsigned)(fm >> half) & kSlotBits;
+    if (s == 0 && q < n) {
+      const int nf = __builtin_popcount(fr);
+      B.msk[c] = cap | ((unsigned)nf << 26);
+      if (nf) {
+        atomicAdd(&B.rowcnt[(i - w.i0) * w.ey + (j - w.j0)], nf);
+        atomicAdd(&ctr->step_fresh, nf);
+      }
     }
-    if (cap) atomicAdd(&ctr->step_cap, __builtin_popcount(cap));
+    if (hm) {
+      // the wave's captures, one reservation
+      int base = 0;
+      const int lane = threadIdx.x & 63, lead = (int)__builtin_ctzll(hm);
+      if (lane == lead) base = atomicAdd(&ctr->step_cap, (int)__popcll(hm));
+      base = __shfl(base, lead, 64);
+      if (hit) {
+        const int rank = __builtin_popcount(fr & ((1u << s) - 1u));
+        B.clist[base + (int)__popcll(hm & ((1ull << lane) - 1ull))] =
+            make_int2(c, s | (rank << 5) | (fresh ? 1 << 10 : 0));
+      }
+    }
   }
 }
 
 constexpr int kRmScan = 1024;
 
-// time advance and FE frame selection (one thread)
-__device__ void rm_finish(const RmParams& P, const RmBuffers& B) {
+// time advance and FE frame selection (one thread); n_flagged: the step's flagged
+// cells
+__device__ void rm_finish(const RmParams& P, const RmBuffers& B, int n_flagged) {
   RmCounters* ctr = B.ctr;
+  for (int p = 0; p < kRmParts; p++) ctr->n_flag[p] = 0;
   const double t0 = ctr->t;
   const double dt = ctr->dt;
   ctr->t = t0 + dt;
@@ -1074,8 +1122,7 @@ __device__ void rm_finish(const RmParams& P, const RmBuffers& B) {
     row.n_nucleated = ctr->step_nuc;
     row.n_captured = ctr->step_cap;
     row.n_fresh = ctr->step_fresh;
-    row.n_flagged = 0;
-    for (int q = 0; q < 64; q++) row.n_flagged += ctr->flagged_parts[q];
+    row.n_flagged = n_flagged;
     row.n_fallback = 0;
     if (B.fb_slots)
       for (int q = 0; q < 256; q++) row.n_fallback += B.fb_slots[q];
@@ -1088,10 +1135,6 @@ __device__ void rm_finish(const RmParams& P, const RmBuffers& B) {
   if (B.fb_slots)
     for (int q = 0; q < 256; q++) B.fb_slots[q] = 0;
   ctr->armed[st & 1] = 0;
-  for (int q = 0; q < 64; q++) {
-    ctr->flagged_parts[q] = 0;
-    ctr->min_t_keys[q] = ~0ull;
-  }
   ctr->n_fallback = 0;
   // this step's box inputs are spent; the slot serves step + 2
   for (int q = 0; q < 3; q++) {
@@ -1159,6 +1202,7 @@ __global__ void __launch_bounds__(kRmScan) k_rm_rowscan(RmParams P, RmBuffers B)
     for (int r = lo; r < hi; r++) {
       B.rowoff[r] = (int)off;
       off += (unsigned long long)B.rowcnt[r];
+      B.rowcnt[r] = 0;  // the next step's counts start from zero
     }
     __syncthreads();
     if (threadIdx.x == 0) ctr->n_grains += (int)tot;
@@ -1183,70 +1227,62 @@ __global__ void __launch_bounds__(kRmScan) k_rm_rowscan(RmParams P, RmBuffers B)
       }
     }
   }
-  if (threadIdx.x == 0) rm_finish(P, B);
+  if (threadIdx.x < 64) {
+    const int flagged = (int)wave_sum((unsigned long long)ctr->flagged_parts[threadIdx.x]);
+    ctr->flagged_parts[threadIdx.x] = 0;
+    ctr->min_t_keys[threadIdx.x] = ~0ull;
+    if (threadIdx.x == 0) rm_finish(P, B, flagged);
+  }
 }
 
+// One child per thread, from the list of captures.
 __global__ void __launch_bounds__(kRmBlock) k_rm_emit(RmParams P, RmBuffers B) {
   RmCounters* ctr = B.ctr;
-  if (ctr->skip || ctr->step_cap == 0) return;
+  const int n = ctr->step_cap;
+  if (ctr->skip || n == 0) return;
   const long long st = ctr->step - 1;  // k_rm_rowscan has advanced the step
-  const RmRows w = rm_rows_of(P, ctr->box[st & 1]);
-  const int total = w.ex * w.ey * w.ez;
   RmBox cap_box;
   box_empty(cap_box);
   const int stride = gridDim.x * blockDim.x;
-  for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < total; q += stride) {
-    int i, j, k;
-    rm_cell_of(w, q, i, j, k);
-    const int c = k * P.nxyG + j * P.nxG + i;
-    const unsigned char fl = B.flag[c];
+  for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < n; q += stride) {
+    const int2 it = B.clist[q];
+    const int c = it.x, s = it.y & 31;
+    int i, j, k, di, dj, dk;
+    rm_ijk(P, c, i, j, k);
+    slot_delta(s, di, dj, dk);
+    const int nb = c + dk * P.nxyG + dj * P.nxG + di;
     const int g = B.gid[c];
-    const unsigned mk = B.msk[c];
-    if (!fl) continue;
-    if (g < 0) continue;
-    unsigned cap = mk & kSlotBits;
-    if (!cap) continue;
-    // first new id of this cell: the row's first id plus the fresh captures
-    // of the row's flagged cells below it (cells of the row are never
-    // captured in this step, so their flags, ids and masks are settled)
-    int next = 0;
-    if (mk >> 26) {
-      next = B.rowoff[(i - w.i0) * w.ey + (j - w.j0)];
-      for (int kk = w.k0; kk < k; kk++) {
-        const int cc = kk * P.nxyG + j * P.nxG + i;
-        if (B.flag[cc] && B.gid[cc] >= 0) next += (int)(B.msk[cc] >> 26);
-      }
-    }
+    int id = B.gid[nb];
     const double4 e = B.genv[g];
     const int o = B.gco[g].y;
     double r[9];
 #pragma unroll
     for (int x = 0; x < 9; x++) r[x] = B.l2g[9 * (size_t)o + x];
-    while (cap) {
-      const int s = __builtin_ctz(cap);
-      cap &= cap - 1;
-      int di, dj, dk;
-      slot_delta(s, di, dj, dk);
-      const int nb = c + P.off[s];
-      const double gx = centre_coord(P.x0, P.h, i + di) - e.x;
-      const double gy = centre_coord(P.y0, P.h, j + dj) - e.y;
-      const double gz = centre_coord(P.z0, P.h, k + dk) - e.z;
-      double out[4];
-      child_envelope(r, e.w, P.h, P.trunc, P.sqrt2f, gx, gy, gz, out);
-      const double4 ce = make_double4(out[0] + e.x, out[1] + e.y, out[2] + e.z, out[3]);
-      int id = B.gid[nb];
-      if (id < 0) {
-        id = next++;
-        B.gid[nb] = id;
-        B.gco[id] = make_int2(nb, o);
-      } else {
-        B.gco[id].y = o;
+    const double gx = centre_coord(P.x0, P.h, i + di) - e.x;
+    const double gy = centre_coord(P.y0, P.h, j + dj) - e.y;
+    const double gz = centre_coord(P.z0, P.h, k + dk) - e.z;
+    double out[4];
+    child_envelope(r, e.w, P.h, P.trunc, P.sqrt2f, gx, gy, gz, out);
+    const double4 ce = make_double4(out[0] + e.x, out[1] + e.y, out[2] + e.z, out[3]);
+    if (it.y >> 10) {
+      // a new id: the row's first one, plus the fresh captures of the row's
+      // flagged cells below (cells of the row are never captured in this step, so
+      // their flags, ids and masks are settled), plus those of this cell's lower slots
+      const RmRows w = rm_rows_of(P, ctr->box[st & 1]);
+      id = B.rowoff[(i - w.i0) * w.ey + (j - w.j0)] + ((it.y >> 5) & 31);
+      for (int kk = w.k0; kk < k; kk++) {
+        const int cc = kk * P.nxyG + j * P.nxG + i;
+        if (B.flag[cc] && B.gid[cc] >= 0) id += (int)(B.msk[cc] >> 26);
       }
-      B.genv[id] = ce;
-      B.oid[nb] = o;
-      B.claim[nb] = INT_MAX;
-      box_add(cap_box, i + di, j + dj, k + dk);
+      B.gid[nb] = id;
+      B.gco[id] = make_int2(nb, o);
+    } else {
+      B.gco[id].y = o;
     }
+    B.genv[id] = ce;
+    B.oid[nb] = o;
+    B.claim[nb] = INT_MAX;
+    box_add(cap_box, i + di, j + dj, k + dk);
   }
   block_box_merge(cap_box, &ctr->acc[(st + 1) & 1][2]);
 }
@@ -1279,9 +1315,10 @@ const char* const kRmKernelNames[kRmKernels] = {
 hipError_t rm_launch_kernel(int q, const RmParams& P, const RmBuffers& B, int site_blocks,
                             hipStream_t s) {
   const unsigned cells = (unsigned)rm_cell_blocks(P);
-  // the kernels that work only on flagged cells (a small part of the box):
-  // with the box, two blocks per CU (their waves hold many registers)
+  // the minimum over the box: two blocks per CU with the box
   const unsigned sparse = P.window && cells > 512u ? 512u : cells;
+  // the list kernels: 8192 flagged cells, 32 K captures per round of the grid
+  const unsigned lists = cells < 1024u ? cells : 1024u, kids = cells < 128u ? cells : 128u;
   long long nbk = (P.nodes + kRmBlock - 1) / kRmBlock;
   if (nbk > 8192) nbk = 8192;
   if (nbk < 1) nbk = 1;
@@ -1308,10 +1345,10 @@ hipError_t rm_launch_kernel(int q, const RmParams& P, const RmBuffers& B, int si
       hipLaunchKernelGGL(k_rm_nucleate_mint, dim3(sparse + (unsigned)site_blocks), dim3(kRmBlock), 0,
                          s, P, B, site_blocks);
       break;
-    case 6: hipLaunchKernelGGL(k_rm_claim, dim3(sparse), dim3(kRmBlock), 0, s, P, B); break;
-    case 7: hipLaunchKernelGGL(k_rm_resolve, dim3(cells), dim3(kRmBlock), 0, s, P, B); break;
+    case 6: hipLaunchKernelGGL(k_rm_claim, dim3(lists), dim3(kRmBlock), 0, s, P, B); break;
+    case 7: hipLaunchKernelGGL(k_rm_resolve, dim3(lists), dim3(kRmBlock), 0, s, P, B); break;
     case 8: hipLaunchKernelGGL(k_rm_rowscan, dim3(1), dim3(kRmScan), 0, s, P, B); break;
-    case 9: hipLaunchKernelGGL(k_rm_emit, dim3(sparse), dim3(kRmBlock), 0, s, P, B); break;
+    case 9: hipLaunchKernelGGL(k_rm_emit, dim3(kids), dim3(kRmBlock), 0, s, P, B); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
