@@ -386,18 +386,21 @@ amca_status amca_domain_create(const amca_domain_desc* desc, int32_t orient_capa
   d->ids_blocks = (int)std::max(1LL, std::min<long long>((P.N + 32767) / 32768,
                                                          std::min(8LL * cus, (long long)amca::kMaxIdsBlocks)));
   P.ids_blocks = d->ids_blocks;
-  // compaction and retirement: the 64-brick pieces of the grid over at most eight
-  // blocks per CU
-  d->cmp_blocks = (int)std::max(1LL, std::min<long long>((nB + 63) / 64,
-                                                         std::min(8LL * cus, (long long)amca::kMaxBlocks)));
-  P.cmp_blocks = d->cmp_blocks;
   // The short step (see plain_step.hip) for grids of up to kFusedCells whose grains
   // grow at most a quarter of a cell per step (dt <= time_step_factor h / v), which
   // keeps captures by wave 1's fresh envelopes rare: k_tail takes those with one
   // work-group.  Whole runs, short against long form: 131x97x67 46 against 68 us a
-  // step, 256^3 114 against 135; at 512^3 k_tail's one work-group takes 730 us
+  // step, 256^3 98 against 135; at 512^3 k_tail's one work-group takes 730 us
   // of 1050 (long form 347).
   P.fused = P.N <= kFusedCells && desc->time_step_factor <= 0.25 ? 1 : 0;
+  // compaction and retirement: the 64-brick pieces of the grid over at most eight
+  // blocks per CU; two for the short step, whose wave-0 kernels all have these blocks
+  // and each of them starts up for a few dozen entries (256^3: 113, 101 and 98 us a
+  // step at 8, 4 and 2 per CU; 512^3 long form: 347, 346, 381)
+  d->cmp_blocks = (int)std::max(1LL, std::min<long long>((nB + 63) / 64,
+                                                         std::min((P.fused ? 2LL : 8LL) * cus,
+                                                                  (long long)amca::kMaxBlocks)));
+  P.cmp_blocks = d->cmp_blocks;
   if (amca::env_int("AMCA_DOMAIN_GRAPH_STEPS", 0, 1024, &d->graph_steps) < 0) {
     delete d;
     return fail(AMCA_ERR_INVALID, "AMCA_DOMAIN_GRAPH_STEPS must be an integer in [0, 1024]");
@@ -721,6 +724,7 @@ amca_status amca_envelope_selftest(int32_t n, const double* env4, const double* 
 
 struct amca_batch {
   std::vector<amca_domain*> doms;
+  std::vector<amca::DevParams> P;  // the domains' parameters with the batch's step form and grids
   int device = 0;
   hipStream_t stream = nullptr;
   amca::DevParams* dP = nullptr;
@@ -769,9 +773,13 @@ namespace {
 // `list_blocks` blocks (and emit_blocks for resolve/emit) shared in proportion
 // to the domains' cell counts, at least `min_blocks` each, capped by what a
 // domain can use (one block per 256 cells of its grid, kMaxBlocks for the
-// scanned kernels).
+// scanned kernels).  The short step's blocks hold bricks, asleep or not, and start
+// up for a fraction of a tile each: it takes a quarter of the budgets (16 uneven
+// domains, ms for the run at budgets of 2, 4, 8, 16 and 32 blocks per CU: 86, 71, 73,
+// 89, 119).
 void batch_geometry(const amca_batch* b, std::vector<int>& nl, std::vector<int>& ne) {
   const size_t n = b->doms.size();
+  const double part = b->L.fused ? 0.25 : 1.0;
   double total = 0.0;
   for (size_t i = 0; i < n; i++)
     if (b->active[i]) total += (double)b->doms[i]->P.N;
@@ -781,8 +789,8 @@ void batch_geometry(const amca_batch* b, std::vector<int>& nl, std::vector<int>&
     if (!b->active[i]) continue;
     const double share = (double)b->doms[i]->P.N / total;
     const long long cap = std::max(1LL, (b->doms[i]->P.N + amca::kBlock - 1) / amca::kBlock);
-    long long l = (long long)std::llround(share * b->sched.list_blocks);
-    long long e = (long long)std::llround(share * b->sched.emit_blocks);
+    long long l = (long long)std::llround(share * part * b->sched.list_blocks);
+    long long e = (long long)std::llround(share * part * b->sched.emit_blocks);
     l = std::max<long long>(b->sched.min_blocks, std::min(l, cap));
     // resolve / emit blocks keep per-block stats in kMaxBlocks slots
     e = std::min(std::max<long long>(b->sched.min_blocks, std::min(e, cap)), (long long)amca::kMaxBlocks);
@@ -821,7 +829,13 @@ amca_status batch_apply_schedule(amca_batch* b) {
     // a finished domain gets no blocks (its kernels would return at once)
     nn[i] = b->active[i] ? b->doms[i]->nuc_blocks : 0;
     ni[i] = b->active[i] ? b->doms[i]->ids_blocks : 0;
-    nc[i] = b->active[i] ? b->doms[i]->cmp_blocks : 0;
+    // bricks over blocks as the resolve / emit budget has it, whole 64-brick pieces
+    const amca::DevParams& P = b->doms[i]->P;
+    const long long pieces = ((long long)P.nbX * P.nbY * P.nbZ + 63) / 64;
+    nc[i] = b->active[i] ? (int)std::max(1LL, std::min<long long>({(long long)ne[i], pieces,
+                                                                   (long long)amca::kMaxBlocks}))
+                         : 0;
+    b->P[i].cmp_blocks = std::max(1, nc[i]);
     one[i] = b->active[i] ? 1 : 0;
   }
   std::vector<int> order(n);
@@ -850,6 +864,7 @@ amca_status batch_apply_schedule(amca_batch* b) {
   all.insert(all.end(), mi.begin(), mi.end());
   all.insert(all.end(), mc.begin(), mc.end());
   HIP_TRY(hipMemcpy(b->maps, all.data(), sizeof(int4) * total, hipMemcpyHostToDevice));
+  HIP_TRY(hipMemcpy(b->dP, b->P.data(), sizeof(amca::DevParams) * n, hipMemcpyHostToDevice));
   b->L.map_nuc = b->maps;
   b->L.map_list = b->maps + mn.size();
   b->L.map_emit = b->L.map_list + ml.size();
@@ -1017,7 +1032,8 @@ amca_status amca_batch_create(amca_domain* const* doms, int32_t n, amca_batch** 
       st = fail(AMCA_ERR_HIP, "stream creation failed");
       break;
     }
-    std::vector<amca::DevParams> P(n);
+    std::vector<amca::DevParams>& P = b->P;
+    P.resize(n);
     std::vector<amca::DevBuffers> B(n);
     for (int i = 0; i < n; i++) {
       // every domain's own queued work must be done before the batch stream takes over
@@ -1038,8 +1054,7 @@ amca_status amca_batch_create(amca_domain* const* doms, int32_t n, amca_batch** 
       st = fail(AMCA_ERR_HIP, "batch allocation failed");
       break;
     }
-    if (hipMemcpy(b->dP, P.data(), sizeof(amca::DevParams) * n, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(b->dB, B.data(), sizeof(amca::DevBuffers) * n, hipMemcpyHostToDevice) != hipSuccess) {
+    if (hipMemcpy(b->dB, B.data(), sizeof(amca::DevBuffers) * n, hipMemcpyHostToDevice) != hipSuccess) {
       st = fail(AMCA_ERR_HIP, "batch upload failed");
       break;
     }
