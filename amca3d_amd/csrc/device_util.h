@@ -177,7 +177,16 @@ __device__ __forceinline__ unsigned brick_bits26(const DevParams& P, const unsig
     return kCoherent ? ld_coherent(p) : *p;
   });
 }
-// The neighbours that are liquid and claimed (both words of a brick in one load).
+// The neighbours that are liquid and not claimed (both words of a brick in one load).
+__device__ __forceinline__ unsigned open_bits26(const DevParams& P, const DevBuffers& B, int i,
+                                                int j, int k) {
+  const ulonglong2* m = reinterpret_cast<const ulonglong2*>(B.bmap);
+  return block_bits26(P, i, j, k, [&](int b) {
+    const ulonglong2 u = m[b];
+    return u.x & ~u.y;
+  });
+}
+// The neighbours that are liquid and claimed.
 __device__ __forceinline__ unsigned taken_bits26(const DevParams& P, const DevBuffers& B, int i,
                                                  int j, int k) {
   const ulonglong2* m = reinterpret_cast<const ulonglong2*>(B.bmap);

@@ -3,7 +3,7 @@
 // The reference keeps the grid as raw host arrays owned by
 // CellularAutomataManager (CellularAutomataManager.cpp:303-326) and one heap
 // Grain per solid cell.  Here the grid and the per-cell envelopes live in HBM
-// for the lifetime of the handle, a step is a fixed sequence of seven or twelve
+// for the lifetime of the handle, a step is a fixed sequence of six or twelve
 // kernel launches that reads every scalar it needs from device memory, and the host
 // only reads the counters back between batches of steps.
 #include <hip/hip_runtime.h>
@@ -184,7 +184,6 @@ amca_status enqueue_step(amca_domain* d) {
     AMCA_TRY(timed(d, K_RESOLVE, [&] { return amca::launch_resolve(P, B, 0, P.cmp_blocks, s); }));
     AMCA_TRY(timed(d, K_IDSCAN, [&] { return amca::launch_idscan(P, B, 0, P.cmp_blocks, s); }));
     AMCA_TRY(timed(d, K_EMIT, [&] { return amca::launch_emit(P, B, 0, P.cmp_blocks, s); }));
-    AMCA_TRY(timed(d, K_CLAIM, [&] { return amca::launch_claim(P, B, 1, d->list_blocks, s); }));
     AMCA_TRY(timed(d, K_TAIL, [&] { return amca::launch_tail(P, B, s); }));
     return AMCA_OK;
   }
@@ -346,6 +345,7 @@ amca_status amca_domain_create(const amca_domain_desc* desc, int32_t orient_capa
   want_buf(&B.rec, 64 * (size_t)nB);
   want_buf(&B.wake, 64 * (size_t)nB);
   want_buf(&B.inc, amca::kRing);
+  want_buf(&B.cl1, (size_t)nB);
   want_buf(&B.awk, (size_t)nB);
   want_buf(&B.genv, N);
   want_buf(&B.gco, N);
@@ -404,8 +404,8 @@ amca_status amca_domain_create(const amca_domain_desc* desc, int32_t orient_capa
   // The short step (see plain_step.hip) for grids of up to kFusedCells whose grains
   // grow at most a quarter of a cell per step (dt <= time_step_factor h / v), which
   // keeps captures by wave 1's fresh envelopes rare: k_tail takes those with one
-  // work-group.  Whole runs, short against long form: 131x97x67 46 against 68 us a
-  // step, 256^3 98 against 135; at 512^3 k_tail's one work-group takes 730 us
+  // work-group.  Short against long form when the line was drawn (wave 1's tests had
+  // a launch of their own in both): 131x97x67 46 against 68 us a step, 256^3 98 against 135; at 512^3 k_tail's one work-group takes 730 us
   // of 1050 (long form 347).
   P.fused = P.N <= kFusedCells && desc->time_step_factor <= 0.25 ? 1 : 0;
   // compaction and retirement: the 64-brick pieces of the grid over at most eight

@@ -31,7 +31,7 @@ struct DevParams {
   int ids_blocks;         // blocks of the id scan (k_idscan)
   int cmp_blocks;         // blocks of k_count / k_compact, and of the retirement in k_resolve
   int fused;              // the short step: k_wake_claim instead of k_count, k_compact and wave 0's
-                          // k_claim, wave 1's captures in k_tail
+                          // k_claim, no other kernels for wave 1, its captures in k_tail
 };
 
 // Mutable scalars that live on the device, so that a whole step (or many
@@ -124,6 +124,7 @@ struct DevBuffers {
   unsigned short* wake;   // growth clock (kWakeUnits per cell, rounded down) from which the
                           // active grain in the slot may capture a cell [64 nB]
   double* inc;            // growth increments of the last kRing steps, by step [kRing]
+  unsigned long long* cl1;  // brick words: cells claimed in wave 1 [nB]
   unsigned long long* awk;  // brick words: active grains awake in the running step [nB]
   double4* genv;          // envelope by grain id, materialized for downloads [N]
   int2* gco;              // grain -> (cell, orientation), materialized for downloads [N]
@@ -179,7 +180,8 @@ hipError_t launch_init_grid(const DevParams& P, const DevBuffers& B, hipStream_t
 hipError_t launch_nucleate(const DevParams& P, const DevBuffers& B, int blocks, hipStream_t s);
 hipError_t launch_claim(const DevParams& P, const DevBuffers& B, int wave, int blocks,
                         hipStream_t s);
-// Waves 0 and 1: k_claim, k_resolve, k_idscan and k_emit in that order;
+// Waves 0 and 1: k_claim, k_resolve, k_idscan and k_emit in that order (k_emit of
+// wave 0 makes wave 1's claims);
 // k_resolve and k_emit with the same `blocks` (<= kMaxBlocks list chunks)
 hipError_t launch_resolve(const DevParams& P, const DevBuffers& B, int wave, int blocks,
                           hipStream_t s);

@@ -15,7 +15,7 @@
 //   k_count/k_compact: wave 0's list, the awake slots in brick order: the active
 //                     grains that have grown enough to capture a cell (the
 //                     others sleep, see DevBuffers);
-//   k_claim         : per wave entry, liquid test of the 26 neighbours on the
+//   k_claim         : per wave-0 entry, liquid test of the 26 neighbours on the
 //                     1-bit liquid map, envelope tests, and an atomicMin of the
 //                     grain id into each enclosed neighbour's claim word;
 //   k_resolve       : per entry, captured decisions from the claims; capturing
@@ -23,9 +23,11 @@
 //                     a second set of blocks retires the active grains, awake or
 //                     not, that have no liquid neighbour left;
 //   k_idscan        : first child of each capturing grain, a scan over ids;
-//   k_emit          : the child records and the next wave's list;
+//   k_emit          : the child records and the next wave's list; in wave 0 also
+//                     the children's own tests and claims, which are wave 1's;
 //   k_tail          : waves >= 2 (rare) in one work-group, then the time advance.
-// Waves 0 and 1 each run k_claim, k_resolve, k_idscan and k_emit.
+// Waves 0 and 1 each run k_claim, k_resolve, k_idscan and k_emit (wave 1's k_claim
+// only clears the id scan's totals).
 // On small grids a step is bound by its launches (about 4.5 us each, whatever
 // they do), and two shorter forms hold: k_wake_claim makes wave 0's list and tests
 // it in one launch, and k_tail also takes wave 1's captures, which are rare.
@@ -90,6 +92,7 @@ __global__ void k_init_grid(DevParams P, DevBuffers B) {
     B.bmap[2 * b] = bits;
     B.bmap[2 * b + 1] = 0ull;
     B.amap[b] = 0ull;
+    B.cl1[b] = 0ull;
   }
 }
 
@@ -308,7 +311,8 @@ __device__ __forceinline__ unsigned short wake_clock(const DevParams& P, double 
 
 // Envelope tests of grain g (orientation o, envelope e) at cell (ci, cj, ck)
 // against its liquid neighbours lm: each neighbour inside the envelope gets an
-// atomicMin of g into its claim word and its claimed bit.  Returns the inside
+// atomicMin of g into its claim word and its claimed bit (kOwn: wave 1's map, else
+// the brick map's).  Returns the inside
 // bits (none when L == 0: such an envelope captures nothing); dmin is the
 // distance of the nearest liquid neighbour outside (infinity: there is none).
 //
@@ -318,6 +322,7 @@ __device__ __forceinline__ unsigned short wake_clock(const DevParams& P, double 
 // entries, so the 27 products are formed once; a neighbour's local
 // coordinates are then sums of three of them, added in to_local's order
 // (its leading 0.0 + p is p up to the sign of a zero, which fabs drops).
+template <bool kOwn>
 __device__ __forceinline__ unsigned claim_tests(const DevParams& P, const DevBuffers& B, int g,
                                                 int o, int ci, int cj, int ck, unsigned lm,
                                                 const double4& e, WordStage* st, double& dmin) {
@@ -380,9 +385,12 @@ __device__ __forceinline__ unsigned claim_tests(const DevParams& P, const DevBuf
     int di, dj, dk;
     slot_delta(s, di, dj, dk);
     atomicMin(&B.claim[claim_index(P, ci + di, cj + dj, ck + dk)], g);
-    const int wd = brick_word(P, ci + di, cj + dj, ck + dk) + 1;
+    const int wd = brick_word(P, ci + di, cj + dj, ck + dk);
     const unsigned long long bt = brick_bit(ci + di, cj + dj, ck + dk);
-    if (!st || !stage_add(*st, wd, bt)) atomicOr(&B.bmap[wd], bt);
+    if (kOwn)
+      atomicOr(&B.cl1[wd >> 1], bt);
+    else if (!st || !stage_add(*st, wd + 1, bt))
+      atomicOr(&B.bmap[wd + 1], bt);
   }
   return im;
 }
@@ -610,115 +618,89 @@ __device__ __forceinline__ IdRange id_range(const DevParams& P, const DevCounter
   return r;
 }
 
-// Envelope tests of one entry of a wave >= 1 (the grain in slot q).  Its own
+// Envelope tests of one entry of a wave >= 2 (the grain in slot q).  Its own
 // cell's claimed bit (set by the wave that captured it) stays set: the
 // claimed word is read only where the liquid word has the cell's bit, and a
 // captured cell is never liquid again.
-template <bool kCoherent>
 __device__ __forceinline__ unsigned long long claim_entry(const DevParams& P, const DevBuffers& B,
-                                                          int q, WordStage* st) {
+                                                          int q) {
   int ci, cj, ck;
   slot_ijk(P, q, ci, cj, ck);
   const SlotRec r = B.rec[q];
-  const unsigned lm = brick_bits26<0, kCoherent>(P, B.bmap, ci, cj, ck);
+  const unsigned lm = brick_bits26<0, true>(P, B.bmap, ci, cj, ck);
   double dmin;
-  const unsigned im =
-      claim_tests(P, B, r.id, r.o, ci, cj, ck, lm, make_double4(r.x, r.y, r.z, r.L), st, dmin);
+  const unsigned im = claim_tests<false>(P, B, r.id, r.o, ci, cj, ck, lm,
+                                         make_double4(r.x, r.y, r.z, r.L), nullptr, dmin);
   B.wake[q] = wake_clock(P, B.ctr->S, r.L, dmin);
   return ((unsigned long long)im << 32) | lm;
 }
 
-// The tests of list entries [lo, hi) by one block.
-__device__ __forceinline__ void claim_range(const DevParams& P, const DevBuffers& B, int wave,
-                                            int blk, const int* __restrict__ list, int lo, int hi) {
+// The tests of wave 0's list entries [lo, hi) by one block.
+__device__ __forceinline__ void claim_range(const DevParams& P, const DevBuffers& B, int blk,
+                                            const int* __restrict__ list, int lo, int hi) {
   const DevCounters* ctr = B.ctr;
   if (lo >= hi) return;
   // the claimed bits, staged per work-group
   __shared__ WordStage s_st;
   stage_init(s_st);
   __syncthreads();
-  if (wave == 0) {
-    const double S = ctr->S;
-    const bool force = ctr->force != 0;
-    const int end = (int)ctr->step + 1;
-    int id_lo = INT_MAX, id_hi = -1;  // this block's claiming grains
-    for (int t = lo + threadIdx.x; t < hi; t += kBlock) {
-      const long long q = list[t];
-      int i, j, k;
-      slot_ijk(P, q, i, j, k);
-      const SlotRec r = B.rec[q];
-      const double L = grow_to(B, r.L, r.stamp, end);
-      if (force) {
-        B.rec[q].L = L;
-        B.rec[q].stamp = end;
-      }
-      const unsigned lm = brick_bits26<0, false>(P, B.bmap, i, j, k);
-      double dmin;
-      const unsigned im =
-          claim_tests(P, B, r.id, r.o, i, j, k, lm, make_double4(r.x, r.y, r.z, L), &s_st, dmin);
-      B.wake[q] = wake_clock(P, S, L, dmin);
-      B.masks[t] = ((unsigned long long)im << 32) | (unsigned)r.id;
-      if (im) {
-        id_lo = min(id_lo, r.id);
-        id_hi = max(id_hi, r.id);
-      }
+  const double S = ctr->S;
+  const bool force = ctr->force != 0;
+  const int end = (int)ctr->step + 1;
+  int id_lo = INT_MAX, id_hi = -1;  // this block's claiming grains
+  for (int t = lo + threadIdx.x; t < hi; t += kBlock) {
+    const long long q = list[t];
+    int i, j, k;
+    slot_ijk(P, q, i, j, k);
+    const SlotRec r = B.rec[q];
+    const double L = grow_to(B, r.L, r.stamp, end);
+    if (force) {
+      B.rec[q].L = L;
+      B.rec[q].stamp = end;
     }
-    // the block's claimer id range into one of the 64 slots
-    __shared__ int s_lo, s_hi;
+    const unsigned lm = brick_bits26<0, false>(P, B.bmap, i, j, k);
+    double dmin;
+    const unsigned im = claim_tests<false>(P, B, r.id, r.o, i, j, k, lm,
+                                           make_double4(r.x, r.y, r.z, L), &s_st, dmin);
+    B.wake[q] = wake_clock(P, S, L, dmin);
+    B.masks[t] = ((unsigned long long)im << 32) | (unsigned)r.id;
+    if (im) {
+      id_lo = min(id_lo, r.id);
+      id_hi = max(id_hi, r.id);
+    }
+  }
+  // the block's claimer id range into one of the 64 slots
+  __shared__ int s_lo, s_hi;
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      id_lo = min(id_lo, __shfl_xor(id_lo, o, 64));
-      id_hi = max(id_hi, __shfl_xor(id_hi, o, 64));
-    }
-    if (threadIdx.x == 0) {
-      s_lo = INT_MAX;
-      s_hi = -1;
-    }
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0 && id_hi >= 0) {
-      atomicMin(&s_lo, id_lo);
-      atomicMax(&s_hi, id_hi);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0 && s_hi >= 0) {
-      atomicMin(&B.ctr->claim_lo[blk & 63], s_lo);
-      atomicMax(&B.ctr->claim_hi[blk & 63], s_hi);
-    }
-  } else {
-    // A grain without a liquid neighbour leaves the active map here.  Whether one
-    // with liquid neighbours stays is k_resolve's to say only if a grain of the
-    // wave claimed a cell: without claims all of them stay.
-    int ret = 0;
-    unsigned any = 0;
-    for (int t = lo + threadIdx.x; t < hi; t += kBlock) {
-      const int q = list[t];
-      const unsigned long long m = claim_entry<false>(P, B, q, &s_st);
-      B.masks[t] = m;
-      if ((unsigned)m == 0u) {
-        atomicAnd(&B.amap[q >> 6], ~(1ull << (q & 63)));
-        ret++;
-      }
-      any |= (unsigned)(m >> 32);
-    }
-    __shared__ int s_ret;
-    if (threadIdx.x == 0) s_ret = 0;
-    __syncthreads();
-    if (ret) atomicAdd(&s_ret, ret);
-    if (any) B.ctr->w1_claims = 1;
-    __syncthreads();
-    if (threadIdx.x == 0 && s_ret) atomicAdd(&B.ctr->w1_ret[blk & 63], s_ret);
+  for (int o = 32; o > 0; o >>= 1) {
+    id_lo = min(id_lo, __shfl_xor(id_lo, o, 64));
+    id_hi = max(id_hi, __shfl_xor(id_hi, o, 64));
+  }
+  if (threadIdx.x == 0) {
+    s_lo = INT_MAX;
+    s_hi = -1;
+  }
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0 && id_hi >= 0) {
+    atomicMin(&s_lo, id_lo);
+    atomicMax(&s_hi, id_hi);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0 && s_hi >= 0) {
+    atomicMin(&B.ctr->claim_lo[blk & 63], s_lo);
+    atomicMax(&B.ctr->claim_hi[blk & 63], s_hi);
   }
   __syncthreads();
   stage_flush_or(s_st, B.bmap);
 }
 
-// A list wave's envelope tests, one entry per thread: bound by the lines of the
+// Wave 0's envelope tests, one entry per thread: bound by the lines of the
 // awake grains' records, about 340 bytes an entry at 512^3 (88 us a step for 1.1 M
 // awake grains of 5.0 M active; all 5.0 M, packed closer, took 145).  Wave 0 first brings each
 // awake grain's L up to the running step (Grain::grow, Grain.h:27, over the whole
-// list as in :521-538: the sleeping grains' turns come when they wake); wave 1's
-// grains were created in this step and do not grow.  Both leave the clock at
-// which the grain wakes next.
+// list as in :521-538: the sleeping grains' turns come when they wake) and leaves the
+// clock at which the grain wakes next.  Wave 1's tests are made by wave 0's k_emit,
+// which has its grains in registers; its k_claim only clears the id scan's totals.
 // Neighbouring entries sit in the same bricks, so their map words and
 // records share cache lines.
 __device__ __forceinline__ void claim_body(const DevParams& P, const DevBuffers& B, int wave,
@@ -727,10 +709,11 @@ __device__ __forceinline__ void claim_body(const DevParams& P, const DevBuffers&
   if (ctr->skip) return;
   // the id scan's per-block capture totals start from zero (k_resolve adds)
   for (int q = blk * kBlock + threadIdx.x; q < P.ids_blocks; q += nblk * kBlock) B.idtot[q] = 0u;
+  if (wave == 1) return;
   const int* list;
   int lo, hi;
-  wave_chunk(P, B, wave, blk, nblk, list, lo, hi);
-  claim_range(P, B, wave, blk, list, lo, hi);
+  wave_chunk(P, B, 0, blk, nblk, list, lo, hi);
+  claim_range(P, B, blk, list, lo, hi);
 }
 
 // The short step's wave 0 up to the claims in one launch: each block lists the
@@ -760,7 +743,7 @@ __device__ __forceinline__ void wake_claim_body(const DevParams& P, const DevBuf
   }
   if (threadIdx.x == 0) B.cmptot[blk] = (unsigned)(hi - lo);
   __syncthreads();  // the block's list is complete
-  claim_range(P, B, 0, blk, B.alist, lo, hi);
+  claim_range(P, B, blk, B.alist, lo, hi);
 }
 
 // claim_index of neighbour (di, dj, dk) = cx[di + 1] + cy[dj + 1] + cz[dk + 1].
@@ -820,9 +803,16 @@ __device__ __forceinline__ unsigned resolve_bits(const DevParams& P, const DevBu
   return cap | (keep << 31);
 }
 
-// One entry of a wave >= 1 (slot q); a grain that does not stay active leaves
-// the active map.
-template <bool kCoherent>
+// Neighbours of cell (i, j, k) claimed in wave 1.
+__device__ __forceinline__ unsigned claimed1_bits26(const DevParams& P, const DevBuffers& B, int i,
+                                                    int j, int k) {
+  return block_bits26(P, i, j, k, [&](int b) { return B.cl1[b]; });
+}
+
+// One entry of wave 1 or (kDeep) a wave >= 2 in slot q; a grain that does not stay
+// active leaves the active map (wave 1's without a liquid neighbour never entered
+// it).
+template <bool kDeep>
 __device__ __forceinline__ unsigned resolve_entry(const DevParams& P, const DevBuffers& B, int q,
                                                   unsigned long long m) {
   unsigned r = 0u;
@@ -830,10 +820,11 @@ __device__ __forceinline__ unsigned resolve_entry(const DevParams& P, const DevB
     int ci, cj, ck;
     slot_ijk(P, q, ci, cj, ck);
     int g;
-    r = resolve_bits<kCoherent>(P, B, q, m, brick_bits26<1, kCoherent>(P, B.bmap, ci, cj, ck), ci,
-                                cj, ck, g);
+    const unsigned cm = kDeep ? brick_bits26<1, true>(P, B.bmap, ci, cj, ck)
+                              : claimed1_bits26(P, B, ci, cj, ck);
+    r = resolve_bits<kDeep>(P, B, q, m, cm, ci, cj, ck, g);
   }
-  if (!(r >> 31)) atomicAnd(&B.amap[q >> 6], ~(1ull << (q & 63)));
+  if (!(r >> 31) && (kDeep || (unsigned)m != 0u)) atomicAnd(&B.amap[q >> 6], ~(1ull << (q & 63)));
   return r;
 }
 
@@ -1041,9 +1032,9 @@ __device__ __forceinline__ void resolve_body(const DevParams& P, const DevBuffer
       } else {
         if ((unsigned)m != 0u) {
           slot_ijk(P, q, i, j, k);
-          r = resolve_bits<false>(P, B, q, m, brick_bits26<1, false>(P, B.bmap, i, j, k), i, j, k, g);
+          r = resolve_bits<false>(P, B, q, m, claimed1_bits26(P, B, i, j, k), i, j, k, g);
+          if (!(r >> 31)) atomicAnd(&B.amap[q >> 6], ~(1ull << (q & 63)));
         }
-        if (!(r >> 31)) atomicAnd(&B.amap[q >> 6], ~(1ull << (q & 63)));
       }
     }
     const unsigned long long keepm = __ballot(t < hi && (r >> 31));
@@ -1190,10 +1181,11 @@ __device__ __forceinline__ void idscan_body(const DevParams& P, const DevBuffers
 }
 
 // A captured cell's new grain: record, L and id in the cell's slot, liquid bit
-// cleared, active bit set (CellularAutomataManager_3D::capture_cell,
+// cleared, active bit set if `active` (CellularAutomataManager_3D::capture_cell,
 // :676-707; Grain.cpp:13-18).  Returns the slot.
 __device__ __forceinline__ int write_child(const DevParams& P, const DevBuffers& B, int id, int ni,
-                                           int nj, int nk, int o, const double4& env) {
+                                           int nj, int nk, int o, const double4& env,
+                                           bool active) {
   const long long q = claim_index(P, ni, nj, nk);
   SlotRec r{};
   r.x = env.x;
@@ -1205,7 +1197,7 @@ __device__ __forceinline__ int write_child(const DevParams& P, const DevBuffers&
   r.stamp = (int)B.ctr->step + 1;  // grows from the next step on
   B.rec[q] = r;
   brick_clear(P, B.bmap, 0, ni, nj, nk);
-  atomicOr(&B.amap[q >> 6], 1ull << (q & 63));
+  if (active) atomicOr(&B.amap[q >> 6], 1ull << (q & 63));
   return (int)q;
 }
 
@@ -1238,7 +1230,8 @@ __device__ __forceinline__ void emit_from(const DevParams& P, const DevBuffers& 
     int di, dj, dk;
     slot_delta(s, di, dj, dk);
     kids[pos0 + j] =
-        write_child(P, B, id0 + j, ci + di, cj + dj, ck + dk, o, child_of(P, r, e, ci, cj, ck, di, dj, dk));
+        write_child(P, B, id0 + j, ci + di, cj + dj, ck + dk, o,
+                    child_of(P, r, e, ci, cj, ck, di, dj, dk), true);
     j++;
   }
 }
@@ -1268,6 +1261,17 @@ __device__ __forceinline__ void emit_children(const DevParams& P, const DevBuffe
 // not hold up the other lanes of its wave.  Wave 0 lists the children's slots
 // for wave 1 by parent block and position in the block (parents in brick
 // order); wave 1 lists them for the tail in id order.
+//
+// Wave 0's children are wave 1, and their envelope tests are made here, while the
+// envelope is in registers.  A launch of its own for them read record, list and map
+// words again: at 512^3 32 us a step and k_emit 44, now 4 and 60; the short step
+// has a launch less (256^3 98 to 89 us a step, 60^3 42 to 39).  The
+// cells still liquid for wave 1 are the ones that wave 0 left unclaimed: every
+// claimed cell is captured, and its liquid bit may or may not be cleared yet.
+// Wave 1's claimed bits therefore have a map of their own.  A child without a
+// liquid neighbour never enters the active map.  Whether one with liquid
+// neighbours stays active is wave 1's k_resolve's to say only if a grain of the
+// wave claimed a cell: without claims all of them stay.
 __device__ __forceinline__ void emit_body(const DevParams& P, const DevBuffers& B, int wave,
                                           int blk, int nblk) {
   const DevCounters* ctr = B.ctr;
@@ -1286,6 +1290,10 @@ __device__ __forceinline__ void emit_body(const DevParams& P, const DevBuffers& 
   const int4* __restrict__ seg = B.plist + lo;
   const int gbase = ctr->wave_gbase;
   int* __restrict__ kids = B.listW[wave];
+  __shared__ int s_ret;
+  if (threadIdx.x == 0) s_ret = 0;
+  int ret = 0;
+  unsigned any = 0;
   for (int pbase = 0; pbase < np; pbase += kBlock) {
     const int pt = pbase + threadIdx.x;
     int4 pe = make_int4(0, 0, 0, 0);
@@ -1323,11 +1331,31 @@ __device__ __forceinline__ void emit_body(const DevParams& P, const DevBuffers& 
         const int rank = c - pp.w;    // its rank among its parent's children
         const int p0 = B.coff[pp.x];  // the parent's first child in the wave
         const int pos = wave == 0 ? cb + c : p0 + rank;
-        kids[pos] = write_child(P, B, gbase + p0 + rank, ci + di, cj + dj, ck + dk, pr.o,
-                                child_of(P, r, e, ci, cj, ck, di, dj, dk));
+        const int id = gbase + p0 + rank;
+        const int ni = ci + di, nj = cj + dj, nk = ck + dk;
+        const double4 ne = child_of(P, r, e, ci, cj, ck, di, dj, dk);
+        if (wave == 0) {
+          const unsigned lm = open_bits26(P, B, ni, nj, nk);
+          double dmin;
+          const unsigned im = claim_tests<true>(P, B, id, pr.o, ni, nj, nk, lm, ne, nullptr, dmin);
+          const int nq = write_child(P, B, id, ni, nj, nk, pr.o, ne, lm != 0u);
+          kids[pos] = nq;
+          B.wake[nq] = wake_clock(P, ctr->S, ne.w, dmin);
+          B.masks[pos] = ((unsigned long long)im << 32) | lm;
+          ret += lm == 0u;
+          any |= im;
+        } else {
+          kids[pos] = write_child(P, B, id, ni, nj, nk, pr.o, ne, true);
+        }
       }
       __syncthreads();
     }
+  }
+  if (wave == 0) {
+    if (any) B.ctr->w1_claims = 1;
+    if (ret) atomicAdd(&s_ret, ret);
+    __syncthreads();
+    if (threadIdx.x == 0 && s_ret) atomicAdd(&B.ctr->w1_ret[blk & 63], s_ret);
   }
 }
 
@@ -1419,7 +1447,7 @@ __device__ __forceinline__ void tail_body(const DevParams& P, const DevBuffers& 
     const int* list = B.listW[in];
     int* kids = B.listW[wave & 1];
     for (int i = threadIdx.x; i < n; i += kTailBlock)
-      B.masks[i] = claim_entry<true>(P, B, list[i], nullptr);
+      B.masks[i] = claim_entry(P, B, list[i]);
     // one work-group: a work-group-scope fence orders its phases (the claim
     // and map words are read with agent-scope loads); an agent-scope fence
     // would also write back and invalidate the L2
@@ -1671,7 +1699,6 @@ hipError_t launch_batch_step(const BatchLaunch& L, hipStream_t s) {
                        L.map_cmp, 0);
     hipLaunchKernelGGL(kb_idscan, dim3(L.n_ids), dim3(kBlock), 0, s, L.P, L.B, L.map_ids, 0);
     hipLaunchKernelGGL(kb_emit, dim3(L.n_cmp), dim3(kBlock), 0, s, L.P, L.B, L.map_cmp, 0);
-    hipLaunchKernelGGL(kb_claim, dim3(L.n_list), dim3(kBlock), 0, s, L.P, L.B, L.map_list, 1);
     hipLaunchKernelGGL(kb_tail, dim3(L.n_one), dim3(kTailBlock), 0, s, L.P, L.B, L.map_one);
     return hipGetLastError();
   }
