@@ -387,14 +387,18 @@ amca_status amca_domain_create(const amca_domain_desc* desc, int32_t orient_capa
   c.t = 0.0;
   HIP_TRY(hipMemcpyAsync(B.ctr, &c, sizeof(c), hipMemcpyHostToDevice, d->stream));
   HIP_TRY(amca::launch_init_grid(P, B, d->stream));
-  // Grid sizes: enough blocks to fill 256 CUs several times over.
+  // Grid sizes.  The list kernels hold four blocks on a CU (their registers), and an
+  // entry is a chain of dependent loads, so they take as many blocks as the card
+  // holds at once, each with its share of the list: 512^3, claim / resolve / emit of
+  // wave 0 in us at 16, 12, 8 and 4 blocks per CU: 88 / 92 / 60, 86 / 88 / 56,
+  // 83 / 84 / 53, 80 / 80 / 50; at 3 and 2, claim / emit 85 / 52 and 97 / 57.
   int cus = 256;
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, d->device) == hipSuccess && prop.multiProcessorCount > 0)
     cus = prop.multiProcessorCount;
   long long want = (P.N + amca::kBlock - 1) / amca::kBlock;
-  d->list_blocks = (int)std::max(8LL, std::min<long long>((want + 7) / 8 * 8, 16LL * cus));
-  d->emit_blocks = (int)std::max(8LL, std::min<long long>((want + 7) / 8 * 8, std::min(16LL * cus, (long long)amca::kMaxBlocks)));
+  d->list_blocks = (int)std::max(8LL, std::min<long long>((want + 7) / 8 * 8, 4LL * cus));
+  d->emit_blocks = (int)std::max(8LL, std::min<long long>((want + 7) / 8 * 8, std::min(4LL * cus, (long long)amca::kMaxBlocks)));
   d->nuc_blocks = 1;
   // id scan: eight blocks per CU at most (each block's tiles run one after
   // another), at least 32 K ids per block
