@@ -602,7 +602,7 @@ amca_status amca_domain_download(amca_domain* d, int32_t* orient, int32_t* grain
   AMCA_TRY(read_counters(d, &c));
   // the grain-ID fields, materialized from the slots
   if (orient || grain) {
-    HIP_TRY(amca::launch_materialize(d->P, d->B, d->stream));
+    HIP_TRY(amca::launch_materialize(d->P, d->B, amca::kMatFields, d->stream));
     HIP_TRY(hipStreamSynchronize(d->stream));
   }
   if (orient) HIP_TRY(hipMemcpy(orient, d->B.oid, sizeof(int32_t) * NG, hipMemcpyDeviceToHost));
@@ -640,7 +640,7 @@ amca_status amca_domain_download_grains(amca_domain* d, int32_t cap, double* env
   *n_grains = c.n_grains;
   const size_t m = (size_t)std::max(0, std::min(cap, c.n_grains));
   if (m == 0) return AMCA_OK;
-  HIP_TRY(amca::launch_materialize(d->P, d->B, d->stream));
+  HIP_TRY(amca::launch_materialize(d->P, d->B, amca::kMatGrains, d->stream));
   HIP_TRY(hipStreamSynchronize(d->stream));
   if (env4) {
     HIP_TRY(hipMemcpy(env4, d->B.genv, sizeof(double) * 4 * m, hipMemcpyDeviceToHost));
@@ -660,7 +660,7 @@ amca_status amca_domain_device_fields(amca_domain* d, void** orient, void** grai
                                       void** stream) {
   if (!d) return fail(AMCA_ERR_INVALID, "null domain");
   if (orient || grain || env) {
-    HIP_TRY(amca::launch_materialize(d->P, d->B, d->stream));
+    HIP_TRY(amca::launch_materialize(d->P, d->B, amca::kMatDevice, d->stream));
     HIP_TRY(hipStreamSynchronize(d->stream));
   }
   if (orient) *orient = d->B.oid;

@@ -197,8 +197,10 @@ hipError_t launch_wake_claim(const DevParams& P, const DevBuffers& B, hipStream_
 // statistics words it reads)
 hipError_t launch_idscan(const DevParams& P, const DevBuffers& B, int wave, int nres,
                          hipStream_t s);
-// gid / oid on the ghosted grid, genv / gco by grain id, from the slots
-hipError_t launch_materialize(const DevParams& P, const DevBuffers& B, hipStream_t s);
+// from the slots: gid / oid on the ghosted grid (kMatFields), genv / gco by grain id
+// (kMatGrains), or gid / oid and genv (kMatDevice)
+enum { kMatFields, kMatGrains, kMatDevice };
+hipError_t launch_materialize(const DevParams& P, const DevBuffers& B, int what, hipStream_t s);
 // envelopes by cell of the n ghosted cells from c0 on
 hipError_t launch_cell_env(const DevParams& P, const DevBuffers& B, long long c0, int n, double4* out,
                            hipStream_t s);

@@ -1574,30 +1574,48 @@ __global__ void __launch_bounds__(kBlock) k_compact(DevParams P, DevBuffers B) {
 __global__ void __launch_bounds__(kBlock) k_idscan(DevParams P, DevBuffers B, int wave, int nres) {
   idscan_body(P, B, wave, blockIdx.x, nres);
 }
-// The reference's layouts from the slots, for downloads: per interior cell,
-// cellGrainID_ / cellOrientationID_ (-1 when liquid), and per solid cell's
-// grain its envelope and (cell, orientation) by id.  Ghost cells keep the 0
-// that k_init_grid wrote.  In this path a cell never melts again, so every
-// solid cell holds the grain created there.
-__global__ void k_materialize(DevParams P, DevBuffers B) {
-  const long long stride = (long long)gridDim.x * blockDim.x;
-  for (long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x; c < P.NG; c += stride) {
-    int i, j, k;
-    cell_ijk(P, (int)c, i, j, k);
-    if (i == 0 || j == 0 || k == 0 || i > P.nx || j > P.ny || k > P.nz) continue;
+// The reference's layouts from the slots, for downloads: per interior cell
+// (kFields), cellGrainID_ / cellOrientationID_ (-1 when liquid), and per solid cell's
+// grain its envelope (kEnv) and (cell, orientation) by id (kCells).  Ghost cells
+// keep the 0 that k_init_grid wrote.  In this path a cell never melts again, so
+// every solid cell holds the grain created there.
+//
+// Bound by the scattered writes by grain id.  A block takes a row of 16 bricks:
+// its grains are near in space and so, many of them, in id, and their writes
+// meet in one L2.  512^3, all but the cells: 13.1 ms in ghosted cell order with the
+// cells written too, 7.6 ms now.
+template <bool kFields, bool kEnv, bool kCells>
+__global__ void __launch_bounds__(kBlock) k_materialize(DevParams P, DevBuffers B) {
+  const int nx16 = (P.nbX + 15) >> 4;
+  const int blk = xcd_block();
+  const int tx = blk % nx16;
+  const int by = (blk / nx16) % P.nbY, bz = blk / (nx16 * P.nbY);
+  const int i = 64 * tx + (threadIdx.x & 63), k = 4 * bz + (threadIdx.x >> 6);
+  if (bz >= P.nbZ || i < 1 || i > P.nx || k < 1 || k > P.nz) return;
+#pragma unroll
+  for (int dj = 0; dj < 4; dj++) {
+    const int j = 4 * by + dj;
+    if (j < 1 || j > P.ny) continue;
+    const int c = (k * P.nyG + j) * P.nxG + i;
     if (B.bmap[brick_word(P, i, j, k)] & brick_bit(i, j, k)) {
-      B.gid[c] = -1;
-      B.oid[c] = -1;
+      if (kFields) {
+        B.gid[c] = -1;
+        B.oid[c] = -1;
+      }
       continue;
     }
     const long long q = claim_index(P, i, j, k);
     const SlotRec r = B.rec[q];
-    B.gid[c] = r.id;
-    B.oid[c] = r.o;
-    double L = r.L;
-    if ((B.amap[q >> 6] >> (q & 63)) & 1ull) L = grow_to(B, L, r.stamp, (int)B.ctr->step);
-    B.genv[r.id] = make_double4(r.x, r.y, r.z, L);
-    B.gco[r.id] = make_int2((int)c, r.o);
+    if (kFields) {
+      B.gid[c] = r.id;
+      B.oid[c] = r.o;
+    }
+    if (kEnv) {
+      double L = r.L;
+      if ((B.amap[q >> 6] >> (q & 63)) & 1ull) L = grow_to(B, L, r.stamp, (int)B.ctr->step);
+      B.genv[r.id] = make_double4(r.x, r.y, r.z, L);
+    }
+    if (kCells) B.gco[r.id] = make_int2(c, r.o);
   }
 }
 
@@ -1768,11 +1786,16 @@ hipError_t launch_idscan(const DevParams& P, const DevBuffers& B, int wave, int 
   return hipGetLastError();
 }
 
-hipError_t launch_materialize(const DevParams& P, const DevBuffers& B, hipStream_t s) {
-  long long blocks = ((long long)P.NG + 255) / 256;
-  if (blocks > 16384) blocks = 16384;
-  if (blocks < 1) blocks = 1;
-  hipLaunchKernelGGL(k_materialize, dim3((unsigned)blocks), dim3(256), 0, s, P, B);
+hipError_t launch_materialize(const DevParams& P, const DevBuffers& B, int what, hipStream_t s) {
+  // whole eighths, for the XCDs
+  const long long tiles = (long long)((P.nbX + 15) / 16) * P.nbY * P.nbZ;
+  const dim3 grid((unsigned)((tiles + 7) / 8 * 8));
+  if (what == kMatFields)
+    hipLaunchKernelGGL((k_materialize<true, false, false>), grid, dim3(kBlock), 0, s, P, B);
+  else if (what == kMatGrains)
+    hipLaunchKernelGGL((k_materialize<false, true, true>), grid, dim3(kBlock), 0, s, P, B);
+  else
+    hipLaunchKernelGGL((k_materialize<true, true, false>), grid, dim3(kBlock), 0, s, P, B);
   return hipGetLastError();
 }
 

@@ -65,3 +65,40 @@ def test_growth_past_the_clock_span(amca, oracle):
     r = compare(oracle, prm, run_gpu(amca, text))
     grown = np.cumsum(r["steps"]["dt"][:r["n_steps"]])
     assert r["n_orient"] >= 1 and grown.size < 2048
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (3, 62, 6), (62, 3, 2), (63, 5, 7), (130, 9, 4)])
+def test_device_fields_match_the_downloads(amca, shape):
+    """The by-cell and by-id layouts on the device, part-way through a run, on grids
+    around the 16-brick rows that their kernel takes: the same values as the
+    downloads of fields, envelopes and grains."""
+    import ctypes as C
+
+    from amca3d_amd._lib import load
+    memcpy = load().hipMemcpy  # of the runtime that the library is linked to
+    memcpy.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int]
+
+    def host(ptr, shape, dtype):
+        a = np.empty(shape, dtype)
+        assert memcpy(a.ctypes.data, ptr.value, a.nbytes, 2) == 0  # device to host
+        return a
+
+    text, _ = _case(shape, 0.2, 2e-3, density=2e15)
+    s = amca.Simulation(text).initialize()
+    n = s.run(30)["n_grains"]
+    d = s.domain
+    f = d.download()
+    o, g, e = C.c_void_p(), C.c_void_p(), C.c_void_p()
+    assert load().amca_domain_device_fields(d.h, C.byref(o), C.byref(g), C.byref(e), None) == 0
+    ng = f["gid"].size
+    for p, want in ((o, f["ori"]), (g, f["gid"])):
+        assert np.array_equal(host(p, ng, np.int32), want.ravel())
+    r = d.download_grains()
+    assert r["cell"].size == n
+    if n:
+        env = host(e, (n, 4), np.float64)
+        assert np.array_equal(env, r["env"])
+        assert np.array_equal(f["gid"].ravel()[r["cell"]], np.arange(n))
+        assert np.array_equal(f["ori"].ravel()[r["cell"]], r["orient"])
+        assert np.array_equal(f["env"].reshape(-1, 4)[r["cell"]], env)
+    s.close()
