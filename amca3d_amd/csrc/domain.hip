@@ -409,8 +409,9 @@ amca_status amca_domain_create(const amca_domain_desc* desc, int32_t orient_capa
   // grow at most a quarter of a cell per step (dt <= time_step_factor h / v), which
   // keeps captures by wave 1's fresh envelopes rare: k_tail takes those with one
   // work-group.  Short against long form when the line was drawn (wave 1's tests had
-  // a launch of their own in both): 131x97x67 46 against 68 us a step, 256^3 98 against 135; at 512^3 k_tail's one work-group takes 730 us
-  // of 1050 (long form 347).
+  // a launch of their own in both): 131x97x67 46 against 68 us a step, 256^3 98
+  // against 135; at 512^3 k_tail's one work-group takes 730 us of 1050 (long form
+  // 347).
   P.fused = P.N <= kFusedCells && desc->time_step_factor <= 0.25 ? 1 : 0;
   // compaction and retirement: the 64-brick pieces of the grid over at most eight
   // blocks per CU; two for the short step, whose wave-0 kernels all have these blocks
