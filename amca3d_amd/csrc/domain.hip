@@ -789,17 +789,26 @@ struct amca_batch {
 
 namespace {
 
-// Per-domain block counts of the list kernels under a schedule: a budget of
+// The blocks that a budget stands for: all of it up to four per CU, which are
+// resident at once, then four per CU until a quarter of it is more.  Only awake
+// grains are in the lists, so more blocks than that mostly start up for a
+// fraction of a tile each, and far fewer leave the last ones to carry the run.
+// A run's ms at 2, 4, 8 and 16 blocks per CU: 16 uneven domains, short step 83, 68,
+// 70, 87, long step 86, 73, 76, 91; 64 of 32^3, long step 29, 34, 44, 49; 8 of 160^3,
+// long step 63, 61, 64, 71; 4 of 256^3, long step 106, 94, 98, 106.
+int budget_blocks(const amca_batch* b, int budget) {
+  return std::max(budget / 4, std::min(budget, 4 * b->cus));
+}
+
+// Per-domain block counts of the list kernels under a schedule: the budget of
 // `list_blocks` blocks (and emit_blocks for resolve/emit) shared in proportion
 // to the domains' cell counts, at least `min_blocks` each, capped by what a
 // domain can use (one block per 256 cells of its grid, kMaxBlocks for the
-// scanned kernels).  The short step's blocks hold bricks, asleep or not, and start
-// up for a fraction of a tile each: it takes a quarter of the budgets (16 uneven
-// domains, ms for the run at budgets of 2, 4, 8, 16 and 32 blocks per CU: 86, 71, 73,
-// 89, 119).
+// scanned kernels).
 void batch_geometry(const amca_batch* b, std::vector<int>& nl, std::vector<int>& ne) {
   const size_t n = b->doms.size();
-  const double part = b->L.fused ? 0.25 : 1.0;
+  const int list = budget_blocks(b, b->sched.list_blocks);
+  const int emit = budget_blocks(b, b->sched.emit_blocks);
   double total = 0.0;
   for (size_t i = 0; i < n; i++)
     if (b->active[i]) total += (double)b->doms[i]->P.N;
@@ -809,8 +818,8 @@ void batch_geometry(const amca_batch* b, std::vector<int>& nl, std::vector<int>&
     if (!b->active[i]) continue;
     const double share = (double)b->doms[i]->P.N / total;
     const long long cap = std::max(1LL, (b->doms[i]->P.N + amca::kBlock - 1) / amca::kBlock);
-    long long l = (long long)std::llround(share * part * b->sched.list_blocks);
-    long long e = (long long)std::llround(share * part * b->sched.emit_blocks);
+    long long l = (long long)std::llround(share * list);
+    long long e = (long long)std::llround(share * emit);
     l = std::max<long long>(b->sched.min_blocks, std::min(l, cap));
     // resolve / emit blocks keep per-block stats in kMaxBlocks slots
     e = std::min(std::max<long long>(b->sched.min_blocks, std::min(e, cap)), (long long)amca::kMaxBlocks);
