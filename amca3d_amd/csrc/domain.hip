@@ -25,6 +25,30 @@ namespace {
 
 constexpr long long kFusedCells = 1ll << 24;
 
+// When a domain that may take the short step takes the long one: while its wave-1
+// grains in steps with a wave-1 claim (DevCounters::w1_walk) are more than kWalkShort
+// a step.  In the short step k_tail's one work-group walks them, about 4 us for every
+// thousand, against some 18 us a step saved by the shorter form.  How many there are
+// depends on the growth per step, the truncation and the density of the grains, so
+// it is measured as the run goes.  Short against long form, us a step (walked grains a
+// step): 128^3 68.7 / 74.4 (2925), 102 / 94 (7489); 160^3 66.1 / 76.6 (2813), 103 / 89
+// (9347); 200^3 71.8 / 84.2 (2343), 97 / 87 (8538); 256^3 93 / 100 (2863), 102 / 102
+// (4510), 128 / 106 (10600), 372 / 152 (61145).  In a batch the launches are shared
+// (4 to 8 us a step between the forms) and any member's walk holds up the rest, so
+// kWalkBatch is the limit for the members' sum: 8 domains of 160^3 59.2 / 60.6 ms a
+// run (some 400 walked grains a step), 4 of 256^3 111 / 94 (11000).
+constexpr long long kWalkShort = 4500, kWalkBatch = 2000;
+constexpr long long kFormSteps = 8;  // steps between looks at w1_walk, at least
+// More than kBurstSites live sites in more than kBurstCells cells may nucleate in a burst
+// of a few tens of steps, over before a look can answer it, so such a domain takes the
+// long step from the start until an eighth of kBurstSites is left.  256^3 with 2.7e5
+// sites: 50 ms a run by the walk alone, 37 with the long step from the start; 160^3 with
+// 3.3e4: 20.6 and 21.6, but at 1 K a step, where they all nucleate within ten steps, 19.5
+// and 10.0; 200^3 with 1.9e4: 27.8 and 29.7, at 1 K a step 22.7 and 18.5; 240^3 with 1.1e4:
+// 33.3 and 37.6, 25.7 and 26.5.
+constexpr int kBurstSites = 24000;
+constexpr long long kBurstCells = 1ll << 21;
+
 thread_local std::string g_last_error;
 
 amca_status fail(amca_status st, const std::string& msg) {
@@ -61,7 +85,6 @@ struct amca_domain {
   int list_blocks = 1;
   int emit_blocks = 1;
   int ids_blocks = 1;
-  int cmp_blocks = 1;
   bool timing = false;
   // event pairs recorded around timed launches, resolved when times are read
   std::vector<hipEvent_t> ev_pool;
@@ -75,14 +98,30 @@ struct amca_domain {
   // AMCA_DOMAIN_GRAPH_STEPS sets the count (0: no graphs, every step launched
   // on its own, for tools that do not follow graph launches).
   int graph_steps = 16;
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t gexec = nullptr;
+  hipGraph_t graph[2] = {nullptr, nullptr};  // by step form (P.fused)
+  hipGraphExec_t gexec[2] = {nullptr, nullptr};
+  // step form: whether the short one may be taken, compaction blocks by form, and the
+  // counters at the last look at w1_walk
+  bool may_fuse = false, walk_ok = true, many_sites = false;
+  int cmp_blocks[2] = {1, 1};
+  long long seen_step = 0, seen_walk = 0;
+  // counters copied behind a stretch of queued steps (pinned) and the event behind
+  // the copy, for two stretches in flight (run_steps)
+  amca::DevCounters* look[2] = {nullptr, nullptr};
+  hipEvent_t looked[2] = {nullptr, nullptr};
+
+  void set_form(int fused) {
+    P.fused = fused;
+    P.cmp_blocks = cmp_blocks[fused];
+  }
 
   void drop_graph() {
-    if (gexec) (void)hipGraphExecDestroy(gexec);
-    if (graph) (void)hipGraphDestroy(graph);
-    gexec = nullptr;
-    graph = nullptr;
+    for (int f = 0; f < 2; f++) {
+      if (gexec[f]) (void)hipGraphExecDestroy(gexec[f]);
+      if (graph[f]) (void)hipGraphDestroy(graph[f]);
+      gexec[f] = nullptr;
+      graph[f] = nullptr;
+    }
   }
 
   template <class T>
@@ -104,6 +143,10 @@ struct amca_domain {
     for (void* p : allocs) (void)hipFree(p);
     for (auto& e : ev_pool)
       if (e) (void)hipEventDestroy(e);
+    for (auto& e : looked)
+      if (e) (void)hipEventDestroy(e);
+    for (auto& p : look)
+      if (p) (void)hipHostFree(p);
     if (stream) (void)hipStreamDestroy(stream);
   }
 };
@@ -187,8 +230,8 @@ amca_status enqueue_step(amca_domain* d) {
     AMCA_TRY(timed(d, K_TAIL, [&] { return amca::launch_tail(P, B, s); }));
     return AMCA_OK;
   }
-  AMCA_TRY(timed(d, K_CNT, [&] { return amca::launch_count(P, B, d->cmp_blocks, s); }));
-  AMCA_TRY(timed(d, K_COMPACT, [&] { return amca::launch_compact(P, B, d->cmp_blocks, s); }));
+  AMCA_TRY(timed(d, K_CNT, [&] { return amca::launch_count(P, B, P.cmp_blocks, s); }));
+  AMCA_TRY(timed(d, K_COMPACT, [&] { return amca::launch_compact(P, B, P.cmp_blocks, s); }));
   for (int wave = 0; wave < 2; wave++) {
     AMCA_TRY(timed(d, K_CLAIM, [&] { return amca::launch_claim(P, B, wave, d->list_blocks, s); }));
     AMCA_TRY(timed(d, K_RESOLVE,
@@ -202,7 +245,6 @@ amca_status enqueue_step(amca_domain* d) {
 }
 
 amca_status capture_steps(amca_domain* d) {
-  d->drop_graph();
   HIP_TRY(hipStreamBeginCapture(d->stream, hipStreamCaptureModeThreadLocal));
   amca_status st = AMCA_OK;
   for (int q = 0; q < d->graph_steps && st == AMCA_OK; q++) st = enqueue_step(d);
@@ -212,9 +254,25 @@ amca_status capture_steps(amca_domain* d) {
     if (g) (void)hipGraphDestroy(g);
     return st != AMCA_OK ? st : fail(AMCA_ERR_HIP, std::string("graph capture: ") + hipGetErrorString(e));
   }
-  d->graph = g;
-  HIP_TRY(hipGraphInstantiate(&d->gexec, g, nullptr, nullptr, 0));
+  const int f = d->P.fused;
+  if (d->graph[f]) (void)hipGraphDestroy(d->graph[f]);
+  d->graph[f] = g;
+  HIP_TRY(hipGraphInstantiate(&d->gexec[f], g, nullptr, nullptr, 0));
   return AMCA_OK;
+}
+
+// The step form for the coming steps, from the live sites and the walk of the steps
+// since the last look.  Every step leaves the same state in either form.
+void choose_form(amca_domain* d, const amca::DevCounters& c) {
+  if (!d->may_fuse) return;
+  const long long steps = c.step - d->seen_step;
+  if (steps >= kFormSteps) {
+    d->walk_ok = c.w1_walk - d->seen_walk <= kWalkShort * steps;
+    d->seen_step = c.step;
+    d->seen_walk = c.w1_walk;
+  }
+  d->many_sites = d->P.N > kBurstCells && c.n_sites > (d->many_sites ? kBurstSites / 8 : kBurstSites);
+  d->set_form(d->walk_ok && !d->many_sites ? 1 : 0);
 }
 
 // n steps: whole graphs of graph_steps steps, then single launches (every
@@ -223,12 +281,43 @@ amca_status capture_steps(amca_domain* d) {
 amca_status enqueue_steps(amca_domain* d, long long n) {
   if (!d->timing && d->graph_steps > 0) {
     for (; n >= d->graph_steps; n -= d->graph_steps) {
-      if (!d->gexec) AMCA_TRY(capture_steps(d));
-      HIP_TRY(hipGraphLaunch(d->gexec, d->stream));
+      if (!d->gexec[d->P.fused]) AMCA_TRY(capture_steps(d));
+      HIP_TRY(hipGraphLaunch(d->gexec[d->P.fused], d->stream));
     }
   }
   for (; n > 0; n--) AMCA_TRY(enqueue_step(d));
   return AMCA_OK;
+}
+
+// Up to `most` steps (negative: no limit), until the run is over if `to_end`; *c holds
+// the counters before and after.  Two stretches of steps are in flight, so that the
+// look at one stretch's counters costs the GPU nothing; 16 steps each where the form
+// may change with the look, which comes a stretch late (a nucleation burst in 256^3 at
+// 2e15 sites a cubic metre: 373 us a step in stretches of up to 64).
+amca_status run_steps(amca_domain* d, long long most, bool to_end, amca::DevCounters* c) {
+  for (int q = 0; q < 2; q++) {
+    if (!d->look[q]) HIP_TRY(hipHostMalloc(&d->look[q], sizeof(amca::DevCounters)));
+    if (!d->looked[q]) HIP_TRY(hipEventCreateWithFlags(&d->looked[q], hipEventDisableTiming));
+  }
+  const long long longest = d->may_fuse ? 16 : 64;
+  long long len = 8, queued = 0, seen = 0;  // seen, made: stretches looked at and queued
+  long long made = 0;
+  while (true) {
+    const bool over = c->err || (to_end && (c->done || !(c->t < d->desc.final_time)));
+    for (; !over && made - seen < 2 && (most < 0 || queued < most); made++) {
+      const long long k = most < 0 ? len : std::min(len, most - queued);
+      choose_form(d, *c);
+      AMCA_TRY(enqueue_steps(d, k));
+      HIP_TRY(hipMemcpyAsync(d->look[made & 1], d->B.ctr, sizeof(amca::DevCounters),
+                             hipMemcpyDeviceToHost, d->stream));
+      HIP_TRY(hipEventRecord(d->looked[made & 1], d->stream));
+      queued += k;
+      len = std::min(2 * len, longest);
+    }
+    if (made == seen) return AMCA_OK;
+    HIP_TRY(hipEventSynchronize(d->looked[seen & 1]));
+    *c = *d->look[seen++ & 1];
+  }
 }
 
 // Every live site can nucleate once and takes the next orientation row, so a
@@ -405,22 +494,22 @@ amca_status amca_domain_create(const amca_domain_desc* desc, int32_t orient_capa
   d->ids_blocks = (int)std::max(1LL, std::min<long long>((P.N + 32767) / 32768,
                                                          std::min(8LL * cus, (long long)amca::kMaxIdsBlocks)));
   P.ids_blocks = d->ids_blocks;
-  // The short step (see plain_step.hip) for grids of up to kFusedCells whose grains
-  // grow at most a quarter of a cell per step (dt <= time_step_factor h / v), which
-  // keeps captures by wave 1's fresh envelopes rare: k_tail takes those with one
-  // work-group.  Short against long form when the line was drawn (wave 1's tests had
-  // a launch of their own in both): 131x97x67 46 against 68 us a step, 256^3 98
-  // against 135; at 512^3 k_tail's one work-group takes 730 us of 1050 (long form
-  // 347).
-  P.fused = P.N <= kFusedCells && desc->time_step_factor <= 0.25 ? 1 : 0;
+  // The short step (see plain_step.hip) may be taken on grids of up to kFusedCells
+  // whose grains grow at most a quarter of a cell per step (dt <= time_step_factor
+  // h / v): there captures by wave 1's fresh envelopes, which k_tail takes with one
+  // work-group, are rare unless the grains are dense or the truncation is large
+  // (choose_form).  Short against long form, us a step, at 5e13 sites a cubic metre:
+  // 64^3 39 / 53, 128^3 50 / 67, 200^3 64 / 85, 256^3 93 / 100, 320^3 152 / 129.
+  d->may_fuse = P.N <= kFusedCells && desc->time_step_factor <= 0.25;
   // compaction and retirement: the 64-brick pieces of the grid over at most eight
   // blocks per CU; two for the short step, whose wave-0 kernels all have these blocks
   // and each of them starts up for a few dozen entries (256^3: 113, 101 and 98 us a
   // step at 8, 4 and 2 per CU; 512^3 long form: 347, 346, 381)
-  d->cmp_blocks = (int)std::max(1LL, std::min<long long>((nB + 63) / 64,
-                                                         std::min((P.fused ? 2LL : 8LL) * cus,
-                                                                  (long long)amca::kMaxBlocks)));
-  P.cmp_blocks = d->cmp_blocks;
+  for (int f = 0; f < 2; f++)
+    d->cmp_blocks[f] = (int)std::max(1LL, std::min<long long>((nB + 63) / 64,
+                                                              std::min((f ? 2LL : 8LL) * cus,
+                                                                       (long long)amca::kMaxBlocks)));
+  d->set_form(d->may_fuse ? 1 : 0);
   if (amca::env_int("AMCA_DOMAIN_GRAPH_STEPS", 0, 1024, &d->graph_steps) < 0) {
     delete d;
     return fail(AMCA_ERR_INVALID, "AMCA_DOMAIN_GRAPH_STEPS must be an integer in [0, 1024]");
@@ -499,6 +588,7 @@ amca_status amca_domain_step(amca_domain* d, amca_counters* out) {
   amca::DevCounters c;
   AMCA_TRY(read_counters(d, &c));
   AMCA_TRY(check_rows(d, c));
+  choose_form(d, c);
   AMCA_TRY(enqueue_step(d));
   AMCA_TRY(read_counters(d, &c));
   fill_counters(d, c, out);
@@ -510,19 +600,7 @@ amca_status amca_domain_run(amca_domain* d, int64_t max_steps, amca_counters* ou
   amca::DevCounters c;
   AMCA_TRY(read_counters(d, &c));
   AMCA_TRY(check_rows(d, c));
-  const long long start = c.step;
-  long long batch = 8;
-  while (true) {
-    bool finished = c.done || !(c.t < d->desc.final_time);
-    if (finished || c.err) break;
-    long long taken = c.step - start;
-    if (max_steps >= 0 && taken >= max_steps) break;
-    long long k = batch;
-    if (max_steps >= 0) k = std::min<long long>(k, max_steps - taken);
-    AMCA_TRY(enqueue_steps(d, k));
-    AMCA_TRY(read_counters(d, &c));
-    batch = std::min<long long>(batch * 2, 64);
-  }
+  AMCA_TRY(run_steps(d, max_steps, true, &c));
   fill_counters(d, c, out);
   return check_err(d, c);
 }
@@ -532,6 +610,7 @@ amca_status amca_domain_run_fixed(amca_domain* d, int64_t n_steps) {
   amca::DevCounters c;
   AMCA_TRY(read_counters(d, &c));
   AMCA_TRY(check_rows(d, c));
+  if (d->may_fuse) return run_steps(d, n_steps, false, &c);
   AMCA_TRY(enqueue_steps(d, n_steps));
   HIP_TRY(hipStreamSynchronize(d->stream));
   return AMCA_OK;
@@ -745,6 +824,11 @@ amca_status amca_envelope_selftest(int32_t n, const double* env4, const double* 
 struct amca_batch {
   std::vector<amca_domain*> doms;
   std::vector<amca::DevParams> P;  // the domains' parameters with the batch's step form and grids
+  // whether every domain may take the short step; the domains' walks (w1_walk, low 31
+  // bits) when they were last looked at and the steps run since
+  bool may_fuse = false;
+  std::vector<int> walk0;
+  long long walk_steps = 0;
   int device = 0;
   hipStream_t stream = nullptr;
   amca::DevParams* dP = nullptr;
@@ -865,6 +949,7 @@ amca_status batch_apply_schedule(amca_batch* b) {
                                                                    (long long)amca::kMaxBlocks}))
                          : 0;
     b->P[i].cmp_blocks = std::max(1, nc[i]);
+    b->P[i].fused = b->L.fused;
     one[i] = b->active[i] ? 1 : 0;
   }
   std::vector<int> order(n);
@@ -937,7 +1022,9 @@ amca_status batch_capture(amca_batch* b, int steps) {
 // finished runs steps that all skip.  With `remap`, once max(4, n/8) more
 // domains have finished the maps are rebuilt over the domains still running,
 // so that the budgets of the list kernels go to them alone (a finished
-// domain's kernels return at once, so leaving it out changes no result).
+// domain's kernels return at once, so leaving it out changes no result), and the
+// step form is chosen again; from the short form to the long one the batch also
+// goes as soon as its walk asks for it.
 amca_status batch_replay(amca_batch* b, long long max_graphs, int* finished, double* ms,
                          long long* replays, bool remap) {
   if (b->use_graph && (!b->exec || b->graph_steps != b->sched.steps_per_graph))
@@ -967,6 +1054,19 @@ amca_status batch_replay(amca_batch* b, long long max_graphs, int* finished, dou
     if (e == hipSuccess) e = hipEventRecord(b->hready[r & 1], b->stream);
     return e;
   };
+  // the walk of the steps since the last look against the limit (the short form's)
+  bool walk_short = b->L.fused != 0;
+  auto look = [&](const int4* st, long long steps) {
+    b->walk_steps += steps;
+    if (b->walk_steps < kFormSteps) return;
+    long long walk = 0;
+    for (int i = 0; i < n; i++) {
+      walk += (st[i].w - b->walk0[i]) & 0x7fffffff;
+      b->walk0[i] = st[i].w;
+    }
+    walk_short = walk <= kWalkBatch * b->walk_steps;
+    b->walk_steps = 0;
+  };
   HIP_TRY(hipEventRecord(ev.e0, b->stream));
   long long r = 0, queued = 0;
   int fin = 0;
@@ -991,7 +1091,9 @@ amca_status batch_replay(amca_batch* b, long long max_graphs, int* finished, dou
       fin += st[i].x;
     }
     if (fin == n) break;
-    if (remap && fin - b->mapped_finished >= std::max(4, n / 8)) {
+    look(st, b->sched.steps_per_graph);
+    const bool to_long = b->L.fused && !walk_short;
+    if (remap && (to_long || fin - b->mapped_finished >= std::max(4, n / 8))) {
       // rebuild the maps over the running domains: wait for the queued replay,
       // take the finished set from its status, and capture a new graph
       HIP_TRY(hipStreamSynchronize(b->stream));
@@ -1003,9 +1105,11 @@ amca_status batch_replay(amca_batch* b, long long max_graphs, int* finished, dou
         fin += last[i].x;
         b->active[i] = last[i].x ? 0 : 1;
       }
+      if (queued > r) look(last, b->sched.steps_per_graph * (queued - r));
       r = queued;
       if (fin == n) break;
       b->mapped_finished = fin;
+      b->L.fused = b->may_fuse && walk_short;
       AMCA_TRY(batch_apply_schedule(b));
       if (b->use_graph) AMCA_TRY(batch_capture(b, b->sched.steps_per_graph));
       if (max_graphs < 0 || queued < max_graphs) {
@@ -1033,6 +1137,7 @@ amca_status amca_batch_create(amca_domain* const* doms, int32_t n, amca_batch** 
   if (!doms || n < 1 || !out) return fail(AMCA_ERR_INVALID, "need at least one domain");
   *out = nullptr;
   auto* b = new amca_batch();
+  bool many_sites = false;
   for (int i = 0; i < n; i++) {
     if (!doms[i]) {
       delete b;
@@ -1050,6 +1155,9 @@ amca_status amca_batch_create(amca_domain* const* doms, int32_t n, amca_batch** 
       return rows;
     }
     b->doms.push_back(doms[i]);
+    b->walk0.push_back((int)(c.w1_walk & 0x7fffffffll));
+    choose_form(doms[i], c);
+    many_sites |= doms[i]->many_sites;
   }
   amca_status st = AMCA_OK;
   do {
@@ -1069,11 +1177,12 @@ amca_status amca_batch_create(amca_domain* const* doms, int32_t n, amca_batch** 
       if (hipStreamSynchronize(b->doms[i]->stream) != hipSuccess) { st = fail(AMCA_ERR_HIP, "sync"); break; }
       P[i] = b->doms[i]->P;
       B[i] = b->doms[i]->B;
-      b->L.fused = (i == 0 || b->L.fused) && P[i].fused;
+      b->may_fuse = (i == 0 || b->may_fuse) && b->doms[i]->may_fuse;
     }
     if (st != AMCA_OK) break;
-    // one launch sequence for the batch: the short one if every domain takes it
-    for (auto& p : P) p.fused = b->L.fused;
+    // one launch sequence for the batch: the short one if every domain may take it,
+    // as long as their sites and walks allow (batch_replay)
+    b->L.fused = b->may_fuse && !many_sites ? 1 : 0;
     if (hipMalloc(&b->dP, sizeof(amca::DevParams) * n) != hipSuccess ||
         hipMalloc(&b->dB, sizeof(amca::DevBuffers) * n) != hipSuccess ||
         hipMalloc(&b->status, sizeof(int4) * n) != hipSuccess ||

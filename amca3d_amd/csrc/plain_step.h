@@ -70,6 +70,9 @@ struct DevCounters {
   // liquid neighbour, spread over 64 slots
   int w1_claims;
   int w1_ret[64];
+  // wave-1 grains of the steps in which one of them claimed a cell, since the domain
+  // was made: what k_tail's one work-group walks in the short step
+  long long w1_walk;
 };
 
 struct StepLogRow {
@@ -220,10 +223,11 @@ struct BatchLaunch {
   const int4* map_ids;   // id-scan geometry
   const int4* map_cmp;   // compaction geometry (k_count and k_compact)
   int n_nuc, n_list, n_emit, n_one, n_ids, n_cmp;
-  int fused;             // every domain takes the short step
+  int fused;             // the domains take the short step
 };
 hipError_t launch_batch_step(const BatchLaunch& L, hipStream_t s);
-// out[d] = (finished, error, step & 0x7fffffff, step >> 31) for each of n domains
+// out[d] = (finished, error, step, w1_walk), the last two their low 31 bits, for each
+// of n domains
 hipError_t launch_batch_status(const BatchLaunch& L, int n, int4* out, hipStream_t s);
 hipError_t launch_envelope_selftest(int n, const double* env4, const double* l2g9,
                                     const double* cell3, double h, double trunc, double sqrt2f,

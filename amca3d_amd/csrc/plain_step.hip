@@ -1497,6 +1497,7 @@ __device__ __forceinline__ void tail_body(const DevParams& P, const DevBuffers& 
     ctr->n_solid = solid;
     const long long liquid = P.N - solid;
     if (liquid == 0) ctr->done = 1;
+    if (ctr->w1_claims) ctr->w1_walk += n_wave1;
     if (B.log && st < ctr->log_cap) {
       StepLogRow row;
       row.time_before = t0;
@@ -1694,14 +1695,14 @@ __global__ void __launch_bounds__(kBlock) kb_idscan(const DevParams* Ps, const D
   idscan_body(Ps[m.x], Bs[m.x], wave, m.y, m.w);
 }
 
-// per-domain status after a batch of steps: (finished, error, steps low, steps high)
+// per-domain status after a batch of steps: (finished, error, steps, w1_walk), the last
+// two their low 31 bits
 __global__ void kb_status(const DevParams* Ps, const DevBuffers* Bs, int n, int4* out) {
   const int d = blockIdx.x * blockDim.x + threadIdx.x;
   if (d >= n) return;
   const DevCounters* c = Bs[d].ctr;
   const int fin = (c->done || !(c->t < Ps[d].final_time)) ? 1 : 0;
-  const unsigned long long st = (unsigned long long)c->step;
-  out[d] = make_int4(fin, c->err, (int)(st & 0x7fffffffull), (int)(st >> 31));
+  out[d] = make_int4(fin, c->err, (int)(c->step & 0x7fffffffll), (int)(c->w1_walk & 0x7fffffffll));
 }
 
 hipError_t launch_batch_status(const BatchLaunch& L, int n, int4* out, hipStream_t s) {
