@@ -112,7 +112,8 @@ struct RmBuffers {
   int* flist;             // the step's flagged cells that carry a grain, in no order
                           // [kRmParts * flist_cap]
   int2* clist;            // the step's captures: capturing cell; slot, rank among the cell's
-                          // fresh captures << 5, fresh << 10 [N]
+                          // fresh captures << 5, fresh << 10 (between steps,
+                          // scratch of the downloads) [N]
   double4* genv;          // grain envelope by grain id [N]
   int2* gco;              // grain -> (cell, orientation) [N]
   const double* frames;   // nodal frames [n_frames * nodes]

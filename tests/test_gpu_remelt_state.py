@@ -48,6 +48,30 @@ def _state(holes=0):
                 grain_orient=rng.integers(0, 3, n).astype(np.int32))
 
 
+@pytest.mark.parametrize("spare", [0, 1, 305, 2**18 - 120, 2**18 - 119, 2**18 + 1])
+def test_download_of_more_records_than_cells(amca, spare):
+    """Records that no cell owns, on both sides of 2^18 in all: above it cells and
+    orientations come back in pieces of one record per cell (120), whole ones (a cap of
+    2^18 + 56 is 2185 of them) and a remainder."""
+    d = _domain(amca)
+    st = _state()
+    n = len(st["grain_cell"])
+    assert n == NX * NY * NZ
+    rng = np.random.default_rng(2)
+    st["grain_cell"] = np.concatenate([st["grain_cell"],
+                                       rng.integers(0, len(st["ori"]), spare).astype(np.int32)])
+    st["grain_orient"] = np.concatenate([st["grain_orient"],
+                                         rng.integers(0, 3, spare).astype(np.int32)])
+    d.set_state(st)
+    for cap in (None, n + spare // 2, 2**18 + 56, 1):
+        g = d.download(None if cap is None else min(cap, n + spare))
+        m = n + spare if cap is None else min(cap, n + spare)
+        assert g["n_grains"] == n + spare and len(g["grain_cell"]) == m
+        assert np.array_equal(g["grain_cell"], st["grain_cell"][:m])
+        assert np.array_equal(g["grain_orient"], st["grain_orient"][:m])
+    d.close()
+
+
 @pytest.mark.parametrize("holes", [0, 9])
 def test_loaded_layout(amca, holes):
     d = _domain(amca)
