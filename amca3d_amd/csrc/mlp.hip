@@ -136,7 +136,7 @@ enum FusedMode : int {
 struct NetImage;
 size_t net_image_bytes();
 hipError_t fused_setup();
-hipError_t launch_pack(const float* p, NetImage* img, hipStream_t st);
+hipError_t launch_pack(const float* p, NetImage* img, float* m, float* v, hipStream_t st);
 // training (defined at the end of the kernels): one 64-row group per work-group
 // and pass, at most one work-group per CU
 constexpr int kTrainRows = 64;
@@ -281,10 +281,8 @@ amca_status train_blocks(amca_mlp* h, int n, int* blocks) {
 amca_status load_params(amca_mlp* h, const float* p) {
   const size_t bytes = sizeof(float) * h->lay.total;
   MLP_HIP(hipMemcpyAsync(h->params, p, bytes, hipMemcpyHostToDevice, h->stream));
-  MLP_HIP(hipMemsetAsync(h->adam_m, 0, bytes, h->stream));
-  MLP_HIP(hipMemsetAsync(h->adam_v, 0, bytes, h->stream));
   h->adam_t = 0;
-  MLP_HIP(launch_pack(h->params, h->image, h->stream));
+  MLP_HIP(launch_pack(h->params, h->image, h->adam_m, h->adam_v, h->stream));
   MLP_HIP(hipStreamSynchronize(h->stream));
   return AMCA_OK;
 }
@@ -792,15 +790,21 @@ __device__ __forceinline__ void pack_param(NetImage& N, int i, float v) {
   N.wb[l - 1][in >> 5][out >> 4][((out >> 3) & 1) * 32 + (in & 31)][out & 7] = (__bf16)v;
 }
 
+// The images of all parameters, and Adam's moments from zero.
 __global__ void __launch_bounds__(kThreads) k_pack(const float* __restrict__ p,
-                                                   NetImage* __restrict__ img) {
+                                                   NetImage* __restrict__ img,
+                                                   float* __restrict__ m, float* __restrict__ v) {
   const int i = blockIdx.x * kThreads + threadIdx.x;
-  if (i < fused_b(3) + 2 * kHid + 1) pack_param(*img, i, p[i]);
+  if (i >= fused_b(3) + 2 * kHid + 1) return;
+  pack_param(*img, i, p[i]);
+  m[i] = 0.0f;
+  v[i] = 0.0f;
 }
 
-hipError_t launch_pack(const float* p, NetImage* img, hipStream_t st) {
+hipError_t launch_pack(const float* p, NetImage* img, float* m, float* v, hipStream_t st) {
   const int n = Layout().total;
-  hipLaunchKernelGGL(k_pack, dim3((n + kThreads - 1) / kThreads), dim3(kThreads), 0, st, p, img);
+  hipLaunchKernelGGL(k_pack, dim3((n + kThreads - 1) / kThreads), dim3(kThreads), 0, st, p, img, m,
+                     v);
   return hipGetLastError();
 }
 

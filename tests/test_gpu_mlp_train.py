@@ -111,3 +111,24 @@ def test_training_right_after_create_repeats(amca):
         first = p if first is None else first
         np.testing.assert_array_equal(p.view(np.uint32), first.view(np.uint32))
     hip.close()
+
+
+def test_set_params_starts_training_anew(amca):
+    """Setting the parameters also sets Adam's moments to zero, every one of them: steps
+    after other steps end as the first ones did."""
+    from amca3d_amd import surrogate as S
+    rng = np.random.default_rng(9)
+    X = rng.uniform(-1, 1, (64, 5)).astype(np.float32)
+    Y = rng.uniform(-1, 1, 64).astype(np.float32)
+    hip = _Hip()
+    dX, dY = hip.upload(X), hip.upload(Y)
+    m = S.MLP(5)
+    ends = []
+    for lr in (1e-3, 3e-2, 1e-3):
+        m.set_params(_params(4))
+        assert S.lib().amca_mlp_train_device(m.h, 64, dX, dY, 64, 5, lr, 9, None) == 0
+        ends.append(m.params().view(np.uint32))
+    np.testing.assert_array_equal(ends[0], ends[2])
+    assert (ends[0] != ends[1]).mean() > 0.9
+    hip.close()
+    m.close()
