@@ -1261,10 +1261,12 @@ amca_status amca_batch_run(amca_batch* b, int64_t max_graphs, int32_t* n_finishe
 // schedule with the least mean time per step wins.  The batch's work per step
 // drifts while the trials run, so odd rounds visit the candidates in reverse
 // order, which cancels a steady drift over each pair of rounds.  Stage 1 tries
-// one block budget for all list kernels (4, 16, 64 blocks per CU) in both
-// block orders; stage 2 sizes the claim grid and the resolve / emit grid
-// apart, a factor 4 up and down from the stage-1 choice.  Schedules do not
-// change results, so the trial steps are ordinary steps of the run.
+// one block budget for all list kernels (2, 16, 64 blocks per CU: 4 would stand for
+// the same blocks as 16) in both block orders; stage 2 sizes the claim grid and the
+// resolve / emit grid apart, a factor 4 up and down from the stage-1 choice, where
+// that is another number of blocks (the short step has one grid for both, of
+// emit_blocks).  Schedules do not change results, so the trial steps are ordinary
+// steps of the run.
 amca_status amca_batch_autotune(amca_batch* b, int32_t trial_graphs, int32_t rounds,
                                 amca_batch_schedule* chosen) {
   if (!b || trial_graphs < 1 || rounds < 1) return fail(AMCA_ERR_INVALID, "bad arguments");
@@ -1323,7 +1325,7 @@ amca_status amca_batch_autotune(amca_batch* b, int32_t trial_graphs, int32_t rou
   };
   // stage 1: one budget for every list kernel, both block orders
   std::vector<amca_batch_schedule> cand;
-  for (int budget : {4, 16, 64})
+  for (int budget : {2, 16, 64})
     for (int inter : {0, 1}) cand.push_back(make(budget, budget, inter));
   size_t best = 0;
   AMCA_TRY(pick(cand, &best));
@@ -1336,8 +1338,11 @@ amca_status amca_batch_autotune(amca_batch* b, int32_t trial_graphs, int32_t rou
     for (int f : {4, -4}) {
       const int l2 = f > 0 ? lb * f : std::max(1, lb / -f);
       const int e2 = f > 0 ? eb * f : std::max(1, eb / -f);
-      if (l2 != lb) c2.push_back(make(l2, eb, win.interleave));
-      if (e2 != eb) c2.push_back(make(lb, e2, win.interleave));
+      const auto other = [&](int p, int q) {
+        return budget_blocks(b, p * b->cus) != budget_blocks(b, q * b->cus);
+      };
+      if (!b->L.fused && other(l2, lb)) c2.push_back(make(l2, eb, win.interleave));
+      if (other(e2, eb)) c2.push_back(make(lb, e2, win.interleave));
     }
     AMCA_TRY(pick(c2, &best));
     win = c2[best];

@@ -176,9 +176,14 @@ amca_status amca_domain_kernel_times(amca_domain* d, double* ms, int64_t* launch
 typedef struct amca_batch amca_batch;
 
 typedef struct {
-  int32_t list_blocks;      /* claim blocks, shared in proportion to domain cell counts */
-  int32_t emit_blocks;      /* resolve / emit blocks, same sharing */
-  int32_t min_blocks;       /* at least this many per domain (1..4096) */
+  /* Budgets of blocks, shared in proportion to domain cell counts.  A budget is taken
+   * whole up to four blocks per CU; above that it stands for four per CU until a
+   * quarter of it is more. */
+  int32_t list_blocks;      /* claim blocks (no effect while the batch takes the short step,
+                               whose claims run on the grid of emit_blocks) */
+  int32_t emit_blocks;      /* resolve / emit blocks */
+  int32_t min_blocks;       /* at least this many per domain (1..4096), as far as its grid has
+                               that many pieces of 64 bricks (short step) */
   int32_t interleave;       /* 0: blocks domain by domain (largest first), 1: round robin */
   int32_t steps_per_graph;  /* steps captured in one graph replay */
 } amca_batch_schedule;
@@ -199,10 +204,10 @@ amca_status amca_batch_run(amca_batch* b, int64_t max_graphs, int32_t* n_finishe
 /* Tries candidate schedules on the running batch (trial_graphs replays each of
  * a graph of min(4, steps_per_graph) steps, `rounds` rounds, odd rounds in
  * reverse candidate order) and keeps the fastest per step: first one block
- * budget for every list kernel (4, 16 or 64 blocks per CU) in both block
- * orders, then the claim grid and the resolve / emit grid sized apart around
- * that choice.  The trial steps are ordinary steps of the run; the schedule's
- * steps_per_graph is kept. */
+ * budget for every list kernel (2, 16 or 64 blocks per CU) in both block
+ * orders, then the claim grid (long step only) and the resolve / emit grid sized
+ * apart around that choice.  The trial steps are ordinary steps of the run; the
+ * schedule's steps_per_graph is kept. */
 amca_status amca_batch_autotune(amca_batch* b, int32_t trial_graphs, int32_t rounds,
                                 amca_batch_schedule* chosen);
 

@@ -90,6 +90,25 @@ def test_after_autotune(amca, singles, factors):
     _check(amca, singles, factors, autotune=True)
 
 
+def test_autotune_of_the_short_step_leaves_the_claim_budget(amca):
+    """The short step's claims run on the grid of emit_blocks: the claim budget stays the
+    one tried for all kernels together."""
+    from amca3d_amd.batch import Batch
+    sims = [amca.Simulation(_text(m, 0.2)).initialize() for m in MEMBERS]
+    for s in sims:
+        s.domain.counters()
+    b = Batch([s.domain for s in sims])
+    cus = b.schedule()["list_blocks"] // 16
+    for _ in range(3):
+        c = b.autotune(trial_graphs=1, rounds=1)
+        assert c["list_blocks"] in [2 * cus, 16 * cus, 64 * cus]
+        assert c["emit_blocks"] in [cus * e for e in (1, 2, 4, 8, 16, 64, 128)]
+        assert b.schedule() == c
+    b.close()
+    for s in sims:
+        s.close()
+
+
 def test_members_with_steps_of_their_own(amca, singles):
     """Members that ran in their own form first, to different steps, join a long batch."""
     _check(amca, singles, MIXED, dict(steps_per_graph=5), before=[1, 0, 37, 150, 16])
