@@ -56,8 +56,9 @@ __device__ __forceinline__ float sigmoid(float z) {
   return __builtin_amdgcn_rcpf(1.0f + __expf(-z));
 }
 
-// C = opA(A) * opB(B), operands rounded to BF16 when staged into LDS: the matrix
-// layout check behind amca_mlp_gemm_selftest.  opA(A)[m][k] = TrA ? A[k*lda + m] :
+// C = opA(A) * opB(B), operands rounded to BF16 when staged into LDS:
+// amca_mlp_gemm_selftest, the lane layouts of the matrix instruction that the network's
+// kernels use, against any operands (they do not run this kernel).  opA(A)[m][k] = TrA ? A[k*lda + m] :
 // A[m*lda + k]; opB(B)[k][n] = TrB ? B[n*ldb + k] : B[k*ldb + n].  A work-group of
 // 4 waves owns a 128 x 128 block of C (ldc = N), each wave 32 rows and four
 // 32 x 32 MFMA tiles; elements outside the matrices stage as zero.
@@ -656,25 +657,6 @@ __global__ void k_sample(Sampler S, long long n, double near_fraction, unsigned 
     inputs(d, s, x, y, z, t, X + 5 * i);
     Y[i] = (float)to_target(d, T);
   }
-}
-
-__global__ void k_lattice_inputs(amca_surrogate_desc d, amca_scan s, SurLattice g, long long r0,
-                                 int m, float* __restrict__ X) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= m) return;
-  const long long q = r0 + r;
-  const int i = (int)(q % g.nxi);
-  const int j = (int)((q / g.nxi) % g.ny);
-  const int k = (int)(q / ((long long)g.nxi * g.ny));
-  // a lattice point is (xi, y, z) in the moving frame: feed x = xi + x_start at t = 0
-  inputs(d, s, g.xi0 + i * g.dxi + s.x_start, g.y0 + j * g.dy, g.z0 + k * g.dz, 0.0, X + 5 * r);
-}
-
-__global__ void k_denorm(const float* __restrict__ t, int m, amca_surrogate_desc d,
-                         float* __restrict__ out) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= m) return;
-  out[r] = (float)from_target(d, (double)t[r]);
 }
 
 // ---------------------------------------------------------------------------

@@ -44,7 +44,6 @@ struct DevCounters {
   long long n_solid;      // solid interior cells
   int skip;               // 1: this step is past termination, every kernel returns
   int done;               // no liquid cell left
-  int parity;             // which active-list buffer is the input of this step
   int site_sel;           // which site buffer holds the live sites
   int n_grains, n_orient;
   int nA_in, nA_out;      // active list lengths (input / survivors)
@@ -154,7 +153,6 @@ struct DevBuffers {
 };
 
 constexpr int kBlock = 256;       // threads per block of the list kernels
-constexpr int kItems = 4;         // consecutive list entries per thread in scan passes
 constexpr int kMaxBlocks = 4096;  // blocks of a look-back kernel
 constexpr int kLbSites = 2;       // look-back arrays: [0] k_nucleate's look-back, [1] k_resolve's
                                   // per-block statistics (lb_agg, lb_pref at kStatBase + block)

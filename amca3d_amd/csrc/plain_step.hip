@@ -1512,7 +1512,6 @@ __device__ __forceinline__ void tail_body(const DevParams& P, const DevBuffers& 
       row.n_sites = ctr->step_sites;
       B.log[st] = row;
     }
-    ctr->parity ^= 1;
     ctr->nA_in = ctr->nA_out;
     ctr->nA_out = 0;
   }

@@ -297,7 +297,8 @@ amca_status amca_surrogate_eval_lattice(amca_mlp* m, const amca_surrogate_desc* 
 amca_status amca_surrogate_eval(amca_mlp* m, const amca_surrogate_desc* d, const amca_scan* s,
                                 int32_t n, const double* xyzt, double* T_surrogate, double* T_fe);
 
-/* The tiled BF16 GEMM alone: C[M][N] = opA(A) opB(B) with FP32 host matrices
+/* A tiled BF16 GEMM alone, for checks of the matrix instruction's operand layouts (the
+ * network's own calls do not use it): C[M][N] = opA(A) opB(B) with FP32 host matrices
  * (row-major; trans_a: A is K x M, trans_b: B is N x K). */
 amca_status amca_mlp_gemm_selftest(int32_t M, int32_t N, int32_t K, int32_t trans_a,
                                    int32_t trans_b, const float* A, const float* B, float* C);
