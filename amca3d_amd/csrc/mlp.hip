@@ -1054,8 +1054,8 @@ hipError_t launch_fused_timed(amca_mlp* h, FusedMode mode, long long n, const fl
 // and the bias gradients are FP32 up to there, and the sums run in a fixed
 // order, so the gradients are the same on every run.
 //
-// Bound by the latency of its chain of layers (one work-group per CU, 13
-// barrier phases).  One GEMM launch per layer and direction, with the
+// Bound by the latency of its chain of layers (one work-group per CU, 16
+// barriers a group of rows).  One GEMM launch per layer and direction, with the
 // activations, dZ and atomic gradient sums through memory, took 285 us per step
 // of 8192 rows; k_train and k_reduce take 40 us.
 struct TrainLds {

@@ -100,8 +100,8 @@ struct alignas(64) SlotRec {
 // is on the reference's active list).  Per slot: the grain occupying the cell
 // (its record) and the claim word of the capture waves.  Steps read and write
 // only these: wave 0 walks the awake slots in brick order, so neighbouring
-// entries share map words, and the lists of waves >= 1 hold slots in grain-id
-// order.  The reference's layouts (cellGrainID_ / cellOrientationID_ on the
+// entries share map words; wave 1's list holds slots in its parents' brick order,
+// the lists of waves >= 2 in grain-id order.  The reference's layouts (cellGrainID_ / cellOrientationID_ on the
 // ghosted grid, x fastest; records by grain id) are materialized from the slots
 // when a download asks for them.
 //
@@ -138,7 +138,8 @@ struct DevBuffers {
   int* coff;              // first child (wave-relative) per capturing grain id [N]
   unsigned* idtot;        // wave-0 captures per id-scan block [kMaxIdsBlocks]
   unsigned* cmptot;       // awake grains per compaction block [kMaxBlocks]
-  int* listW[2];          // capture-wave lists (slots, in grain-id order) [N]
+  int* listW[2];          // capture-wave lists (slots): [0] wave 1, in its parents' brick order,
+                          // then alternately the waves >= 2, in grain-id order [N]
   unsigned long long* masks;  // per wave entry: inside bits << 32 | grain id (wave 0) or liquid
                               // bits (waves >= 1) [64 nB]
   int* site_cell[2];      // live nucleation sites, ascending cell, ping-pong

@@ -28,9 +28,10 @@
 //   k_tail          : waves >= 2 (rare) in one work-group, then the time advance.
 // Waves 0 and 1 each run k_claim, k_resolve, k_idscan and k_emit (wave 1's k_claim
 // only clears the id scan's totals).
-// On small grids a step is bound by its launches (about 4.5 us each, whatever
-// they do), and two shorter forms hold: k_wake_claim makes wave 0's list and tests
-// it in one launch, and k_tail also takes wave 1's captures, which are rare.
+// On small grids a step is bound by its launches (64^3: 53 us for the twelve, most of
+// which have next to nothing to do), and the short step takes six (39 us): k_wake_claim
+// makes wave 0's list and tests it in one launch, and k_tail also takes wave 1's
+// captures, as long as they are rare (choose_form in domain.hip).
 // Claims need no reset: every claimed cell is captured in the same wave and is
 // never liquid again.
 #include <hip/hip_runtime.h>
@@ -695,7 +696,7 @@ __device__ __forceinline__ void claim_range(const DevParams& P, const DevBuffers
 }
 
 // Wave 0's envelope tests, one entry per thread: bound by the lines of the
-// awake grains' records, about 340 bytes an entry at 512^3 (88 us a step for 1.1 M
+// awake grains' records, about 340 bytes an entry at 512^3 (80 us a step for 1.1 M
 // awake grains of 5.0 M active; all 5.0 M, packed closer, took 145).  Wave 0 first brings each
 // awake grain's L up to the running step (Grain::grow, Grain.h:27, over the whole
 // list as in :521-538: the sleeping grains' turns come when they wake) and leaves the

@@ -231,7 +231,10 @@ amca_status amca_mlp_forward(amca_mlp* m, int32_t n, const float* x5, float* t);
 amca_status amca_mlp_gradients(amca_mlp* m, int32_t n, const float* x5, const float* y,
                                float* grads, float* loss);
 /* `steps` Adam steps over random contiguous batches of device-resident samples
- * (dX[n][5], dY[n], pre-shuffled); optional per-step loss trace (host). */
+ * (dX[n][5], dY[n], pre-shuffled); optional per-step loss trace (host).  A network
+ * works on a stream of its own that waits for no other, the null stream included:
+ * whatever writes device rows handed to this call or to the forward calls below must
+ * have finished before it.  The calls return when their results are there. */
 amca_status amca_mlp_train_device(amca_mlp* m, int64_t n, const float* dX, const float* dY,
                                   int32_t batch, int32_t steps, float lr, uint64_t seed,
                                   float* loss_trace);
@@ -241,7 +244,8 @@ amca_status amca_mlp_train_device(amca_mlp* m, int64_t n, const float* dX, const
  * rounding of the hidden activations, which this kernel rounds scaled by
  * -log2(e) (the scaling cancels in the next layer). */
 amca_status amca_mlp_forward_fused(amca_mlp* h, int32_t n, const float* x5, float* t);
-/* Device rows dX[n][5] -> dT[n]. */
+/* Device rows dX[n][5] -> dT[n]; dX complete and dT free to be overwritten (no other
+ * stream still reads it) when the call is made. */
 amca_status amca_mlp_forward_device(amca_mlp* m, int64_t n, const float* dX, float* dT);
 /* amca_mlp_forward_device without any allocation: no counterpart in the
  * reference; for callers that cannot allocate (code under HIP graph capture,
