@@ -114,3 +114,14 @@ def test_batch_workload_specs():
     assert f"random_seed: {s5['seed']}\n" in deck
     assert f"number_cells: [{s5['edge']}, {s5['edge']}, {s5['edge']}]" in deck
     assert f"t_dot: {s5['Tdot']!r}" in deck
+
+
+def test_coupled_bytes_of_the_list_kernels():
+    """The sweep's kernels run on lists: no byte per box cell."""
+    log = {"n_box": np.array([1000, 3000]), "n_flagged": np.array([20, 0]),
+           "n_captured": np.array([7, 0])}
+    b = bench.remelt_algorithmic_bytes(dict(nodes=50), log)
+    np.testing.assert_array_equal(b["k_rm_claim"], [60 * 20, 0])
+    np.testing.assert_array_equal(b["k_rm_emit"], [52 * 7, 0])
+    np.testing.assert_array_equal(b["k_rm_nucleate_mint"], [1000 + 24 * 20, 3000])
+    np.testing.assert_array_equal(b["k_rm_phase"], [46 * 1000 + 400, 46 * 3000 + 400])
