@@ -438,14 +438,12 @@ amca_status amca_domain_create(const amca_domain_desc* desc, int32_t orient_capa
   want_buf(&B.cl1, (size_t)nB);
   want_buf(&B.awk, (size_t)nB);
   want_buf(&B.genv, N);
-  want_buf(&B.gco, N);
   want_buf(&B.alist, 64 * (size_t)nB);
   want_buf(&B.plist, 64 * (size_t)nB);
   want_buf(&B.cnt, N + 64);  // the id scan reads whole 16-byte groups past the last id
   want_buf(&B.coff, N);
   want_buf(&B.idtot, amca::kMaxIdsBlocks);
   want_buf(&B.cmptot, amca::kMaxBlocks);
-  want_buf(&B.listW[0], N);
   want_buf(&B.listW[1], N);
   want_buf(&B.masks, 64 * (size_t)nB);
   want_buf(&B.l2g, 9 * (size_t)std::max(orient_capacity, 1));
@@ -469,6 +467,13 @@ amca_status amca_domain_create(const amca_domain_desc* desc, int32_t orient_capa
     *q.p = arena;
     arena += q.bytes;
   }
+  // Shared room (12 bytes a cell, 1.6 of 22 GB at 512^3: the driver clears what a
+  // domain gives back, 0.45 s for 22 GB, and a program that makes large domains one
+  // after another waits for it).  Wave 0's list is last read by its k_resolve, and its
+  // k_emit then writes wave 1's; the parent list holds nothing between steps, when a
+  // download writes the (cell, orientation) pairs.
+  B.listW[0] = B.alist;
+  B.gco = reinterpret_cast<int2*>(B.plist);
   B.log = nullptr;
   d->site_cap = 1;
   HIP_TRY(hipMemsetAsync(B.lb_flag, 0, sizeof(unsigned) * amca::kLbSites * amca::kMaxBlocks, d->stream));

@@ -129,7 +129,8 @@ struct DevBuffers {
   unsigned long long* cl1;  // brick words: cells claimed in wave 1 [nB]
   unsigned long long* awk;  // brick words: active grains awake in the running step [nB]
   double4* genv;          // envelope by grain id, materialized for downloads [N]
-  int2* gco;              // grain -> (cell, orientation), materialized for downloads [N]
+  int2* gco;              // grain -> (cell, orientation), materialized for downloads into the
+                          // room of plist [N]
   int* alist;             // wave-0 list: awake slots in brick order (short step: one segment per
                           // k_wake_claim block, from the block's first slot) [64 nB]
   int4* plist;            // wave-0 capturing grains: (id, slot, captured slots), one segment
@@ -138,8 +139,9 @@ struct DevBuffers {
   int* coff;              // first child (wave-relative) per capturing grain id [N]
   unsigned* idtot;        // wave-0 captures per id-scan block [kMaxIdsBlocks]
   unsigned* cmptot;       // awake grains per compaction block [kMaxBlocks]
-  int* listW[2];          // capture-wave lists (slots): [0] wave 1, in its parents' brick order,
-                          // then alternately the waves >= 2, in grain-id order [N]
+  int* listW[2];          // capture-wave lists (slots): [0] wave 1, in its parents' brick order
+                          // and in the room of alist, then alternately the waves >= 2, in
+                          // grain-id order [N]
   unsigned long long* masks;  // per wave entry: inside bits << 32 | grain id (wave 0) or liquid
                               // bits (waves >= 1) [64 nB]
   int* site_cell[2];      // live nucleation sites, ascending cell, ping-pong
