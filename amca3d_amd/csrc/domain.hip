@@ -33,11 +33,15 @@ constexpr long long kFusedCells = 1ll << 24;
 // it is measured as the run goes.  Short against long form, us a step (walked grains a
 // step): 128^3 68.7 / 74.4 (2925), 102 / 94 (7489); 160^3 66.1 / 76.6 (2813), 103 / 89
 // (9347); 200^3 71.8 / 84.2 (2343), 97 / 87 (8538); 256^3 93 / 100 (2863), 102 / 102
-// (4510), 128 / 106 (10600), 372 / 152 (61145).  In a batch the launches are shared
-// (4 to 8 us a step between the forms) and any member's walk holds up the rest, so
-// kWalkBatch is the limit for the members' sum: 8 domains of 160^3 59.2 / 60.6 ms a
-// run (some 400 walked grains a step), 4 of 256^3 111 / 94 (11000).
-constexpr long long kWalkShort = 4500, kWalkBatch = 2000;
+// (4510), 128 / 106 (10600), 372 / 152 (61145).  They break even near 5000; claims come
+// singly at first, and a limit that a few of them within one look pass makes the form
+// change for nothing (256^3 at factor 0.1, ms a run at limits of 4500, 6000 and 9000:
+// 60.4, 59.5, 58.8, short throughout 58.3; at factor 0.25 38.2, 38.1, 40.4 and 42.8).
+// In a batch the launches are shared (4 to 8 us a step between the forms) and any
+// member's walk holds up the rest, so kWalkBatch is the limit for the members' sum: 8
+// domains of 160^3 58.1 ms a run, short or long throughout 59.3 and 60.4; 4 of 256^3
+// 94.0, 112 and 92.9.
+constexpr long long kWalkShort = 7000, kWalkBatch = 2000;
 constexpr long long kFormSteps = 8;  // steps between looks at w1_walk, at least
 // More than kBurstSites live sites in more than kBurstCells cells may nucleate in a burst
 // of a few tens of steps, over before a look can answer it, so such a domain takes the
@@ -830,24 +834,26 @@ amca_status amca_envelope_selftest(int32_t n, const double* env4, const double* 
 struct amca_batch {
   std::vector<amca_domain*> doms;
   std::vector<amca::DevParams> P;  // the domains' parameters with the batch's step form and grids
-  // whether every domain may take the short step; the domains' walks (w1_walk, low 31
-  // bits) when they were last looked at and the steps run since
-  bool may_fuse = false;
+  // step form: whether every domain may take the short step, whether a nucleation burst
+  // is still to come, and the form of the next replay; the domains' walks (w1_walk, low
+  // 31 bits) when they were last looked at and the steps run since
+  bool may_fuse = false, burst = false;
+  int form = 0;
   std::vector<int> walk0;
   long long walk_steps = 0;
   int device = 0;
   hipStream_t stream = nullptr;
-  amca::DevParams* dP = nullptr;
+  amca::DevParams* dP = nullptr;  // by step form, n each
   amca::DevBuffers* dB = nullptr;
-  int4* maps = nullptr;  // nuc | list | emit | scan | ids | compaction, back to back
+  int4* maps = nullptr;  // nuc | list | emit | tail | ids by form | compaction, back to back
   int4* status = nullptr;
   int4* hstatus = nullptr;  // pinned: two slots of n statuses, one per replay in flight
   hipEvent_t hready[2] = {nullptr, nullptr};
-  amca::BatchLaunch L{};
+  amca::BatchLaunch L[2] = {};  // by step form
   amca_batch_schedule sched{};
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
-  int graph_steps = 0;
+  hipGraph_t graph[2] = {nullptr, nullptr};
+  hipGraphExec_t exec[2] = {nullptr, nullptr};
+  int graph_steps = 0;  // of both graphs
   bool use_graph = true;  // false: every replay launches its kernels one by one
   int cus = 256;
   double last_ms_per_step = 0.0;
@@ -857,10 +863,12 @@ struct amca_batch {
   int mapped_finished = 0;
 
   void drop_graph() {
-    if (exec) (void)hipGraphExecDestroy(exec);
-    if (graph) (void)hipGraphDestroy(graph);
-    exec = nullptr;
-    graph = nullptr;
+    for (int f = 0; f < 2; f++) {
+      if (exec[f]) (void)hipGraphExecDestroy(exec[f]);
+      if (graph[f]) (void)hipGraphDestroy(graph[f]);
+      exec[f] = nullptr;
+      graph[f] = nullptr;
+    }
     graph_steps = 0;
   }
   ~amca_batch() {
@@ -955,7 +963,6 @@ amca_status batch_apply_schedule(amca_batch* b) {
                                                                    (long long)amca::kMaxBlocks}))
                          : 0;
     b->P[i].cmp_blocks = std::max(1, nc[i]);
-    b->P[i].fused = b->L.fused;
     one[i] = b->active[i] ? 1 : 0;
   }
   std::vector<int> order(n);
@@ -963,16 +970,19 @@ amca_status batch_apply_schedule(amca_batch* b) {
   // larger domains first: their blocks start earliest
   std::stable_sort(order.begin(), order.end(),
                    [&](int a, int c) { return b->doms[a]->P.N > b->doms[c]->P.N; });
-  std::vector<int4> mn, ml, me, ms, mi, mc;
+  std::vector<int4> mn, ml, me, ms, mi[2], mc;
   build_map(order, nn, b->sched.interleave, mn);
-  build_map(order, ni, b->sched.interleave, mi);
   // the id scan sums the domain's k_resolve blocks (short step: of wave 0 only)
-  for (auto& m : mi) m.w = b->L.fused ? nc[m.x] : ne[m.x];
+  for (int f = 0; f < 2; f++) {
+    build_map(order, ni, b->sched.interleave, mi[f]);
+    for (auto& m : mi[f]) m.w = f ? nc[m.x] : ne[m.x];
+  }
   build_map(order, nc, b->sched.interleave, mc);
   build_map(order, nl, b->sched.interleave, ml);
   build_map(order, ne, b->sched.interleave, me);
   build_map(order, one, 0, ms);
-  const size_t total = mn.size() + ml.size() + me.size() + ms.size() + mi.size() + mc.size();
+  const size_t total =
+      mn.size() + ml.size() + me.size() + ms.size() + 2 * mi[0].size() + mc.size();
   if (b->maps) HIP_TRY(hipFree(b->maps));
   b->maps = nullptr;
   HIP_TRY(hipMalloc(&b->maps, sizeof(int4) * total));
@@ -981,32 +991,44 @@ amca_status batch_apply_schedule(amca_batch* b) {
   all.insert(all.end(), ml.begin(), ml.end());
   all.insert(all.end(), me.begin(), me.end());
   all.insert(all.end(), ms.begin(), ms.end());
-  all.insert(all.end(), mi.begin(), mi.end());
+  for (int f = 0; f < 2; f++) all.insert(all.end(), mi[f].begin(), mi[f].end());
   all.insert(all.end(), mc.begin(), mc.end());
   HIP_TRY(hipMemcpy(b->maps, all.data(), sizeof(int4) * total, hipMemcpyHostToDevice));
-  HIP_TRY(hipMemcpy(b->dP, b->P.data(), sizeof(amca::DevParams) * n, hipMemcpyHostToDevice));
-  b->L.map_nuc = b->maps;
-  b->L.map_list = b->maps + mn.size();
-  b->L.map_emit = b->L.map_list + ml.size();
-  b->L.map_one = b->L.map_emit + me.size();
-  b->L.map_ids = b->L.map_one + ms.size();
-  b->L.map_cmp = b->L.map_ids + mi.size();
-  b->L.n_nuc = (int)mn.size();
-  b->L.n_list = (int)ml.size();
-  b->L.n_emit = (int)me.size();
-  b->L.n_one = (int)ms.size();
-  b->L.n_ids = (int)mi.size();
-  b->L.n_cmp = (int)mc.size();
+  for (int f = 0; f < 2; f++) {
+    for (auto& p : b->P) p.fused = f;
+    HIP_TRY(hipMemcpy(b->dP + (size_t)f * n, b->P.data(), sizeof(amca::DevParams) * n,
+                      hipMemcpyHostToDevice));
+    amca::BatchLaunch& L = b->L[f];
+    L.P = b->dP + (size_t)f * n;
+    L.B = b->dB;
+    L.fused = f;
+    L.map_nuc = b->maps;
+    L.map_list = L.map_nuc + mn.size();
+    L.map_emit = L.map_list + ml.size();
+    L.map_one = L.map_emit + me.size();
+    L.map_ids = L.map_one + ms.size() + (size_t)f * mi[0].size();
+    L.map_cmp = L.map_one + ms.size() + 2 * mi[0].size();
+    L.n_nuc = (int)mn.size();
+    L.n_list = (int)ml.size();
+    L.n_emit = (int)me.size();
+    L.n_one = (int)ms.size();
+    L.n_ids = (int)mi[f].size();
+    L.n_cmp = (int)mc.size();
+  }
   b->drop_graph();
   return AMCA_OK;
 }
 
-amca_status batch_capture(amca_batch* b, int steps) {
-  b->drop_graph();
+// The graph of the batch's form; both are of the schedule's steps_per_graph.
+amca_status batch_capture(amca_batch* b) {
+  const int steps = b->sched.steps_per_graph, f = b->form;
+  if (b->graph_steps != steps) b->drop_graph();
+  if (b->exec[f]) return AMCA_OK;
   HIP_TRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
   hipError_t e = hipSuccess;
-  for (int q = 0; q < steps && e == hipSuccess; q++) e = amca::launch_batch_step(b->L, b->stream);
-  if (e == hipSuccess) e = amca::launch_batch_status(b->L, (int)b->doms.size(), b->status, b->stream);
+  for (int q = 0; q < steps && e == hipSuccess; q++) e = amca::launch_batch_step(b->L[f], b->stream);
+  if (e == hipSuccess)
+    e = amca::launch_batch_status(b->L[f], (int)b->doms.size(), b->status, b->stream);
   hipGraph_t g = nullptr;
   const hipError_t e2 = hipStreamEndCapture(b->stream, &g);
   if (e != hipSuccess || e2 != hipSuccess) {
@@ -1014,9 +1036,10 @@ amca_status batch_capture(amca_batch* b, int steps) {
     return fail(AMCA_ERR_HIP, std::string("graph capture: ") +
                                   hipGetErrorString(e != hipSuccess ? e : e2));
   }
-  b->graph = g;
-  HIP_TRY(hipGraphInstantiate(&b->exec, g, nullptr, nullptr, 0));
+  if (b->graph[f]) (void)hipGraphDestroy(b->graph[f]);
+  b->graph[f] = g;
   b->graph_steps = steps;
+  HIP_TRY(hipGraphInstantiate(&b->exec[f], g, nullptr, nullptr, 0));
   return AMCA_OK;
 }
 
@@ -1029,12 +1052,9 @@ amca_status batch_capture(amca_batch* b, int steps) {
 // domains have finished the maps are rebuilt over the domains still running,
 // so that the budgets of the list kernels go to them alone (a finished
 // domain's kernels return at once, so leaving it out changes no result), and the
-// step form is chosen again; from the short form to the long one the batch also
-// goes as soon as its walk asks for it.
+// step form of the next replay follows the walk of the last ones.
 amca_status batch_replay(amca_batch* b, long long max_graphs, int* finished, double* ms,
                          long long* replays, bool remap) {
-  if (b->use_graph && (!b->exec || b->graph_steps != b->sched.steps_per_graph))
-    AMCA_TRY(batch_capture(b, b->sched.steps_per_graph));
   const int n = (int)b->doms.size();
   struct Events {  // destroyed on every return
     hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -1045,23 +1065,23 @@ amca_status batch_replay(amca_batch* b, long long max_graphs, int* finished, dou
   } ev;
   HIP_TRY(hipEventCreate(&ev.e0));
   HIP_TRY(hipEventCreate(&ev.e1));
-  auto queue = [&](long long r) -> hipError_t {
-    hipError_t e = hipSuccess;
+  auto queue = [&](long long r) -> amca_status {
+    const amca::BatchLaunch& L = b->L[b->form];
     if (b->use_graph) {
-      e = hipGraphLaunch(b->exec, b->stream);
+      AMCA_TRY(batch_capture(b));
+      HIP_TRY(hipGraphLaunch(b->exec[b->form], b->stream));
     } else {
-      for (int q = 0; q < b->sched.steps_per_graph && e == hipSuccess; q++)
-        e = amca::launch_batch_step(b->L, b->stream);
-      if (e == hipSuccess) e = amca::launch_batch_status(b->L, n, b->status, b->stream);
+      for (int q = 0; q < b->sched.steps_per_graph; q++)
+        HIP_TRY(amca::launch_batch_step(L, b->stream));
+      HIP_TRY(amca::launch_batch_status(L, n, b->status, b->stream));
     }
-    if (e == hipSuccess)
-      e = hipMemcpyAsync(b->hstatus + (r & 1) * n, b->status, sizeof(int4) * n,
-                         hipMemcpyDeviceToHost, b->stream);
-    if (e == hipSuccess) e = hipEventRecord(b->hready[r & 1], b->stream);
-    return e;
+    HIP_TRY(hipMemcpyAsync(b->hstatus + (r & 1) * n, b->status, sizeof(int4) * n,
+                           hipMemcpyDeviceToHost, b->stream));
+    HIP_TRY(hipEventRecord(b->hready[r & 1], b->stream));
+    return AMCA_OK;
   };
-  // the walk of the steps since the last look against the limit (the short form's)
-  bool walk_short = b->L.fused != 0;
+  // the form by the walk of the steps since the last look (every step leaves the same
+  // state in either); the autotuner's trials keep theirs
   auto look = [&](const int4* st, long long steps) {
     b->walk_steps += steps;
     if (b->walk_steps < kFormSteps) return;
@@ -1070,19 +1090,22 @@ amca_status batch_replay(amca_batch* b, long long max_graphs, int* finished, dou
       walk += (st[i].w - b->walk0[i]) & 0x7fffffff;
       b->walk0[i] = st[i].w;
     }
-    walk_short = walk <= kWalkBatch * b->walk_steps;
+    const bool light = walk <= kWalkBatch * b->walk_steps;
     b->walk_steps = 0;
+    if (!light) b->burst = false;  // it has begun, and its walk decides from here on
+    if (remap) b->form = b->may_fuse && light && !b->burst ? 1 : 0;
   };
+  if (b->use_graph) AMCA_TRY(batch_capture(b));
   HIP_TRY(hipEventRecord(ev.e0, b->stream));
   long long r = 0, queued = 0;
   int fin = 0;
   if (max_graphs != 0) {
-    HIP_TRY(queue(0));
+    AMCA_TRY(queue(0));
     queued = 1;
   }
   while (r < queued) {
     if (max_graphs < 0 || queued < max_graphs) {
-      HIP_TRY(queue(queued));
+      AMCA_TRY(queue(queued));
       queued++;
     }
     HIP_TRY(hipEventSynchronize(b->hready[r & 1]));
@@ -1098,8 +1121,7 @@ amca_status batch_replay(amca_batch* b, long long max_graphs, int* finished, dou
     }
     if (fin == n) break;
     look(st, b->sched.steps_per_graph);
-    const bool to_long = b->L.fused && !walk_short;
-    if (remap && (to_long || fin - b->mapped_finished >= std::max(4, n / 8))) {
+    if (remap && fin - b->mapped_finished >= std::max(4, n / 8)) {
       // rebuild the maps over the running domains: wait for the queued replay,
       // take the finished set from its status, and capture a new graph
       HIP_TRY(hipStreamSynchronize(b->stream));
@@ -1115,11 +1137,10 @@ amca_status batch_replay(amca_batch* b, long long max_graphs, int* finished, dou
       r = queued;
       if (fin == n) break;
       b->mapped_finished = fin;
-      b->L.fused = b->may_fuse && walk_short;
+      b->burst = false;
       AMCA_TRY(batch_apply_schedule(b));
-      if (b->use_graph) AMCA_TRY(batch_capture(b, b->sched.steps_per_graph));
       if (max_graphs < 0 || queued < max_graphs) {
-        HIP_TRY(queue(queued));
+        AMCA_TRY(queue(queued));
         queued++;
       }
     }
@@ -1188,8 +1209,9 @@ amca_status amca_batch_create(amca_domain* const* doms, int32_t n, amca_batch** 
     if (st != AMCA_OK) break;
     // one launch sequence for the batch: the short one if every domain may take it,
     // as long as their sites and walks allow (batch_replay)
-    b->L.fused = b->may_fuse && !many_sites ? 1 : 0;
-    if (hipMalloc(&b->dP, sizeof(amca::DevParams) * n) != hipSuccess ||
+    b->burst = many_sites;
+    b->form = b->may_fuse && !b->burst ? 1 : 0;
+    if (hipMalloc(&b->dP, sizeof(amca::DevParams) * 2 * n) != hipSuccess ||
         hipMalloc(&b->dB, sizeof(amca::DevBuffers) * n) != hipSuccess ||
         hipMalloc(&b->status, sizeof(int4) * n) != hipSuccess ||
         hipHostMalloc(&b->hstatus, sizeof(int4) * 2 * n) != hipSuccess ||
@@ -1202,8 +1224,6 @@ amca_status amca_batch_create(amca_domain* const* doms, int32_t n, amca_batch** 
       st = fail(AMCA_ERR_HIP, "batch upload failed");
       break;
     }
-    b->L.P = b->dP;
-    b->L.B = b->dB;
     b->sched.list_blocks = 16 * b->cus;
     b->sched.emit_blocks = 16 * b->cus;
     b->sched.min_blocks = 1;
@@ -1346,7 +1366,7 @@ amca_status amca_batch_autotune(amca_batch* b, int32_t trial_graphs, int32_t rou
       const auto other = [&](int p, int q) {
         return budget_blocks(b, p * b->cus) != budget_blocks(b, q * b->cus);
       };
-      if (!b->L.fused && other(l2, lb)) c2.push_back(make(l2, eb, win.interleave));
+      if (!b->form && other(l2, lb)) c2.push_back(make(l2, eb, win.interleave));
       if (other(e2, eb)) c2.push_back(make(lb, e2, win.interleave));
     }
     AMCA_TRY(pick(c2, &best));
