@@ -109,6 +109,9 @@ struct amca_domain {
   bool may_fuse = false, walk_ok = true, many_sites = false;
   int cmp_blocks[2] = {1, 1};
   long long seen_step = 0, seen_walk = 0;
+  // room of the lists that only a running step holds anything in
+  void* scratch = nullptr;
+  size_t scratch_bytes = 0;
   // counters copied behind a stretch of queued steps (pinned) and the event behind
   // the copy, for two stretches in flight (run_steps)
   amca::DevCounters* look[2] = {nullptr, nullptr};
@@ -443,14 +446,14 @@ amca_status amca_domain_create(const amca_domain_desc* desc, int32_t orient_capa
   want_buf(&B.cl1, (size_t)nB);
   want_buf(&B.awk, (size_t)nB);
   want_buf(&B.genv, N);
-  want_buf(&B.alist, 64 * (size_t)nB);
+  want_buf(&B.alist, 64 * (size_t)nB);  // from here to masks: of a step, `scratch` between steps
   want_buf(&B.plist, 64 * (size_t)nB);
+  want_buf(&B.masks, 64 * (size_t)nB);
   want_buf(&B.cnt, N + 64);  // the id scan reads whole 16-byte groups past the last id
   want_buf(&B.coff, N);
   want_buf(&B.idtot, amca::kMaxIdsBlocks);
   want_buf(&B.cmptot, amca::kMaxBlocks);
   want_buf(&B.listW[1], N);
-  want_buf(&B.masks, 64 * (size_t)nB);
   want_buf(&B.l2g, 9 * (size_t)std::max(orient_capacity, 1));
   want_buf(&B.lb_flag, (size_t)amca::kLbSites * amca::kMaxBlocks);
   want_buf(&B.lb_agg, (size_t)amca::kLbSites * amca::kMaxBlocks);
@@ -479,6 +482,8 @@ amca_status amca_domain_create(const amca_domain_desc* desc, int32_t orient_capa
   // download writes the (cell, orientation) pairs.
   B.listW[0] = B.alist;
   B.gco = reinterpret_cast<int2*>(B.plist);
+  d->scratch = B.alist;
+  d->scratch_bytes = reinterpret_cast<char*>(B.masks + 64 * (size_t)nB) - reinterpret_cast<char*>(B.alist);
   B.log = nullptr;
   d->site_cap = 1;
   HIP_TRY(hipMemsetAsync(B.lb_flag, 0, sizeof(unsigned) * amca::kLbSites * amca::kMaxBlocks, d->stream));
@@ -699,14 +704,11 @@ amca_status amca_domain_download(amca_domain* d, int32_t* orient, int32_t* grain
   if (orient) HIP_TRY(hipMemcpy(orient, d->B.oid, sizeof(int32_t) * NG, hipMemcpyDeviceToHost));
   if (grain) HIP_TRY(hipMemcpy(grain, d->B.gid, sizeof(int32_t) * NG, hipMemcpyDeviceToHost));
   if (env) {
-    // laid out by cell on the device, a piece of 64 MB at a time (the host's
-    // memset and scatter of the records took longer than the run of a small grid)
-    const size_t piece = std::min<size_t>(NG, (size_t)1 << 21);
-    double4* buf = nullptr;
-    const auto release = on_scope_exit([&] {
-      if (buf) (void)hipFree(buf);
-    });
-    HIP_TRY(hipMalloc(&buf, sizeof(double4) * piece));
+    // laid out by cell on the device, a piece of up to 64 MB at a time (the host's
+    // memset and scatter of the records took longer than the run of a small grid), in
+    // the room of a step's lists: no allocation that could fail or be waited for
+    const size_t piece = std::min<size_t>({NG, d->scratch_bytes / sizeof(double4), (size_t)1 << 21});
+    double4* buf = static_cast<double4*>(d->scratch);
     for (size_t c0 = 0; c0 < NG; c0 += piece) {
       const int n = (int)std::min(piece, NG - c0);
       HIP_TRY(amca::launch_cell_env(d->P, d->B, (long long)c0, n, buf, d->stream));
