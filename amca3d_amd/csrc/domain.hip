@@ -298,17 +298,18 @@ amca_status enqueue_steps(amca_domain* d, long long n) {
 
 // Up to `most` steps (negative: no limit), until the run is over if `to_end`; *c holds
 // the counters before and after.  Two stretches of steps are in flight, so that the
-// look at one stretch's counters costs the GPU nothing; 16 steps each where the form
-// may change with the look, which comes a stretch late, else 32 (the steps queued past
-// the end of a run do nothing, but 512^3 takes 30 us for each), or a graph's length
-// where that was set longer.
+// look at one stretch's counters costs the GPU no more than the copy; 16 steps each
+// where the form, which follows the look a stretch late, may cost more than the copies
+// (128^3 with 8.3e4 sites 19.7 ms in stretches of 32, 17.7 of 16; 60^3 0.9 % slower in
+// those), else 32 (the steps queued past the end of a run do nothing, but 512^3 takes
+// 30 us for each), or a graph's length where that was set longer.
 amca_status run_steps(amca_domain* d, long long most, bool to_end, amca::DevCounters* c) {
   for (int q = 0; q < 2; q++) {
     if (!d->look[q]) HIP_TRY(hipHostMalloc(&d->look[q], sizeof(amca::DevCounters)));
     if (!d->looked[q]) HIP_TRY(hipEventCreateWithFlags(&d->looked[q], hipEventDisableTiming));
   }
   const long long graph = to_end ? std::min(d->graph_steps, 64) : d->graph_steps;
-  const long long longest = std::max(d->may_fuse ? 16LL : 32LL, graph);
+  const long long longest = std::max(d->may_fuse && d->P.N > (1ll << 20) ? 16LL : 32LL, graph);
   long long len = 8, queued = 0;
   long long made = 0, seen = 0;  // stretches queued and looked at
   while (true) {
